@@ -38,8 +38,8 @@ from sedcol.params import (ADAPTIVE_EULER, EULER, NVAR, PARTICULATE,  # noqa: E4
 
 DAY = 86400.0
 METHODS = {"euler": EULER, "rk4": RUNGE_KUTTA_4, "adaptive-euler": ADAPTIVE_EULER, "rk4-38": RUNGE_KUTTA_4_38}
-#: adaptive attempts per column and day near the seasonal state
-ATTEMPTS_PER_DAY = {"product": 2000.0, "geometric": 4000.0, "ros2": 150.0}
+#: adaptive attempts per column and day in the first hours from these states
+ATTEMPTS_PER_DAY = {"product": 20000.0, "geometric": 25000.0, "ros2": 2600.0}
 
 
 def listed():
