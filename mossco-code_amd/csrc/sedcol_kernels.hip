@@ -889,72 +889,122 @@ __global__ __launch_bounds__(BLK, SEDCOL_EMP2_MIN_WAVES) void k_emp_adaptive2(
 
 constexpr double ROS_GAMMA = 1.7071067811865475;
 
+// two doubles in one 16-byte LDS access
+typedef double dbl2 __attribute__((ext_vector_type(2)));
+
 // per-group LDS of the stepper
 template <int LPC>
-struct RosShared {
-  double G[2][LPC];     // transport coefficients D/dzc (D/dz at the top): [0] particulate, [1] dissolved
-  double W[LPC];        // 1/(phi dz)
-  double ph[LPC];       // porosity
-  // Species rows padded by one double: the sweep of species n runs in lane
-  // n, so the lanes read one layer of 11 different rows at once; with the
-  // padding those sit in different LDS banks (unpadded, the row pitch is a
-  // multiple of the bank count and the 11 reads serialise)
-  double T[NV][LPC + 1];    // right-hand sides and solutions of the species sweeps
-  double inv[NV][LPC + 1];  // reciprocal Thomas pivots
-  double A[NV][LPC + 1];    // sub-diagonal couplings of the forward sweep
-  double E[NV][LPC + 1];    // super-diagonal coupling times reciprocal pivot (back substitution)
-  double top[2][NV];    // linearised Dirichlet top-flux terms of the two stages
+struct alignas(16) RosShared {
+  // Species rows padded by two doubles: the sweep of species n runs in lane
+  // n, so the lanes read one pair of layers of 11 different rows at once;
+  // with this pitch the 16-byte reads fall into different LDS banks
+  double T[NV][LPC + 2];  // right-hand sides and solutions of the species sweeps
+  // The transport factor is the same for all particulate variables ([0]) and
+  // for all dissolved ones ([1]): they share diffusivity and top condition
+  dbl2 BC[2][LPC];     // diagonal and super-diagonal coupling
+  dbl2 AI[2][LPC];     // sub-diagonal coupling of the forward sweep, reciprocal pivot
+  double E[2][LPC + 2];   // super-diagonal coupling times reciprocal pivot (back substitution)
+  double top[2][NV];      // linearised Dirichlet top-flux terms of the two stages
 };
 
-// Thomas factor of species n = l (lanes l < NV of the group): reciprocal
-// pivots, the forward-sweep couplings a_k and the back-substitution
-// couplings c_k / piv_k, so that a sweep is one dependent fma-and-multiply
-// (forward) or multiply-and-add (backward) per layer with operands that do
-// not depend on the chain
+// the lane's transport coefficients: D/dzc (D/dz at the top) of the
+// particulate and dissolved variables, 1/(phi dz)
+struct RosLane {
+  double Gp, Gd, W;
+};
+
+// correctly rounded 1/b for b well inside the normal range: the hardware
+// estimate (relative error 2^-24), one third-order step to the last place,
+// and Markstein's final correction
+__device__ __forceinline__ double rcp_exact(double b)
+{
+  double y = __builtin_amdgcn_rcp(b);
+  const double e = fma(-b, y, 1.0);
+  y = fma(y, fma(e, e, e), y);
+  return fma(fma(-b, y, 1.0), y, y);
+}
+
+// Matrix rows of both classes, one layer per lane: everything of the Thomas
+// factorisation that is not on its serial chain.  Lanes beyond the column
+// write identity rows.
 template <int LPC>
-__device__ __forceinline__ void ros_factor(RosShared<LPC> &R, int l, int K, double g, unsigned dirmask)
+__device__ __forceinline__ void ros_rows(RosShared<LPC> &R, const RosLane &C, int l, int K, bool act, double phi,
+                                         double g, unsigned dirmask)
+{
+  const bool first = l == 0, last = l == K - 1;
+  const double phu = lg_up(phi), phd = lg_dn(phi);
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const double G = m == 0 ? C.Gp : C.Gd;
+    const double Gdn = lg_dn(G);
+    const bool dir = (dirmask >> (m == 0 ? 0 : 5)) & 1u;
+    const double s = ((!first || dir) ? G : 0.0) + (last ? 0.0 : Gdn);
+    const double b = 1.0 + g * (C.W * (m == 0 ? s * phi : s));
+    const double a = g * (m == 0 ? (C.W * G) * phu : C.W * G);
+    const double c = g * (m == 0 ? (C.W * Gdn) * phd : C.W * Gdn);
+    R.BC[m][l] = dbl2{act ? b : 1.0, act && !last ? c : 0.0};
+    R.AI[m][l].x = act && !first ? a : 0.0;
+  }
+}
+
+// The sweeps exist twice.  ros_*_lds (lane n < NV sweeps species n, all
+// operands in LDS, IEEE divisions) serves columns of up to 16 layers and any
+// value.  For LPC = 32 and 64 RosSweep does the same operations with the
+// factor in registers: LDS traffic bounds the LDS form, because an access by
+// 11 lanes costs a full wave's (68 cycles a layer against a chain of 24).
+// A factor with its first sweep went from 6700 to 3300 cycles (24 layers), a
+// sweep down from 2200 to 930 and up from 2700 to 850; half a day of 3000
+// columns of 20 to 40 layers, a spin-up's chunk, from 222 to 122 ms.
+
+// Thomas factor of species l's class and forward sweep of the first solve
+template <int LPC>
+__device__ __forceinline__ void ros_factor_lds(RosShared<LPC> &R, int l, int K)
 {
   if (l < NV) {
-    const bool pt = part(l);
-    const double *__restrict__ G = R.G[pt ? 0 : 1];
-    const double *__restrict__ W = R.W;
-    const double *__restrict__ ph = R.ph;
-    double *__restrict__ inv = R.inv[l];
-    double *__restrict__ A = R.A[l];
-    double *__restrict__ E = R.E[l];
-    const bool dir = (dirmask >> l) & 1u;
-    double e = 0.0;
+    const int m = part(l) ? 0 : 1;
+    double *T = R.T[l];
+    const bool keep = l == 0 || l == 5;  // one lane per class stores the factor
+    double e = 0.0, d = 0.0;
     for (int k = 0; k < K; ++k) {
-      const double qk = pt ? ph[k] : 1.0;
-      const double s = ((k > 0 || dir) ? G[k] : 0.0) + (k < K - 1 ? G[k + 1] : 0.0);
-      const double b = 1.0 + g * (W[k] * (s * qk));
-      const double a = k > 0 ? g * ((W[k] * G[k]) * (pt ? ph[k - 1] : 1.0)) : 0.0;
-      const double piv = k > 0 ? b - a * e : b;
+      const dbl2 bc = R.BC[m][k];
+      const double a = R.AI[m][k].x;
+      const double piv = bc.x - a * e;  // a = 0 in the first row
       const double iv = 1.0 / piv;
-      const double c = k < K - 1 ? g * ((W[k] * G[k + 1]) * (pt ? ph[k + 1] : 1.0)) : 0.0;
-      e = c * iv;
-      inv[k] = iv;
-      A[k] = a;
-      E[k] = e;
+      e = bc.y * iv;
+      d = k > 0 ? (T[k] + a * d) * iv : T[k] * iv;
+      T[k] = d;
+      if (keep) {
+        R.AI[m][k].y = iv;
+        R.E[m][k] = e;
+      }
     }
   }
 }
 
-// B z = T in place, species n = l
+// forward sweep of species l: T_k <- (T_k + a_k T_{k-1}) / pivot_k
 template <int LPC>
-__device__ __forceinline__ void ros_sweep(RosShared<LPC> &R, int l, int K)
+__device__ __forceinline__ void ros_forward_lds(RosShared<LPC> &R, int l, int K)
 {
   if (l < NV) {
-    double *__restrict__ T = R.T[l];
-    const double *__restrict__ iv = R.inv[l];
-    const double *__restrict__ A = R.A[l];
-    const double *__restrict__ E = R.E[l];
-    double d = T[0] * iv[0];
+    double *T = R.T[l];
+    const dbl2 *AI = R.AI[part(l) ? 0 : 1];
+    double d = T[0] * AI[0].y;
     T[0] = d;
     for (int k = 1; k < K; ++k) {
-      d = (T[k] + A[k] * d) * iv[k];
+      d = (T[k] + AI[k].x * d) * AI[k].y;
       T[k] = d;
     }
+  }
+}
+
+// back substitution of species l: T_k <- T_k + E_k T_{k+1}
+template <int LPC>
+__device__ __forceinline__ void ros_backward_lds(RosShared<LPC> &R, int l, int K)
+{
+  if (l < NV) {
+    double *T = R.T[l];
+    const double *E = R.E[part(l) ? 0 : 1];
+    double d = T[K - 1];
     for (int k = K - 2; k >= 0; --k) {
       d = T[k] + E[k] * d;
       T[k] = d;
@@ -962,17 +1012,224 @@ __device__ __forceinline__ void ros_sweep(RosShared<LPC> &R, int l, int K)
   }
 }
 
-// B^-1 r for the lane's layer: stage through LDS, sweep, read back
+// value of lane J of the lane's row of 16
+template <int J>
+__device__ __forceinline__ double row_bcast(double v)
+{
+  return __longlong_as_double(__builtin_amdgcn_update_dpp(0ll, __double_as_longlong(v), 0x150 + J, 0xf, 0xf, true));
+}
+
+// Sweeps of a column of more than 16 layers: the particulate species in
+// lanes 0..5 of the group's first row of 16 lanes, the dissolved ones in
+// lanes 0..4 of the second.  Lane j of a row keeps the rows j, j + 16, ... of
+// its class's factor, and each step takes its coefficients by a row
+// broadcast, one VALU move each.  A species' right-hand side is read from
+// LDS once, swept down and up in registers and written back.  Layers beyond
+// the column are identity rows with right-hand side 0, so a finite last value
+// leaves T_{K-1} as it is; ok() is false when it is not finite.
 template <int LPC>
-__device__ __forceinline__ void ros_bsolve(RosShared<LPC> &R, int l, int K, bool act, double g, const double (&r)[NV],
-                                           double (&v)[NV])
+struct RosSweep {
+  static constexpr int R16 = LPC / 16;
+  double a[R16], iv[R16], E[R16];
+  double *T;   // the lane's species row
+  int m, j;    // class and lane of its row
+  bool own;    // sweeps a species (the others run along)
+
+  __device__ __forceinline__ void init(RosShared<LPC> &R, int l)
+  {
+    m = (l >> 4) & 1;
+    j = l & 15;
+    own = l < 32 && j < (m == 0 ? 6 : 5);
+    T = R.T[m == 0 ? (j < 5 ? j : 10) : (j < 5 ? 5 + j : 5)];
+  }
+  __device__ __forceinline__ void load_factor(const RosShared<LPC> &R)
+  {
+#pragma unroll
+    for (int i = 0; i < R16; ++i) {
+      const dbl2 ai = R.AI[m][16 * i + j];
+      a[i] = ai.x;
+      iv[i] = ai.y;
+      E[i] = R.E[m][16 * i + j];
+    }
+  }
+  template <int B>
+  __device__ __forceinline__ void load_block(double (&t)[LPC]) const
+  {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const dbl2 v = *reinterpret_cast<const dbl2 *>(T + 8 * B + 2 * q);
+      t[8 * B + 2 * q] = v.x;
+      t[8 * B + 2 * q + 1] = v.y;
+    }
+  }
+  template <int B>
+  __device__ __forceinline__ void store_block(const double (&t)[LPC])
+  {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      *reinterpret_cast<dbl2 *>(T + 8 * B + 2 * q) = dbl2{t[8 * B + 2 * q], t[8 * B + 2 * q + 1]};
+  }
+  template <int B, int Q = 0>
+  __device__ __forceinline__ void fwd_block(double (&t)[LPC], double &d) const
+  {
+    if constexpr (Q < 8) {
+      constexpr int k = 8 * B + Q;
+      d = (t[k] + row_bcast<k % 16>(a[k / 16]) * d) * row_bcast<k % 16>(iv[k / 16]);
+      t[k] = d;
+      fwd_block<B, Q + 1>(t, d);
+    }
+  }
+  template <int B, int Q = 7>
+  __device__ __forceinline__ void bwd_block(double (&t)[LPC], double &d) const
+  {
+    if constexpr (Q >= 0) {
+      constexpr int k = 8 * B + Q;
+      d = t[k] + row_bcast<k % 16>(E[k / 16]) * d;
+      t[k] = d;
+      bwd_block<B, Q - 1>(t, d);
+    }
+  }
+  // factor and forward sweep together: the factor's chain is a
+  // multiply-subtract, a reciprocal and a multiply per layer; every lane of
+  // the row computes it, and lane k % 16 keeps row k
+  template <int B, int Q = 0>
+  __device__ __forceinline__ void fac_block(const double (&b)[R16], const double (&c)[R16], double (&t)[LPC],
+                                            double &d, double &e)
+  {
+    if constexpr (Q < 8) {
+      constexpr int k = 8 * B + Q;
+      const double ak = row_bcast<k % 16>(a[k / 16]);
+      const double piv = row_bcast<k % 16>(b[k / 16]) - ak * e;
+      const double ivk = rcp_exact(piv);
+      e = row_bcast<k % 16>(c[k / 16]) * ivk;
+      d = (t[k] + ak * d) * ivk;
+      t[k] = d;
+      const bool mine = j == k % 16;
+      iv[k / 16] = mine ? ivk : iv[k / 16];
+      E[k / 16] = mine ? e : E[k / 16];
+      fac_block<B, Q + 1>(b, c, t, d, e);
+    }
+  }
+  template <int B = 0>
+  __device__ __forceinline__ void load_all(double (&t)[LPC], int kw) const
+  {
+    if constexpr (B < LPC / 8) {
+      if (8 * B < kw) {
+        load_block<B>(t);
+        load_all<B + 1>(t, kw);
+      }
+    }
+  }
+  template <int B = 0>
+  __device__ __forceinline__ void store_all(const double (&t)[LPC], int kw)
+  {
+    if constexpr (B < LPC / 8) {
+      if (8 * B < kw) {
+        if (own) store_block<B>(t);
+        store_all<B + 1>(t, kw);
+      }
+    }
+  }
+  template <int B = 0>
+  __device__ __forceinline__ void forward(double (&t)[LPC], double &d, int kw) const
+  {
+    if constexpr (B < LPC / 8) {
+      if (8 * B < kw) {
+        fwd_block<B>(t, d);
+        forward<B + 1>(t, d, kw);
+      }
+    }
+  }
+  template <int B = 0>
+  __device__ __forceinline__ void factor(const double (&b)[R16], const double (&c)[R16], double (&t)[LPC], double &d,
+                                         double &e, int kw)
+  {
+    if constexpr (B < LPC / 8) {
+      if (8 * B < kw) {
+        fac_block<B>(b, c, t, d, e);
+        factor<B + 1>(b, c, t, d, e, kw);
+      }
+    }
+  }
+  template <int B = LPC / 8 - 1>
+  __device__ __forceinline__ void backward(double (&t)[LPC], double &d, int kw) const
+  {
+    if constexpr (B >= 0) {
+      if (8 * B < kw) bwd_block<B>(t, d);
+      backward<B - 1>(t, d, kw);
+    }
+  }
+
+  // B z = T for the group's species; FACTOR makes the factor first.  False
+  // (with T untouched) when a pivot is outside the range of rcp_exact or a
+  // value is not finite in any active group: the LDS form then takes over.
+  template <bool FACTOR>
+  __device__ __forceinline__ bool solve(RosShared<LPC> &R, int kw)
+  {
+    double t[LPC];
+    double d = -0.0;  // a = 0 in the first row: x + 0 * -0 is x
+    bool ok = true;
+    load_all(t, kw);
+    if (FACTOR) {
+      double b[R16], c[R16], e = 0.0;
+#pragma unroll
+      for (int i = 0; i < R16; ++i) {
+        const dbl2 bc = R.BC[m][16 * i + j];
+        b[i] = bc.x;
+        c[i] = bc.y;
+        a[i] = R.AI[m][16 * i + j].x;
+        iv[i] = 1.0;
+        E[i] = 0.0;
+      }
+      factor(b, c, t, d, e, kw);
+#pragma unroll
+      for (int i = 0; i < R16; ++i) ok = ok && iv[i] > 0x1p-900 && iv[i] < 0x1p900;
+    } else {
+      forward(t, d, kw);
+    }
+    if (__any(!(ok && fabs(d) < INFINITY))) return false;
+    backward(t, d, kw);
+    store_all(t, kw);
+    return true;
+  }
+};
+
+// the most layers of the wave's columns, in a scalar register (a group that
+// has no column counts with its last one, which costs time only)
+template <int LPC>
+__device__ __forceinline__ int wave_layers(int K)
+{
+  int kw = __builtin_amdgcn_readlane(K, 0);
+  if (LPC == 32) {
+    const int k2 = __builtin_amdgcn_readlane(K, 32);
+    kw = k2 > kw ? k2 : kw;
+  }
+  return kw < LPC ? kw : LPC;
+}
+
+// B^-1 r for the lane's layer: stage through LDS, sweep, read back.  FACTOR
+// makes the factor first (from the rows in LDS).  kw: the most layers of the
+// wave's columns.
+template <int LPC, bool FACTOR>
+__device__ __forceinline__ void ros_bsolve(RosShared<LPC> &R, RosSweep<LPC> &S, int l, int K, int kw, bool act,
+                                           const double (&r)[NV], double (&v)[NV])
 {
   __builtin_amdgcn_wave_barrier();
 #pragma unroll
-  for (int n = 0; n < NV; ++n)
-    if (act) R.T[n][l] = r[n];
+  for (int n = 0; n < NV; ++n) R.T[n][l] = act ? r[n] : 0.0;
   __builtin_amdgcn_wave_barrier();
-  ros_sweep<LPC>(R, l, K);
+  bool done = false;
+  if constexpr (LPC > 16) done = S.template solve<FACTOR>(R, kw);
+  if (!done) {
+    if (FACTOR) ros_factor_lds<LPC>(R, l, K);
+    else ros_forward_lds<LPC>(R, l, K);
+    __builtin_amdgcn_wave_barrier();
+    ros_backward_lds<LPC>(R, l, K);
+    if constexpr (LPC > 16) {
+      __builtin_amdgcn_wave_barrier();
+      if (FACTOR) S.load_factor(R);
+    }
+  }
   __builtin_amdgcn_wave_barrier();
 #pragma unroll
   for (int n = 0; n < NV; ++n) v[n] = act ? R.T[n][l] : 0.0;
@@ -982,17 +1239,14 @@ __device__ __forceinline__ void ros_bsolve(RosShared<LPC> &R, int l, int K, bool
 // k = W^-1 r (AMF and one correction); r is overwritten.  Lane 0 stores
 // the stage's linearised Dirichlet top-flux terms in top[n].  Returns the
 // lane's local solve status.
-template <int LPC>
-__device__ __forceinline__ bool ros_wsolve(RosShared<LPC> &R, const KJac &J, int l, int K, bool act, double g,
-                                           unsigned dirmask, double phi, double (&r)[NV], double (&k)[NV],
-                                           double *top)
+template <int LPC, bool FACTOR>
+__device__ __forceinline__ bool ros_wsolve(RosShared<LPC> &R, RosSweep<LPC> &S, const KJac &J, const RosLane &C,
+                                           int l, int K, int kw, bool act, double g, unsigned dirmask, double phi,
+                                           double (&r)[NV], double (&k)[NV], double *top)
 {
-  // the lane's transport coefficients, read from the group's LDS
-  const double W = R.W[l];
-  const double Gn_p = l + 1 < K ? R.G[0][l + 1] : 0.0, Gn_d = l + 1 < K ? R.G[1][l + 1] : 0.0;
-  const double Gtop_p = R.G[0][0], Gtop_d = R.G[1][0];
+  const double Gn_p = lg_dn(C.Gp), Gn_d = lg_dn(C.Gd);  // used above the last layer only
   double a[NV];
-  ros_bsolve<LPC>(R, l, K, act, g, r, a);
+  ros_bsolve<LPC, FACTOR>(R, S, l, K, kw, act, r, a);
   bool ok = kjac_solve(J, g, a, k);  // k = k0
   kjac_apply(J, k, a);               // a = J_R k0
   // residual (r - k0) + g (J_T k0 + J_R k0), into r
@@ -1005,16 +1259,16 @@ __device__ __forceinline__ bool ros_wsolve(RosShared<LPC> &R, const KJac &J, int
     const double Gn = pt ? Gn_p : Gn_d;
     const double Fd = l < K - 1 ? -(Gn * (zpn - zp)) : 0.0;
     double Fu = lg_up(Fd);
-    if (l == 0) Fu = ((dirmask >> n) & 1u) ? -((pt ? Gtop_p : Gtop_d) * zp) : 0.0;
-    const double t = (Fu - Fd) * W;
+    if (l == 0) Fu = ((dirmask >> n) & 1u) ? -((pt ? C.Gp : C.Gd) * zp) : 0.0;
+    const double t = (Fu - Fd) * C.W;
     r[n] = (r[n] - k[n]) + g * (t + a[n]);
   }
-  ros_bsolve<LPC>(R, l, K, act, g, r, a);  // a = v2
+  ros_bsolve<LPC, false>(R, S, l, K, kw, act, r, a);  // a = v2
   if (l == 0) {
 #pragma unroll
     for (int n = 0; n < NV; ++n) {
       const bool pt = part(n);
-      top[n] = ((dirmask >> n) & 1u) ? 0.0 - (((pt ? Gtop_p : Gtop_d) * (pt ? phi : 1.0)) * (k[n] + a[n])) : 0.0;
+      top[n] = ((dirmask >> n) & 1u) ? 0.0 - (((pt ? C.Gp : C.Gd) * (pt ? phi : 1.0)) * (k[n] + a[n])) : 0.0;
     }
   }
   ok = kjac_solve(J, g, a, r) && ok;  // r = kc
@@ -1067,26 +1321,17 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
   double dt = 0.0, rem = 0.0;
   bool have = false, act = false;
 
+  RosLane C{0.0, 0.0, 0.0};
+  RosSweep<LPC> S;
+  S.init(R, l);
   auto coefficients = [&]() {
     // W-matrix coefficients of the record (the right-hand side's
-    // diffusivities) into the group's LDS
-    double Gp, Gd, Wl;
+    // diffusivities)
     if (ARITH == ARITH_FAST) {
-      Gp = L.Gb;
-      Gd = L.Gd;
-      Wl = L.W;
+      C = RosLane{L.Gb, L.Gd, L.W};
     } else {
       const double len = l == 0 ? L.dz : L.dzc;
-      Gp = L.Dbio / len;
-      Gd = L.Ddis / len;
-      Wl = 1.0 / (L.phi * L.dz);
-    }
-    __builtin_amdgcn_wave_barrier();
-    if (act) {
-      R.G[0][l] = Gp;
-      R.G[1][l] = Gd;
-      R.W[l] = Wl;
-      R.ph[l] = L.phi;
+      C = RosLane{L.Dbio / len, L.Ddis / len, 1.0 / (L.phi * L.dz)};
     }
     __builtin_amdgcn_wave_barrier();
   };
@@ -1163,15 +1408,14 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
       const double h = clipped ? rem : dt;
       const double gh = ROS_GAMMA * h;
       const int K = L.K;
+      const int kw = wave_layers<LPC>(K);
       double f[NV], k1[NV], k2[NV];
       double s0C, s0N, s1C = 0.0, s1N = 0.0;
       column_rhs<LPC, ARITH>(p, L, bc, x, s0C, s0N, [&](int n, double rr, double Fv) {
         f[n] = rr;
         if (l == 0) F[0][n] = Fv;
       });
-      __builtin_amdgcn_wave_barrier();
-      ros_factor<LPC>(R, l, K, gh, dirmask);
-      __builtin_amdgcn_wave_barrier();
+      ros_rows<LPC>(R, C, l, K, act, L.phi, gh, dirmask);
       // the Jacobian is evaluated again for the second stage (same values)
       // rather than kept live across the second right-hand side
       double gC = 0.0, gN = 0.0;
@@ -1179,7 +1423,7 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
       {
         KJac J;
         kin_jac(p, L.fT, x, J);
-        ok = ros_wsolve<LPC>(R, J, l, K, act, gh, dirmask, L.phi, f, k1, R.top[0]);
+        ok = ros_wsolve<LPC, true>(R, S, J, C, l, K, kw, act, gh, dirmask, L.phi, f, k1, R.top[0]);
         gC = kjac_sinkC(J, k1);
         gN = kjac_sinkN(J, k1);
       }
@@ -1199,7 +1443,7 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
         });
         KJac J;
         kin_jac(p, L.fT, x, J);
-        ok = ros_wsolve<LPC>(R, J, l, K, act, gh, dirmask, L.phi, f, k2, R.top[1]);
+        ok = ros_wsolve<LPC, false>(R, S, J, C, l, K, kw, act, gh, dirmask, L.phi, f, k2, R.top[1]);
         fail = group_any<LPC>(!ok);
         gC = gC + kjac_sinkC(J, k2);
         gN = gN + kjac_sinkN(J, k2);
