@@ -154,7 +154,7 @@ typedef struct {
 /* Schedule of adaptive integrations (sedcol_integrate).  No reference
  * counterpart: the reference steps the whole domain with one dt per
  * ode_solver call (solver_library.F90:80-189).  The default {0, 0, 1, 0}
- * integrates each layer bin in one persistent launch.  Results are identical
+ * integrates each layer bin in one persistent launch, the bins side by side.  Results are identical
  * for every schedule. */
 typedef struct {
   int32_t window;          /* attempts per column per launch; 0 = no limit */
@@ -163,7 +163,9 @@ typedef struct {
                               windows directly (one launch per step with
                               window = 1) */
   int32_t check_every;     /* direct windows launched between completion checks (>= 1) */
-  int32_t concurrent_bins; /* 1 = the layer bins run as concurrent branches */
+  int32_t concurrent_bins; /* 1 = the layer bins of a window run as concurrent
+                              branches (the bins of a persistent launch always
+                              do) */
 } sedcol_schedule;
 
 /* Kernel shape of the adaptive kernel per layer bin (bins hold the wet
