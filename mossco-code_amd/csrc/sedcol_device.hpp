@@ -140,6 +140,50 @@ __device__ __forceinline__ double drsqrt(double x)
   return y;
 }
 
+// Correctly rounded quotients without the range scaling of the IEEE
+// division: the hardware reciprocal estimate (relative error 2^-24), one
+// third-order step to the last place (rcp_near), and Markstein's correction of
+// the quotient by its residual.  They equal the IEEE division's results while
+// b and 1/b are well inside the normal range, |a| is 0 or at least 2^-970 (so
+// that the residual is exact) and the quotient is normal; callers check the
+// range.  In issue slots of 4 cycles: 10 for a division against 14, 9 for a
+// reciprocal, 3 for a division by a b whose reciprocal is at hand.
+__device__ __forceinline__ double rcp_near(double b)
+{
+  const double y = __builtin_amdgcn_rcp(b);
+  const double e = fma(-b, y, 1.0);
+  return fma(y, fma(e, e, e), y);
+}
+__device__ __forceinline__ double rcp_exact(double b)
+{
+  const double y = rcp_near(b);
+  return fma(fma(-b, y, 1.0), y, y);
+}
+// a / b with y = 1/b rounded
+__device__ __forceinline__ double div_by(double a, double b, double y)
+{
+  const double q = a * y;
+  return fma(fma(-b, q, a), y, q);
+}
+template <bool FD>
+__device__ __forceinline__ double quot(double a, double b)
+{
+  if constexpr (FD) return div_by(a, b, rcp_near(b));
+  else return a / b;
+}
+template <bool FD>
+__device__ __forceinline__ double recip(double b)
+{
+  if constexpr (FD) return rcp_exact(b);
+  else return 1.0 / b;
+}
+// |v| is 0 or in [2^lo, 2^hi]
+__device__ __forceinline__ bool in_range(double v, int lo, int hi)
+{
+  const int e = __builtin_amdgcn_frexp_exp(v);  // 0 for 0
+  return e > lo && e <= hi && fabs(v) < INFINITY;
+}
+
 // temperature factor of get_rhs, fabm_sediment_driver.F90:648
 __device__ __forceinline__ double temp_factor(double T)
 {
@@ -153,7 +197,9 @@ __device__ __forceinline__ double temp_factor(double T)
 // (fabm_sediment_driver.F90:700); that module is not part of the reference,
 // so this is the library's own definition.  Each destruction term is
 // proportional to the destroyed species.  sC = DIC release, sN = N2 release.
-template <int ARITH>
+// FD: the reference form's divisions by quot<true> (the caller has checked
+// the ranges).
+template <int ARITH, bool FD = false>
 __device__ __forceinline__ void kinetics(const sedcol_params &p, double fT, const double (&c)[NV], double (&R)[NV],
                                          double &sC, double &sN)
 {
@@ -165,7 +211,7 @@ __device__ __forceinline__ void kinetics(const sedcol_params &p, double fT, cons
   double kS = fT * p.rS;
   double dL = kL * ldC;
   double dS = kS * sdC;
-  double lim = p.CprodMax / (p.CprodMax + (dL + dS));
+  double lim = quot<FD>(p.CprodMax, p.CprodMax + (dL + dS));
   double CpL = dL * lim;
   double CpS = dS * lim;
   double Cprod = CpL + CpS;
@@ -175,12 +221,12 @@ __device__ __forceinline__ void kinetics(const sedcol_params &p, double fT, cons
 
   double oxlim, dnlim, anlim, nitlim, o2odu, odulim;
   if (ARITH != ARITH_FAST) {
-    oxlim = O2 / (O2 + p.ksO2oxic);
-    dnlim = (p.kinO2denit / (O2 + p.kinO2denit)) * (NO3 / (NO3 + p.ksNO3denit));
-    anlim = (p.kinO2anox / (O2 + p.kinO2anox)) * (p.kinNO3anox / (NO3 + p.kinNO3anox));
-    nitlim = O2 / (O2 + p.ksO2nitri);
-    o2odu = O2 / (O2 + p.ksO2oduox);
-    odulim = ODU / (ODU + p.PAdsODU);
+    oxlim = quot<FD>(O2, O2 + p.ksO2oxic);
+    dnlim = quot<FD>(p.kinO2denit, O2 + p.kinO2denit) * quot<FD>(NO3, NO3 + p.ksNO3denit);
+    anlim = quot<FD>(p.kinO2anox, O2 + p.kinO2anox) * quot<FD>(p.kinNO3anox, NO3 + p.kinNO3anox);
+    nitlim = quot<FD>(O2, O2 + p.ksO2nitri);
+    o2odu = quot<FD>(O2, O2 + p.ksO2oduox);
+    odulim = quot<FD>(ODU, ODU + p.PAdsODU);
   } else {
     // the six Monod denominators share one reciprocal of their product,
     // split back with prefix/suffix products (range: concentrations < 1e30,
@@ -201,7 +247,7 @@ __device__ __forceinline__ void kinetics(const sedcol_params &p, double fT, cons
     o2odu = O2 * ((inv * a2346) * q8);
     odulim = ODU * (inv * a23467);
   }
-  double rescale = 1.0 / ((oxlim + dnlim) + anlim);
+  double rescale = recip<FD>((oxlim + dnlim) + anlim);
   double OxicMin = (Cprod * oxlim) * rescale;
   double Denit = (Cprod * dnlim) * rescale;
   double AnoxMin = (Cprod * anlim) * rescale;
@@ -477,8 +523,14 @@ struct Lane {
   bool active;  // l < K
   double phi;
   double fT;
-  // reference form: geometry and interface diffusivities
+  // reference form: geometry and interface diffusivities (dzc is dz on the
+  // top layer, whose flux is taken over dz)
   double dz, dzc, Dbio, Ddis;
+  // reference form: reciprocals of its divisors dzc, (1 - phi) dz, phi dz and
+  // phi, and whether the column has a value outside the range in which a
+  // division by them is exact
+  double ydzc, yVp, yVd, yphi;
+  bool wide;
   // fast form: Dbio/dzc, Ddis/dzc (D/dz on the top layer), 1/(phi dz)
   double Gb, Gd, W;
   // distributed-POM flux cap of the layer (bcup_part = 4; 0 when unset)
@@ -511,38 +563,82 @@ __device__ __forceinline__ void diffusivities(const sedcol_params &p, double B, 
   if (ARITH != ARITH_FAST) {
     L.Dbio = Dbio;
     L.Ddis = Ddis;
+    if (ARITH == ARITH_REF) {
+      L.ydzc = 1.0 / L.dzc;
+      L.yVp = 1.0 / ((1.0 - L.phi) * L.dz);
+      L.yVd = 1.0 / (L.phi * L.dz);
+      L.yphi = 1.0 / L.phi;
+    }
     if (ARITH == ARITH_EXT) {
       // profile 3: B = f_T = 1 (fabm_sediment_driver.F90:622-623)
       L.zq = (((1.0 * 1.0) / 86400.0) / 10000.0) * (1.0 - phiI);
       L.Dmol = Dmol;
     }
   } else {
-    const double len = L.l == 0 ? L.dz : L.dzc;
-    L.Gb = Dbio / len;
-    L.Gd = Ddis / len;
+    L.Gb = Dbio / L.dzc;
+    L.Gd = Ddis / L.dzc;
     L.W = 1.0 / (L.phi * L.dz);
   }
 }
 
+// Ranges in which the reference form's divisions are exact by reciprocals.
+// With states in 0 or [2^-500, 2^500], diffusivities and rates in 0 or
+// [2^-100, 2^100] and divisors in [2^-60, 2^60], every dividend of a
+// right-hand side is 0 or at least 2^-946: a difference of two states or two
+// fluxes is 0 or no less than the last place of the smaller one, and each
+// product or quotient takes off what its factors allow.
+constexpr int kStateLo = -500, kStateHi = 500;
+__device__ __forceinline__ bool rate_ok(double v) { return in_range(v, -100, 100); }
+__device__ __forceinline__ bool divisor_ok(double v) { return v != 0.0 && in_range(v, -60, 60); }
+__device__ __forceinline__ bool params_ok(const sedcol_params &p)
+{
+  return divisor_ok(p.CprodMax) && divisor_ok(p.ksO2nitri) && divisor_ok(p.ksO2oduox) && divisor_ok(p.ksO2oxic) &&
+         divisor_ok(p.ksNO3denit) && divisor_ok(p.kinO2denit) && divisor_ok(p.kinNO3anox) && divisor_ok(p.kinO2anox) &&
+         divisor_ok(p.PAdsODU) && rate_ok(p.rL) && rate_ok(p.rS) && p.CprodMax > 0.0 && p.ksO2nitri > 0.0 &&
+         p.ksO2oduox > 0.0 && p.ksO2oxic > 0.0 && p.ksNO3denit > 0.0 && p.kinO2denit > 0.0 && p.kinNO3anox > 0.0 &&
+         p.kinO2anox > 0.0 && p.PAdsODU > 0.0 && p.rL >= 0.0 && p.rS >= 0.0;
+}
+__device__ __forceinline__ bool lane_ok(const Lane &L)
+{
+  return rate_ok(L.Dbio) && rate_ok(L.Ddis) && divisor_ok(L.fT) && divisor_ok(L.dzc) && divisor_ok(L.phi) &&
+         divisor_ok(1.0 - L.phi) && divisor_ok((1.0 - L.phi) * L.dz) && divisor_ok(L.phi * L.dz);
+}
+// every state of the layer in range: the least exponent (0 for a zero), and
+// the sum of the magnitudes for the largest, infinities and NaN
+__device__ __forceinline__ bool state_ok(const double (&c)[NV])
+{
+  int e = 0;
+  double m = 0.0;
+#pragma unroll
+  for (int n = 0; n < NV; ++n) {
+    const int en = __builtin_amdgcn_frexp_exp(c[n]);
+    e = en < e ? en : e;
+    m = m + fabs(c[n]);
+  }
+  return e > kStateLo && m < 0x1p500;
+}
+
 // One get_rhs evaluation for the lane's layer.  sbc[0..NV) bottom-water
-// concentrations, sbc[NV..2NV) prescribed top fluxes (LDS, per group).
+// concentrations, sbc[NV..2NV) top fluxes (LDS, per group; load_forcing puts
+// 0 for a closed top).
 // For each variable n the callback receives (n, rhs_n, F) where F is the flux
 // through the lane's upper interface (lane 0: the top flux intFlux(:,:,1)).
 // Transport: diff3d (fabm_sediment_driver.F90:739-825) with the particulate
 // bulk/volume-fraction handling of get_rhs :658-678 and dissolved :680-692.
 // The fast form requires bcdown != 2.
-template <int LPC, int ARITH, class CB>
-__device__ __forceinline__ void column_rhs(const sedcol_params &p, const Lane &L, const double *sbc,
-                                           const double (&c)[NV], double &sC, double &sN, CB &&cb,
-                                           const ZwDev *zw = nullptr)
+// The top layer's flux is the given one (bcup 1, 3 and 4) or, with bcup 2,
+// the same expression as the interior's against the bottom water: a select,
+// so that the evaluation is one stretch of code over all variables.
+// FD: divisions by reciprocals (reference form).
+template <int LPC, int ARITH, bool FD, class CB>
+__device__ __forceinline__ void column_terms(const sedcol_params &p, const Lane &L, const double *sbc,
+                                             const double (&c)[NV], double &sC, double &sN, CB &&cb, const ZwDev *zw)
 {
-  // Callbacks may stage values in LDS for other lanes of the same wave; the
-  // wave barriers keep those accesses ordered around the evaluation.
-  __builtin_amdgcn_wave_barrier();
   double R[NV];
-  kinetics<ARITH>(p, L.fT, c, R, sC, sN);
+  kinetics<ARITH, FD>(p, L.fT, c, R, sC, sN);
   const bool top = L.l == 0;
   const bool bottom = L.l == L.K - 1;
+  const bool givenp = top && p.bcup_part != 2, givend = top && p.bcup_dis != 2;
   double Dbio = ARITH != ARITH_FAST ? L.Dbio : 0.0;
   double Ddis = ARITH != ARITH_FAST ? L.Ddis : 0.0;
   if (ARITH == ARITH_EXT && zw && zw->on) {
@@ -564,22 +660,14 @@ __device__ __forceinline__ void column_rhs(const sedcol_params &p, const Lane &L
     const bool pt = part(n);
     const double x = pt ? c[n] * L.phi : c[n];
     const double xup = lg_up(x);
-    const int bc = pt ? p.bcup_part : p.bcup_dis;
+    const double xo = top ? sbc[n] : xup;
     double F;
     if (ARITH != ARITH_FAST) {
       const double D = pt ? Dbio : Ddis;
-      {
-        // one flux expression for the top (bcup = 2, against the bottom
-        // water over dz) and the interior (against the layer above over
-        // dzc), then a select: the same operations as two branches, without
-        // the divergent control flow around every variable
-        const double xo = top ? sbc[n] : xup;
-        const double den = top ? L.dz : L.dzc;
-        const double Fd = -((D * (x - xo)) / den);
-        const double Ft = (bc == 1 || bc == 4) ? sbc[NV + n] : bc == 2 ? Fd : 0.0;
-        F = top ? Ft : Fd;
-      }
-      if (ARITH == ARITH_EXT && bc == 4) {
+      const double num = D * (x - xo);
+      const double Fd = -(FD ? div_by(num, L.dzc, L.ydzc) : num / L.dzc);
+      F = (pt ? givenp : givend) ? sbc[NV + n] : Fd;
+      if (ARITH == ARITH_EXT && pt && p.bcup_part == 4) {
         // diff3d BcUp = 4 (fabm_sediment_driver.F90:791-802): the top flux
         // beyond the first layer's cap is added to the interfaces below,
         // each layer's cap taken off in turn, sequentially as written there;
@@ -603,17 +691,16 @@ __device__ __forceinline__ void column_rhs(const sedcol_params &p, const Lane &L
       double Fdn = lg_dn(F);
       if (bottom) Fdn = p.bcdown == 2 ? -((D * (0.0 - x)) / L.dz) : 0.0;
       const double VF = pt ? (1.0 - L.phi) : L.phi;
-      const double dC = (F - Fdn) / (VF * L.dz);
-      const double Q = pt ? (dC * (1.0 - L.phi)) / L.phi : dC;
+      const double V = VF * L.dz;
+      const double dF = F - Fdn;
+      const double dC = FD ? div_by(dF, V, pt ? L.yVp : L.yVd) : dF / V;
+      double Q = dC;
+      if (pt) Q = FD ? div_by(dC * (1.0 - L.phi), L.phi, L.yphi) : (dC * (1.0 - L.phi)) / L.phi;
       cb(n, R[n] + Q, F);
     } else {
       const double G = pt ? L.Gb : L.Gd;
-      {
-        const double xo = top ? sbc[n] : xup;
-        const double Fd = -(G * (x - xo));
-        const double Ft = bc == 1 ? sbc[NV + n] : bc == 2 ? Fd : 0.0;
-        F = top ? Ft : Fd;
-      }
+      const double Fd = -(G * (x - xo));
+      F = (pt ? givenp : givend) ? sbc[NV + n] : Fd;
       // the lane exchange runs on every lane (a lane outside the exec mask
       // reads as 0 to the lane above it), then the bottom value replaces it;
       // written as a select on lg_dn's result it would only be evaluated
@@ -623,6 +710,22 @@ __device__ __forceinline__ void column_rhs(const sedcol_params &p, const Lane &L
       const double Q = (F - Fdn) * L.W;
       cb(n, R[n] + Q, F);
     }
+  }
+}
+
+template <int LPC, int ARITH, class CB>
+__device__ __forceinline__ void column_rhs(const sedcol_params &p, const Lane &L, const double *sbc,
+                                           const double (&c)[NV], double &sC, double &sN, CB &&cb,
+                                           const ZwDev *zw = nullptr)
+{
+  // Callbacks may stage values in LDS for other lanes of the same wave; the
+  // wave barriers keep those accesses ordered around the evaluation.
+  __builtin_amdgcn_wave_barrier();
+  if constexpr (ARITH == ARITH_REF) {
+    if (__any(L.active && (L.wide || !state_ok(c)))) column_terms<LPC, ARITH, false>(p, L, sbc, c, sC, sN, cb, zw);
+    else column_terms<LPC, ARITH, true>(p, L, sbc, c, sC, sN, cb, zw);
+  } else {
+    column_terms<LPC, ARITH, false>(p, L, sbc, c, sC, sN, cb, zw);
   }
   __builtin_amdgcn_wave_barrier();
 }
@@ -834,9 +937,8 @@ __device__ __forceinline__ void column_rhs2(const sedcol_params &p, const Lane (
     if (ARITH == ARITH_REF) {
       const double D0 = pt ? L[0].Dbio : L[0].Ddis;
       const double D1 = pt ? L[1].Dbio : L[1].Ddis;
-      double F0;
-      if (top) F0 = (bc == 1 || bc == 4) ? sbc[NV + n] : bc == 2 ? -((D0 * (x0 - sbc[n])) / L[0].dz) : 0.0;
-      else F0 = -((D0 * (x0 - xup)) / L[0].dzc);
+      double F0 = -((D0 * (x0 - (top ? sbc[n] : xup))) / L[0].dzc);
+      if (top && bc != 2) F0 = sbc[NV + n];
       const double F1 = -((D1 * (x1 - x0)) / L[1].dzc);
       double Fdn0 = F1;
       if (bottom0) Fdn0 = p.bcdown == 2 ? -((D0 * (0.0 - x0)) / L[0].dz) : 0.0;
@@ -853,9 +955,8 @@ __device__ __forceinline__ void column_rhs2(const sedcol_params &p, const Lane (
     } else {
       const double G0 = pt ? L[0].Gb : L[0].Gd;
       const double G1 = pt ? L[1].Gb : L[1].Gd;
-      double F0;
-      if (top) F0 = bc == 1 ? sbc[NV + n] : bc == 2 ? -(G0 * (x0 - sbc[n])) : 0.0;
-      else F0 = -(G0 * (x0 - xup));
+      double F0 = -(G0 * (x0 - (top ? sbc[n] : xup)));
+      if (top && bc != 2) F0 = sbc[NV + n];
       const double F1 = -(G1 * (x1 - x0));
       double Fdn0 = F1;
       if (bottom0) Fdn0 = 0.0;

@@ -34,7 +34,7 @@ __device__ __forceinline__ void setup_lane(const Dev &d, int c, int l, Lane &L, 
   L.active = l < L.K;
   cell = (long long)o + l;
   L.dz = L.active ? d.dz[cell] : 1.0;
-  L.dzc = (L.active && l > 0) ? d.dzc[cell] : 1.0;
+  L.dzc = L.active ? (l > 0 ? d.dzc[cell] : L.dz) : 1.0;
   L.phi = L.active ? d.phi[cell] : 0.5;
   G.phiI = L.active ? d.phiI[cell] : 0.5;
   L.cap = (L.active && d.fcap) ? d.fcap[cell] : 0.0;
@@ -45,24 +45,49 @@ __device__ __forceinline__ void setup_lane(const Dev &d, int c, int l, Lane &L, 
   G.B = d.biot[c];
 }
 
-// load forcing record r of column c: bottom-water concentrations and top
-// fluxes to the group's LDS slot, temperature-dependent coefficients to L
-template <int ARITH>
-__device__ __forceinline__ void load_forcing(const Dev &d, const sedcol_params &p, int c, int r, const Geo &G,
-                                             Lane &L, double *sbc)
-{
-  if (L.l < NV) {
-    sbc[L.l] = d.cbw[((long long)r * NV + L.l) * d.ncol + c];
-    sbc[NV + L.l] = d.fup[(long long)r * d.fup_rec_stride + (long long)L.l * d.ncol + c];
-  }
-  const double T = d.temp[(long long)r * d.ncol + c];
-  diffusivities<ARITH>(p, G.B, T, G.phiI, G.bfac, L);
-}
-
 template <int LPC>
 __device__ __forceinline__ bool group_any(bool b)
 {
   return lg_max<LPC>(b ? 1.0 : 0.0) > 0.0;
+}
+
+// load forcing record r of column c: bottom-water concentrations and top
+// fluxes (0 for a closed top) to the group's LDS slot, temperature-dependent
+// coefficients to L
+__device__ __forceinline__ bool load_top(const Dev &d, const sedcol_params &p, int c, int r, int n, double *sbc)
+{
+  const int bc = part(n) ? p.bcup_part : p.bcup_dis;
+  const double w = d.cbw[((long long)r * NV + n) * d.ncol + c];
+  const double f = d.fup[(long long)r * d.fup_rec_stride + (long long)n * d.ncol + c];
+  const double t = (bc == 1 || bc == 4) ? f : 0.0;
+  sbc[n] = w;
+  sbc[NV + n] = t;
+  return in_range(w, kStateLo, kStateHi) && in_range(t, kStateLo, kStateHi);
+}
+
+template <int LPC, int ARITH>
+__device__ __forceinline__ void load_forcing(const Dev &d, const sedcol_params &p, int c, int r, const Geo &G,
+                                             Lane &L, double *sbc)
+{
+  bool ok = true;
+  if (L.l < NV) ok = load_top(d, p, c, r, L.l, sbc);
+  const double T = d.temp[(long long)r * d.ncol + c];
+  diffusivities<ARITH>(p, G.B, T, G.phiI, G.bfac, L);
+  if (ARITH == ARITH_REF) {
+    ok = ok && params_ok(p) && (!L.active || lane_ok(L));
+    L.wide = group_any<LPC>(!ok);
+  }
+}
+
+// top fluxes of one right-hand side, held by the group's first lane, into the
+// group's LDS slot: one branch for all variables
+__device__ __forceinline__ void store_top(bool first, const double (&Ft)[NV], double *F)
+{
+  if (first) {
+#pragma unroll
+    for (int n = 0; n < NV; ++n) F[n] = Ft[n];
+  }
+  __builtin_amdgcn_wave_barrier();
 }
 
 // ---------------------------------------------------------------------------
@@ -84,7 +109,7 @@ __global__ __launch_bounds__(BLOCK) void k_rhs(Dev d, const int *list, int nlist
   long long cell = 0;
   if (valid) {
     setup_lane(d, c, l, L, Gm, cell);
-    load_forcing<ARITH>(d, p, c, rec, Gm, L, sbc[g]);
+    load_forcing<LPC, ARITH>(d, p, c, rec, Gm, L, sbc[g]);
   }
   __syncthreads();
   if (!valid) return;
@@ -124,11 +149,15 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
   long long cell = 0;
   if (valid) {
     setup_lane(d, c, l, L, Gm, cell);
-    load_forcing<ARITH>(d, p, c, rec, Gm, L, sbc[g]);
+    load_forcing<LPC, ARITH>(d, p, c, rec, Gm, L, sbc[g]);
   }
   __syncthreads();
   if (!valid) return;
-  const double *bc = sbc[g];
+  // the boundary values stay in registers for the whole run: read from LDS in
+  // every right-hand side, they cost a lone wave 1600 of 4900 cycles
+  double bc[2 * NV];
+#pragma unroll
+  for (int n = 0; n < 2 * NV; ++n) bc[n] = sbc[g][n];
   double(*F)[NV] = sF[g];
   const bool act = L.active;
   const bool own = l < NV;  // lane l accumulates the top flux of variable l
@@ -150,13 +179,14 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
   const double third = 1.0 / 3.0;
 
   for (int s = 0; s < nsteps; ++s) {
-    double sC, sN;
+    double sC, sN, Ft[NV];
     if (METHOD == SEDCOL_EULER) {
       double r0[NV];
       column_rhs<LPC, ARITH>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
         r0[n] = r;
-        if (l == 0) F[0][n] = Fv;
+        Ft[n] = Fv;
       }, &d.zw);
+      store_top(l == 0, Ft, F[0]);
 #pragma unroll
       for (int n = 0; n < NV; ++n) x[n] = x[n] + dt * r0[n];
       if (own) {
@@ -172,28 +202,32 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       column_rhs<LPC, ARITH>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
         k[n] = 0.5 * r;
         cs[n] = x[n] + (0.5 * dt) * r;
-        if (l == 0) F[0][n] = Fv;
+        Ft[n] = Fv;
       }, &d.zw);
+      store_top(l == 0, Ft, F[0]);
       aC = 0.5 * sC;
       aN = 0.5 * sN;
       column_rhs<LPC, ARITH>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k[n] = k[n] + r;
         cs[n] = x[n] + (0.5 * dt) * r;
-        if (l == 0) F[1][n] = Fv;
+        Ft[n] = Fv;
       }, &d.zw);
+      store_top(l == 0, Ft, F[1]);
       aC = aC + sC;
       aN = aN + sN;
       column_rhs<LPC, ARITH>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k[n] = k[n] + r;
         cs[n] = x[n] + dt * r;
-        if (l == 0) F[2][n] = Fv;
+        Ft[n] = Fv;
       }, &d.zw);
+      store_top(l == 0, Ft, F[2]);
       aC = aC + sC;
       aN = aN + sN;
       column_rhs<LPC, ARITH>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k[n] = k[n] + 0.5 * r;
-        if (l == 0) F[3][n] = Fv;
+        Ft[n] = Fv;
       }, &d.zw);
+      store_top(l == 0, Ft, F[3]);
       aC = aC + 0.5 * sC;
       aN = aN + 0.5 * sN;
       const double w = dt * third;
@@ -212,28 +246,32 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       column_rhs<LPC, ARITH>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
         k1[n] = r;
         cs[n] = x[n] + (third * dt) * r;
-        if (l == 0) F[0][n] = Fv;
+        Ft[n] = Fv;
       }, &d.zw);
+      store_top(l == 0, Ft, F[0]);
       s1C = sC;
       s1N = sN;
       column_rhs<LPC, ARITH>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k2[n] = r;
         cs[n] = x[n] + dt * (r - third * k1[n]);
-        if (l == 0) F[1][n] = Fv;
+        Ft[n] = Fv;
       }, &d.zw);
+      store_top(l == 0, Ft, F[1]);
       s2C = sC;
       s2N = sN;
       column_rhs<LPC, ARITH>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         cs[n] = x[n] + dt * ((k1[n] - k2[n]) + r);
         k1[n] = (k1[n] + 3.0 * k2[n]) + 3.0 * r;
-        if (l == 0) F[2][n] = Fv;
+        Ft[n] = Fv;
       }, &d.zw);
+      store_top(l == 0, Ft, F[2]);
       double aC = (s1C + 3.0 * s2C) + 3.0 * sC;
       double aN = (s1N + 3.0 * s2N) + 3.0 * sN;
       column_rhs<LPC, ARITH>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k1[n] = k1[n] + r;
-        if (l == 0) F[3][n] = Fv;
+        Ft[n] = Fv;
       }, &d.zw);
+      store_top(l == 0, Ft, F[3]);
       aC = aC + sC;
       aN = aN + sN;
       const double w = (dt * 1.0) / 8.0;
@@ -249,8 +287,9 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       double f0[NV];
       column_rhs<LPC, ARITH>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
         f0[n] = r;
-        if (l == 0) F[0][n] = Fv;
+        Ft[n] = Fv;
       }, &d.zw);
+      store_top(l == 0, Ft, F[0]);
       const double p1 = pfactor<LPC, false, PW, BLOCK>(x, f0, x, dt, act, zs, dg.newton, &sgeo[0][threadIdx.x]);
       if (p1 < dg.p_min) dg.p_min = p1;
       if (METHOD == SEDCOL_EMP1) {
@@ -272,8 +311,9 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
         const double s0C = sC, s0N = sN;
         column_rhs<LPC, ARITH>(p, L, bc, c1, sC, sN, [&](int n, double r, double Fv) {
           f0[n] = (f0[n] + r) * 0.5;
-          if (l == 0) F[1][n] = Fv;
+          Ft[n] = Fv;
         }, &d.zw);
+      store_top(l == 0, Ft, F[1]);
         const double p2 = pfactor<LPC, true, PW, BLOCK>(x, f0, c1, dt, act, zs, dg.newton, &sgeo[0][threadIdx.x]);
         if (p2 < dg.p_min) dg.p_min = p2;
 #pragma unroll
@@ -286,25 +326,31 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
         kadd(acc[1], accc[1], (dt * p2) * ((s0N + sN) * 0.5));
       }
     }
-    // clamp: Patankar rounding guard (EMP), or the callers' minimum clamp
-    if (METHOD >= SEDCOL_EMP1 || p.clamp) {
-#pragma unroll
-      for (int n = 0; n < NV; ++n)
-        if (x[n] < 0.0) {
-          if (elem(n) >= 0) kadd(acc[2 + elem(n)], accc[2 + elem(n)], 0.0 - x[n]);
-          x[n] = 0.0;
-        }
-    }
-    bool nan = false;
-#pragma unroll
-    for (int n = 0; n < NV; ++n) nan |= act && (x[n] != x[n]);
     dg.accepted += 1;
     dg.dt_last = dt;
     if (dt < dg.dt_minacc) dg.dt_minacc = dt;
-    if (group_any<LPC>(nan)) {
-      dg.status = 1;
-      if (l == 0) atomicOr(errflag, 1);
-      break;
+    // clamp: Patankar rounding guard (EMP), or the callers' minimum clamp;
+    // one test for negative values and NaN, most steps have neither
+    bool odd = false;
+#pragma unroll
+    for (int n = 0; n < NV; ++n) odd |= !(x[n] >= 0.0);
+    if (__any(odd)) {
+      if (METHOD >= SEDCOL_EMP1 || p.clamp) {
+#pragma unroll
+        for (int n = 0; n < NV; ++n)
+          if (x[n] < 0.0) {
+            if (elem(n) >= 0) kadd(acc[2 + elem(n)], accc[2 + elem(n)], 0.0 - x[n]);
+            x[n] = 0.0;
+          }
+      }
+      bool nan = false;
+#pragma unroll
+      for (int n = 0; n < NV; ++n) nan |= act && (x[n] != x[n]);
+      if (group_any<LPC>(nan)) {
+        dg.status = 1;
+        if (l == 0) atomicOr(errflag, 1);
+        break;
+      }
     }
   }
 
@@ -436,7 +482,7 @@ __global__ __launch_bounds__(BLK, SEDCOL_EMP_MIN_WAVES) void k_emp_adaptive(
       have = true;
       if (rem > 0.0) {
         // resumed inside record r
-        load_forcing<ARITH>(d, p, c, r, Gm, L, sbc[g]);
+        load_forcing<LPC, ARITH>(d, p, c, r, Gm, L, sbc[g]);
         __builtin_amdgcn_wave_barrier();
       }
     }
@@ -452,7 +498,7 @@ __global__ __launch_bounds__(BLK, SEDCOL_EMP_MIN_WAVES) void k_emp_adaptive(
         const double a = ctl.t_start > lo ? ctl.t_start : lo;
         const double b = ctl.t_end < hi ? ctl.t_end : hi;
         rem = b - a;
-        load_forcing<ARITH>(d, p, c, r, Gm, L, sbc[g]);
+        load_forcing<LPC, ARITH>(d, p, c, r, Gm, L, sbc[g]);
         __builtin_amdgcn_wave_barrier();
         continue;
       }
@@ -619,10 +665,7 @@ template <int ARITH>
 __device__ __forceinline__ void load_forcing2(const Dev &d, const sedcol_params &p, int c, int r, int l,
                                               const Geo (&G)[2], Lane (&L)[2], double *sbc)
 {
-  if (l < NV) {
-    sbc[l] = d.cbw[((long long)r * NV + l) * d.ncol + c];
-    sbc[NV + l] = d.fup[(long long)r * d.fup_rec_stride + (long long)l * d.ncol + c];
-  }
+  if (l < NV) (void)load_top(d, p, c, r, l, sbc);
   const double T = d.temp[(long long)r * d.ncol + c];
   diffusivities<ARITH>(p, G[0].B, T, G[0].phiI, G[0].bfac, L[0]);
   diffusivities<ARITH>(p, G[1].B, T, G[1].phiI, G[1].bfac, L[1]);
@@ -912,17 +955,6 @@ struct alignas(16) RosShared {
 struct RosLane {
   double Gp, Gd, W;
 };
-
-// correctly rounded 1/b for b well inside the normal range: the hardware
-// estimate (relative error 2^-24), one third-order step to the last place,
-// and Markstein's final correction
-__device__ __forceinline__ double rcp_exact(double b)
-{
-  double y = __builtin_amdgcn_rcp(b);
-  const double e = fma(-b, y, 1.0);
-  y = fma(y, fma(e, e, e), y);
-  return fma(fma(-b, y, 1.0), y, y);
-}
 
 // Matrix rows of both classes, one layer per lane: everything of the Thomas
 // factorisation that is not on its serial chain.  Lanes beyond the column
@@ -1330,8 +1362,7 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
     if (ARITH == ARITH_FAST) {
       C = RosLane{L.Gb, L.Gd, L.W};
     } else {
-      const double len = l == 0 ? L.dz : L.dzc;
-      C = RosLane{L.Dbio / len, L.Ddis / len, 1.0 / (L.phi * L.dz)};
+      C = RosLane{L.Dbio / L.dzc, L.Ddis / L.dzc, 1.0 / (L.phi * L.dz)};
     }
     __builtin_amdgcn_wave_barrier();
   };
@@ -1371,7 +1402,7 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
       wn = 0;
       have = true;
       if (rem > 0.0) {
-        load_forcing<ARITH>(d, p, c, r, Gm, L, sbc[g]);
+        load_forcing<LPC, ARITH>(d, p, c, r, Gm, L, sbc[g]);
         coefficients();
       }
     }
@@ -1386,7 +1417,7 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
         const double a = ctl.t_start > lo ? ctl.t_start : lo;
         const double b = ctl.t_end < hi ? ctl.t_end : hi;
         rem = b - a;
-        load_forcing<ARITH>(d, p, c, r, Gm, L, sbc[g]);
+        load_forcing<LPC, ARITH>(d, p, c, r, Gm, L, sbc[g]);
         coefficients();
         continue;
       }
@@ -1411,10 +1442,12 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
       const int kw = wave_layers<LPC>(K);
       double f[NV], k1[NV], k2[NV];
       double s0C, s0N, s1C = 0.0, s1N = 0.0;
+      double Ft[NV];
       column_rhs<LPC, ARITH>(p, L, bc, x, s0C, s0N, [&](int n, double rr, double Fv) {
         f[n] = rr;
-        if (l == 0) F[0][n] = Fv;
+        Ft[n] = Fv;
       });
+      store_top(l == 0, Ft, F[0]);
       ros_rows<LPC>(R, C, l, K, act, L.phi, gh, dirmask);
       // the Jacobian is evaluated again for the second stage (same values)
       // rather than kept live across the second right-hand side
@@ -1439,8 +1472,9 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
         for (int n = 0; n < NV; ++n) c1[n] = f[n];
         column_rhs<LPC, ARITH>(p, L, bc, c1, s1C, s1N, [&](int n, double rr, double Fv) {
           f[n] = rr - 2.0 * k1[n];
-          if (l == 0) F[1][n] = Fv;
+          Ft[n] = Fv;
         });
+        store_top(l == 0, Ft, F[1]);
         KJac J;
         kin_jac(p, L.fT, x, J);
         ok = ros_wsolve<LPC, false>(R, S, J, C, l, K, kw, act, gh, dirmask, L.phi, f, k2, R.top[1]);
@@ -1484,15 +1518,21 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
         if (fac < 0.2) fac = 0.2;
         if (fac > 5.0) fac = 5.0;
         if (accept) {
+          bool odd = false;
 #pragma unroll
           for (int n = 0; n < NV; ++n) {
-            double y = x[n] + h * (1.5 * k1[n] + 0.5 * k2[n]);
-            if (y < 0.0) {
-              if (elem(n) >= 0 && act)
-                kadd(d.cellacc[(2 + elem(n)) * d.ncell + cell], d.cellacc[(7 + elem(n)) * d.ncell + cell], 0.0 - y);
-              y = 0.0;
-            }
-            x[n] = y;
+            x[n] = x[n] + h * (1.5 * k1[n] + 0.5 * k2[n]);
+            odd |= x[n] < 0.0;
+          }
+          if (__any(odd)) {
+#pragma unroll
+            for (int n = 0; n < NV; ++n)
+              if (x[n] < 0.0) {
+                if (elem(n) >= 0 && act)
+                  kadd(d.cellacc[(2 + elem(n)) * d.ncell + cell], d.cellacc[(7 + elem(n)) * d.ncell + cell],
+                       0.0 - x[n]);
+                x[n] = 0.0;
+              }
           }
           __builtin_amdgcn_wave_barrier();
           if (own) {
@@ -1574,7 +1614,7 @@ __global__ __launch_bounds__(BLOCK) void k_rhs_store(Dev d, const int *list, int
   long long cell = 0;
   if (valid) {
     setup_lane(d, c, l, L, Gm, cell);
-    load_forcing<ARITH>(d, p, c, rec, Gm, L, sbc[g]);
+    load_forcing<LPC, ARITH>(d, p, c, rec, Gm, L, sbc[g]);
   }
   __syncthreads();
   if (!valid) return;
@@ -1652,16 +1692,24 @@ __global__ __launch_bounds__(BLOCK) void k_ae_commit(Dev d, const int *list, int
 // stays in registers; the top fluxes of the last right-hand side go to LDS
 // for the lanes that accumulate them.  *min_dt receives the smallest step
 // taken.  A launch stops after kAeFusedMaxAttempts attempts (errflag bit 2).
-template <int LPC, int ARITH>
-__global__ __launch_bounds__(kAeFusedBlock) void k_ae_fused(const Dev *dptr, const int *list, int nlist,
-                                                           const sedcol_params *__restrict__ pptr, int rec, double dt,
-                                                           int nsteps, int *errflag, double *min_dt)
+// The time is that of one dependent chain, so a domain of one wave runs as a
+// block of one wave (BLK = 64): the vote and the barriers stay inside the
+// wave and a lane has all the registers it asks for.
+template <int LPC, int ARITH, int BLK>
+__global__ __launch_bounds__(BLK) void k_ae_fused(const Dev *dptr, const int *list, int nlist,
+                                                  const sedcol_params *__restrict__ pptr, int rec, double dt,
+                                                  int nsteps, int *errflag, double *min_dt)
 {
   // domain and parameters through pointers to device copies: passed by
   // value they would sit in scalar registers for the whole run and spill
   const Dev &d = *dptr;
   const sedcol_params &p = *pptr;
-  constexpr int G = kAeFusedBlock / LPC;
+  constexpr int G = BLK / LPC;
+  constexpr bool ONE = BLK == 64;  // one wave
+  auto sync = [] {
+    if constexpr (ONE) __builtin_amdgcn_wave_barrier();
+    else __syncthreads();
+  };
   __shared__ double sbc[G][2 * NV];
   __shared__ double sF[G][NV];
   const int g = threadIdx.x / LPC, l = threadIdx.x % LPC;
@@ -1672,7 +1720,7 @@ __global__ __launch_bounds__(kAeFusedBlock) void k_ae_fused(const Dev *dptr, con
   long long cell = 0;
   if (valid) {
     setup_lane(d, c, l, L, Gm, cell);
-    load_forcing<ARITH>(d, p, c, rec, Gm, L, sbc[g]);
+    load_forcing<LPC, ARITH>(d, p, c, rec, Gm, L, sbc[g]);
   } else {
     L.l = l;
     L.K = 0;
@@ -1681,26 +1729,37 @@ __global__ __launch_bounds__(kAeFusedBlock) void k_ae_fused(const Dev *dptr, con
   __syncthreads();
   const bool act = valid && L.active;
   const bool own = valid && l < NV;
+  // boundary values: in registers for one wave, as in k_fixed
+  double rbc[2 * NV];
+  if constexpr (ONE) {
+#pragma unroll
+    for (int n = 0; n < 2 * NV; ++n) rbc[n] = sbc[g][n];
+  }
+  const double *bc = ONE ? rbc : sbc[g];
   double x[NV], r[NV];
 #pragma unroll
   for (int n = 0; n < NV; ++n) x[n] = act ? d.conc[n * d.ncell + cell] : 0.0;
   double sC = 0.0, sN = 0.0;
-  // sums touched only by accepted attempts live in LDS, leaving the
-  // registers to the right-hand side: the DIC and N2 sinks with their
-  // compensations, the lane's top-flux sum and compensation, and the
-  // column's diagnostics (updated by its top lane)
-  __shared__ double sacc[6][kAeFusedBlock];
-  __shared__ sedcol_coldiag sdg[G];
-  double(&acc)[6][kAeFusedBlock] = sacc;
+  // sums touched only by accepted attempts: in registers for one wave, else
+  // in LDS, leaving the registers to the right-hand side.  The DIC and N2
+  // sinks with their compensations, the lane's top-flux sum and compensation
+  __shared__ double sacc[6][ONE ? 1 : BLK];
+  double racc[6];
   const int t = threadIdx.x;
-  sedcol_coldiag &dg = sdg[g];
-  acc[0][t] = act ? d.cellacc[cell] : 0.0;
-  acc[1][t] = act ? d.cellacc[d.ncell + cell] : 0.0;
-  acc[2][t] = act ? d.cellacc[5 * d.ncell + cell] : 0.0;
-  acc[3][t] = act ? d.cellacc[6 * d.ncell + cell] : 0.0;
-  acc[4][t] = own ? d.colacc[(long long)l * d.ncol + c] : 0.0;
-  acc[5][t] = own ? d.colacc[(long long)(NV + l) * d.ncol + c] : 0.0;
-  if (valid && l == 0) dg = d.diag[c];
+  auto acc = [&](int i) -> double & {
+    if constexpr (ONE) return racc[i];
+    else return sacc[i][t];
+  };
+  acc(0) = act ? d.cellacc[cell] : 0.0;
+  acc(1) = act ? d.cellacc[d.ncell + cell] : 0.0;
+  acc(2) = act ? d.cellacc[5 * d.ncell + cell] : 0.0;
+  acc(3) = act ? d.cellacc[6 * d.ncell + cell] : 0.0;
+  acc(4) = own ? d.colacc[(long long)l * d.ncol + c] : 0.0;
+  acc(5) = own ? d.colacc[(long long)(NV + l) * d.ncol + c] : 0.0;
+  // the attempts of this launch enter the columns' diagnostics at its end
+  // (every column takes the same steps)
+  int accepted = 0;
+  double dt_last = 0.0;
   const double rcm = p.relative_change_min;
   double mind = INFINITY;
   int attempts = 0;
@@ -1716,16 +1775,15 @@ __global__ __launch_bounds__(kAeFusedBlock) void k_ae_fused(const Dev *dptr, con
       }
       if (need) {
         if (valid) {
-          column_rhs<LPC, ARITH>(p, L, sbc[g], x, sC, sN, [&](int n, double rr, double F) {
+          double Ft[NV];
+          column_rhs<LPC, ARITH>(p, L, bc, x, sC, sN, [&](int n, double rr, double F) {
             r[n] = rr;
-            if (l == 0) {
-              sF[g][n] = F;
-              d.flux[(long long)n * d.ncol + c] = F;
-            }
+            Ft[n] = F;
           }, &d.zw);
+          store_top(l == 0, Ft, sF[g]);
         }
         need = false;
-        __syncthreads();
+        sync();
       }
       bool v = false;
       if (act) {
@@ -1735,57 +1793,66 @@ __global__ __launch_bounds__(kAeFusedBlock) void k_ae_fused(const Dev *dptr, con
           v |= (c1 - (1.0 + rcm) * x[n]) < 0.0;
         }
       }
-      const int viol = __syncthreads_or(v);
+      const int viol = ONE ? __any(v) : __syncthreads_or(v);
       if (viol && dt_red > p.dt_min) {
         dt_red = dt_red * 0.25;  // the state is unchanged: the right-hand side is reused
       } else {
         if (dt_red < mind) mind = dt_red;
-        if (own) kadd(acc[4][t], acc[5][t], dt_red * sF[g][l]);
-        if (valid && l == 0) {
-          dg.accepted += 1;
-          dg.dt_last = dt_red;
-          if (dt_red < dg.dt_minacc) dg.dt_minacc = dt_red;
-        }
+        if (own) kadd(acc(4), acc(5), dt_red * sF[g][l]);
+        ++accepted;
+        dt_last = dt_red;
         if (act) {
 #pragma unroll
           for (int n = 0; n < NV; ++n) x[n] = x[n] + dt_red * r[n];
-          kadd(acc[0][t], acc[2][t], dt_red * sC);
-          kadd(acc[1][t], acc[3][t], dt_red * sN);
+          kadd(acc(0), acc(2), dt_red * sC);
+          kadd(acc(1), acc(3), dt_red * sN);
         }
         dt_int = dt_int + dt_red;
         need = true;
         // the lanes reading sF are done before the next evaluation writes it
-        __syncthreads();
+        sync();
       }
     }
     if (stop) break;
     if (p.clamp && act) {
-      bool nan = false;
+      bool odd = false;
 #pragma unroll
-      for (int n = 0; n < NV; ++n) {
-        nan |= x[n] != x[n];
-        if (x[n] < 0.0) {
-          if (elem(n) >= 0)
-            kadd(d.cellacc[(2 + elem(n)) * d.ncell + cell], d.cellacc[(7 + elem(n)) * d.ncell + cell], 0.0 - x[n]);
-          x[n] = 0.0;
+      for (int n = 0; n < NV; ++n) odd |= !(x[n] >= 0.0);
+      if (__any(odd)) {
+        bool nan = false;
+#pragma unroll
+        for (int n = 0; n < NV; ++n) {
+          nan |= x[n] != x[n];
+          if (x[n] < 0.0) {
+            if (elem(n) >= 0)
+              kadd(d.cellacc[(2 + elem(n)) * d.ncell + cell], d.cellacc[(7 + elem(n)) * d.ncell + cell], 0.0 - x[n]);
+            x[n] = 0.0;
+          }
         }
+        if (nan) atomicOr(errflag, 1);
       }
-      if (nan) atomicOr(errflag, 1);
     }
   }
   if (act) {
 #pragma unroll
     for (int n = 0; n < NV; ++n) d.conc[n * d.ncell + cell] = x[n];
-    d.cellacc[cell] = acc[0][t];
-    d.cellacc[d.ncell + cell] = acc[1][t];
-    d.cellacc[5 * d.ncell + cell] = acc[2][t];
-    d.cellacc[6 * d.ncell + cell] = acc[3][t];
+    d.cellacc[cell] = acc(0);
+    d.cellacc[d.ncell + cell] = acc(1);
+    d.cellacc[5 * d.ncell + cell] = acc(2);
+    d.cellacc[6 * d.ncell + cell] = acc(3);
   }
   if (own) {
-    d.colacc[(long long)l * d.ncol + c] = acc[4][t];
-    d.colacc[(long long)(NV + l) * d.ncol + c] = acc[5][t];
+    d.colacc[(long long)l * d.ncol + c] = acc(4);
+    d.colacc[(long long)(NV + l) * d.ncol + c] = acc(5);
+    if (attempts > 0) d.flux[(long long)l * d.ncol + c] = sF[g][l];
   }
-  if (valid && l == 0) d.diag[c] = dg;
+  if (valid && l == 0 && accepted > 0) {
+    sedcol_coldiag dg = d.diag[c];
+    dg.accepted += accepted;
+    dg.dt_last = dt_last;
+    if (mind < dg.dt_minacc) dg.dt_minacc = mind;
+    d.diag[c] = dg;
+  }
   if (threadIdx.x == 0) *min_dt = mind;
 }
 
@@ -1876,7 +1943,7 @@ __global__ __launch_bounds__(BLOCK) void k_residual(Dev d, const int *list, int 
   long long cell = 0;
   if (valid) {
     setup_lane(d, c, l, L, Gm, cell);
-    load_forcing<ARITH>(d, p, c, rec, Gm, L, sbc[g]);
+    load_forcing<LPC, ARITH>(d, p, c, rec, Gm, L, sbc[g]);
   }
   __syncthreads();
   if (!valid) return;
@@ -2338,9 +2405,20 @@ void launch_ae_commit(int lpc, hipStream_t st, const Dev &d, const int *list, in
 void launch_ae_fused(int lpc, hipStream_t st, const Dev *d_dev, const int *list, int n, const sedcol_params &p,
                      const sedcol_params *d_params, int rec, double dt, int nsteps, int *errflag, double *min_dt)
 {
-  SC_DISPATCH_ARITH(p, SC_DISPATCH_LPC(lpc, hipLaunchKernelGGL((k_ae_fused<LPC, AR>), dim3(1), dim3(kAeFusedBlock),
-                                                                0, st, d_dev, list, n, d_params, rec, dt, nsteps,
-                                                                errflag, min_dt)));
+  // the smallest block that holds the columns: one wave, one wave per SIMD
+  // (all registers), two
+#define SC_AE_FUSED(BLK)                                                                                           \
+  SC_DISPATCH_ARITH(p, SC_DISPATCH_LPC(lpc, hipLaunchKernelGGL((k_ae_fused<LPC, AR, BLK>), dim3(1), dim3(BLK), 0, st, \
+                                                                d_dev, list, n, d_params, rec, dt, nsteps, errflag, \
+                                                                min_dt)))
+  if (n * lpc <= 64) {
+    SC_AE_FUSED(64);
+  } else if (n * lpc <= 256) {
+    SC_AE_FUSED(256);
+  } else {
+    SC_AE_FUSED(kAeFusedBlock);
+  }
+#undef SC_AE_FUSED
 }
 
 void launch_clamp(int lpc, hipStream_t st, const Dev &d, const int *list, int n, int *errflag)
