@@ -381,9 +381,15 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
 
 // minimum waves per SIMD requested from the register allocator: 2 fits the
 // adaptive step in 256 VGPRs without scratch (1 lets it take 256 + AGPRs,
-// 3 spills about 340 bytes per lane)
+// 3 spills about 340 bytes per lane).  With geometric weights the step does not
+// fit (130 to 190 bytes of scratch per lane) and one wave is faster at every
+// size, reference form, 1 h: 1201 columns of 30 to 60 layers 157 -> 104 ms,
+// 9000 columns of 10 to 60 layers 300 -> 235 ms.
 #ifndef SEDCOL_EMP_MIN_WAVES
 #define SEDCOL_EMP_MIN_WAVES 2
+#endif
+#ifndef SEDCOL_GEO_MIN_WAVES
+#define SEDCOL_GEO_MIN_WAVES 1
 #endif
 
 // Work-queue kernel: a grid sized to the resident capacity, each lane group
@@ -403,7 +409,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
 // attempts are split over launches, so windowed and single-launch runs give
 // identical results.
 template <int LPC, int ARITH, int BLK, int PW>
-__global__ __launch_bounds__(BLK, SEDCOL_EMP_MIN_WAVES) void k_emp_adaptive(
+__global__ __launch_bounds__(BLK, PW == 1 ? SEDCOL_GEO_MIN_WAVES : SEDCOL_EMP_MIN_WAVES) void k_emp_adaptive(
     const Dev *dptr, const int *list, int nlist, const sedcol_params *__restrict__ pptr,
     const EmpCtl *__restrict__ cptr, int *next, int *pending, int *work, int *errflag)
 {
