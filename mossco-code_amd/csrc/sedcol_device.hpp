@@ -4,9 +4,9 @@
 // 64, a power of two >= K), lane l holding layer l with all NV state
 // variables in VGPRs.  Vertical neighbours move between lanes with DPP
 // wave shifts; column sums, products and maxima use a butterfly (DPP quad
-// permutes and row mirrors, a 32-lane swizzle, and a bpermute for the
-// 64-lane level), i.e. a balanced pairwise tree whose grouping does not
-// depend on LPC (padding lanes hold the identity).
+// permutes and row mirrors, and the row swaps for the levels of 16 and 32
+// lanes), i.e. a balanced pairwise tree whose grouping does not depend on
+// LPC (padding lanes hold the identity).
 //
 // Floating point: built with -ffp-contract=off; fused multiply-adds are
 // explicit fma() calls.  Two arithmetic forms exist (template ARITH):
@@ -41,6 +41,13 @@ __host__ __device__ constexpr int elem(int n)
   return (n == 0 || n == 1) ? 0 : (n == 2 || n == 3 || n == 6 || n == 7) ? 1 : (n == 4 || n == 9 || n == 10) ? 2 : -1;
 }
 
+// larger of two values, the other one if one is a NaN, in one instruction
+__device__ __forceinline__ double vmax(double a, double b)
+{
+  double r;
+  __asm__("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
 __device__ __forceinline__ double nn(double c) { return c < 0.0 ? 0.0 : c; }
 
 // Neumaier-compensated running sum: s + c carries the total of every x added.
@@ -456,20 +463,12 @@ __device__ __forceinline__ double dpp_d(double v)
   return __hiloint2double(hi, lo);
 }
 
-template <int PATTERN>
-__device__ __forceinline__ double swz_d(double v)
-{
-  const int lo = __builtin_amdgcn_ds_swizzle(__double2loint(v), PATTERN);
-  const int hi = __builtin_amdgcn_ds_swizzle(__double2hiint(v), PATTERN);
-  return __hiloint2double(hi, lo);
-}
-
 // value held by the previous lane (wave_shr:1); lane 0 of a group never uses it
 __device__ __forceinline__ double lg_up(double v) { return dpp_d<0x138>(v); }
 // value held by the next lane (wave_shl:1); the last layer never uses it
 __device__ __forceinline__ double lg_dn(double v) { return dpp_d<0x130>(v); }
 
-// Partner value at butterfly level S (S = 1, 2, 4, ...).  Levels 4 and 8 use
+// Partner value at butterfly level S (S = 1, 2, 4, 8).  Levels 4 and 8 use
 // row mirrors, which pair the same sub-groups as lane^S once every sub-group
 // of size S holds one value, which the butterfly guarantees because it runs
 // the levels in increasing order.
@@ -479,23 +478,50 @@ __device__ __forceinline__ double bfly(double v)
   if constexpr (S == 1) return dpp_d<0xB1>(v);        // quad_perm [1,0,3,2]
   else if constexpr (S == 2) return dpp_d<0x4E>(v);   // quad_perm [2,3,0,1]
   else if constexpr (S == 4) return dpp_d<0x141>(v);  // row_half_mirror
-  else if constexpr (S == 8) return dpp_d<0x140>(v);  // row_mirror
-  else if constexpr (S == 16) return swz_d<0x401F>(v); // swizzle xor 16 within 32 lanes
-  else return __shfl_xor(v, 32, 64);
+  else return dpp_d<0x140>(v);                        // S == 8: row_mirror
+}
+
+// Levels 16 and 32: a receives the value of the pair's lower row (or half wave),
+// b that of its upper one, on both, by the row swaps: 34 cycles with the sum
+// against 65 through the LDS crossbar (swizzle) and 77 by a bpermute.  Sums and
+// products are the same in either order.
+template <int S>
+__device__ __forceinline__ void pair_d(double v, double &a, double &b)
+{
+  const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+  if constexpr (S == 16) {
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    a = __hiloint2double((int)h[0], (int)l[0]);
+    b = __hiloint2double((int)h[1], (int)l[1]);
+  } else {
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    a = __hiloint2double((int)h[0], (int)l[0]);
+    b = __hiloint2double((int)h[1], (int)l[1]);
+  }
 }
 
 template <int LPC, int S = 1>
 __device__ __forceinline__ double lg_sum(double v)
 {
   if constexpr (S >= LPC) return v;
-  else return lg_sum<LPC, 2 * S>(v + bfly<S>(v));
+  else if constexpr (S >= 16) {
+    double a, b;
+    pair_d<S>(v, a, b);
+    return lg_sum<LPC, 2 * S>(a + b);
+  } else return lg_sum<LPC, 2 * S>(v + bfly<S>(v));
 }
 // maximum over the group; a NaN in any lane gives NaN
 template <int LPC, int S = 1>
 __device__ __forceinline__ double lg_max(double v)
 {
   if constexpr (S >= LPC) return v;
-  else {
+  else if constexpr (S >= 16) {
+    double a, b;
+    pair_d<S>(v, a, b);
+    return lg_max<LPC, 2 * S>((b > a || b != b) ? b : a);
+  } else {
     const double o = bfly<S>(v);
     return lg_max<LPC, 2 * S>((o > v || o != o) ? o : v);
   }
@@ -505,10 +531,18 @@ template <int LPC, int S = 1>
 __device__ __forceinline__ void lg_pd(double &P, double &D)
 {
   if constexpr (S < LPC) {
-    const double Po = bfly<S>(P);
-    const double Do = bfly<S>(D);
-    D = D * Po + P * Do;
-    P = P * Po;
+    if constexpr (S >= 16) {
+      double P0, P1, D0, D1;
+      pair_d<S>(P, P0, P1);
+      pair_d<S>(D, D0, D1);
+      D = D0 * P1 + P0 * D1;
+      P = P0 * P1;
+    } else {
+      const double Po = bfly<S>(P);
+      const double Do = bfly<S>(D);
+      D = D * Po + P * Do;
+      P = P * Po;
+    }
     lg_pd<LPC, 2 * S>(P, D);
   }
 }
@@ -734,7 +768,11 @@ template <int LPC, int S = 1>
 __device__ __forceinline__ double lg_prod(double v)
 {
   if constexpr (S >= LPC) return v;
-  else return lg_prod<LPC, 2 * S>(v * bfly<S>(v));
+  else if constexpr (S >= 16) {
+    double a, b;
+    pair_d<S>(v, a, b);
+    return lg_prod<LPC, 2 * S>(a * b);
+  } else return lg_prod<LPC, 2 * S>(v * bfly<S>(v));
 }
 
 // Patankar factor of one column (Bruggeman et al. 2007), by Newton from

@@ -45,10 +45,20 @@ __device__ __forceinline__ void setup_lane(const Dev &d, int c, int l, Lane &L, 
   G.B = d.biot[c];
 }
 
+// whether b holds on any active lane of the group: the group's bits of the
+// wave's ballot, instead of a reduction over the lanes
 template <int LPC>
 __device__ __forceinline__ bool group_any(bool b)
 {
-  return lg_max<LPC>(b ? 1.0 : 0.0) > 0.0;
+  const unsigned long long m = __ballot(b);
+  if constexpr (LPC == 64) {
+    return m != 0;
+  } else {
+    const unsigned lane = __lane_id();
+    const unsigned half = (lane & 32u) ? (unsigned)(m >> 32) : (unsigned)m;
+    if constexpr (LPC == 32) return half != 0;
+    else return ((lane & 16u) ? half >> 16 : half & 0xffffu) != 0;
+  }
 }
 
 // load forcing record r of column c: bottom-water concentrations and top
@@ -549,10 +559,10 @@ __global__ __launch_bounds__(BLK, PW == 1 ? SEDCOL_GEO_MIN_WAVES : SEDCOL_EMP_MI
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
         const double y = x[n] + (h * p2) * f0[n];
-        const double yp = y < 0.0 ? 0.0 : y;
-        const double sc = p.emp_atol + p.emp_rtol * (yp > x[n] ? yp : x[n]);
+        const double yp = vmax(y, 0.0);
+        const double sc = p.emp_atol + p.emp_rtol * vmax(yp, x[n]);
         const double dv = fabs(yp - c1[n]);
-        bad |= (dv != dv) || (sc != sc);
+        bad |= (y != y) || (sc != sc);
         if (dv * bd > bn * sc) {
           bn = dv;
           bd = sc;
