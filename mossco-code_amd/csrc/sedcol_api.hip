@@ -112,6 +112,7 @@ struct sedcol_handle {
   int lpc[3] = {16, 32, 64};  // lanes per column of each bin in the adaptive kernel
   int blk[3] = {256, 256, 256};  // workgroup size of each bin in the adaptive kernel
   int lpl[3] = {1, 1, 1};        // layers per lane of each bin in the adaptive kernel
+  bool tuned = false;            // a shape was installed (sedcol_set_tuning, sedcol_autotune)
   hipStream_t aux[2] = {nullptr, nullptr};  // for concurrent bins
   hipEvent_t evfork = nullptr, evjoin[2] = {nullptr, nullptr};
   hipGraph_t graph = nullptr;
@@ -325,7 +326,11 @@ int check_tuning(const sedcol_handle *h, const sedcol_tuning *t)
   return SEDCOL_OK;
 }
 
-// kernel shape bin b runs with under the current parameters: an installed
+// kernel shape bin b runs with under the current parameters.  Unless a shape
+// was installed, the linearly implicit stepper runs in blocks of one wave: a
+// block holds its place until its slowest column is done, and at one wave per
+// SIMD a place is a quarter of a CU (a day of spin-up of 3000 columns 189 ->
+// 175 ms; adaptive EMP does not gain).  An installed
 // two-layers-per-lane shape falls back to one layer per lane (with enough
 // lanes for the bin) where that kernel does not cover the parameters
 // (linearly implicit stepper, geometric-mean weights, bioturbation profile
@@ -335,6 +340,7 @@ void effective_shape(const sedcol_handle *h, int b, int *lpc, int *blk, int *lpl
   *lpc = h->lpc[b];
   *blk = h->blk[b];
   *lpl = h->lpl[b];
+  if (!h->tuned && h->p.adaptive_method == SEDCOL_ROS2_ADAPTIVE) *blk = std::max(64, *lpc);
   if (*lpl == 2 && !sc::emp2_supported(h->p)) {
     *lpl = 1;
     *lpc = std::max(*lpc, bin_min_lpc(h, b, 1));
@@ -352,18 +358,27 @@ void drop_graph(sedcol_handle *h)
 
 // One adaptive launch per non-empty bin (only bin `only` when only >= 0).
 // Work-queue counters and the pending count must be zero beforehand.
-// Persistent launches always run as branches forked from the handle's stream,
-// the bin of the longest columns first: each bin ends on a few slow columns
-// that leave most of the device idle, and the next bin's blocks start there.
-// In order, the bins' slowest columns added up (1201 columns of 30 to 60
-// layers, geometric weights, 3 h: 768 ms in order, 405 ms as branches; 9001
-// columns of 10 to 60 layers, 6 h: 650 and 465 ms).  Windowed launches fork as
-// the schedule says.
+// Persistent launches always run as branches forked from the handle's stream:
+// each bin ends on a few slow columns that leave most of the device idle, and
+// the next bin's blocks start there.  The bin with the fewest blocks goes
+// first: its columns all start at once, and the bin that has more columns than
+// places, which works off a queue, fills what they leave.  In order, the bins'
+// slowest columns added up (1201 columns of 30 to 60 layers, geometric weights,
+// 3 h: 768 ms in order, 405 ms as branches; 9001 columns of 10 to 60 layers,
+// 6 h: 650 ms in order, 426 ms with the most blocks first, 266 ms with the
+// fewest first).  Windowed launches fork as the schedule says.
 int launch_bins(sedcol_handle *h, int only, int *launches)
 {
   int list[3], nb = 0;
-  for (int b = 2; b >= 0; --b)
-    if (!h->bins[b].empty() && (only < 0 || only == b)) list[nb++] = b;
+  long long blocks[3] = {0, 0, 0};
+  for (int b = 0; b < 3; ++b)
+    if (!h->bins[b].empty() && (only < 0 || only == b)) {
+      int lpc, blk, lpl;
+      effective_shape(h, b, &lpc, &blk, &lpl);
+      blocks[b] = ((long long)h->bins[b].size() * lpc + blk - 1) / blk * blk;  // in threads: blocks differ in size
+      list[nb++] = b;
+    }
+  std::stable_sort(list, list + nb, [&](int p, int q) { return blocks[p] < blocks[q]; });
   const bool fork = (h->sched.window <= 0 || h->sched.concurrent_bins) && nb > 1;
   if (fork) HIPOK(hipEventRecord(h->evfork, h->stream));
   for (int i = 0; i < nb; ++i) {
@@ -1251,6 +1266,7 @@ int sedcol_set_tuning(sedcol_handle *h, const sedcol_tuning *t)
     h->blk[b] = t->lanes_per_column[b] * t->columns_per_group[b];
     h->lpl[b] = t->layers_per_lane[b] == 2 ? 2 : 1;
   }
+  h->tuned = true;
   drop_graph(h);
   return SEDCOL_OK;
 }
@@ -1313,6 +1329,8 @@ int sedcol_autotune(sedcol_handle *h, double t_start, double t_span, int32_t rep
   std::memcpy(saved_blk, h->blk, sizeof saved_blk);
   std::memcpy(saved_lpl, h->lpl, sizeof saved_lpl);
   h->sched = sedcol_schedule{0, 0, 1, 0};  // one launch per trial
+  const bool saved_tuned = h->tuned;
+  h->tuned = true;
   int best_l[3], best_w[3], best_p[3];
   std::memcpy(best_l, h->lpc, sizeof best_l);
   std::memcpy(best_w, h->blk, sizeof best_w);
@@ -1367,6 +1385,7 @@ int sedcol_autotune(sedcol_handle *h, double t_start, double t_span, int32_t rep
     std::memcpy(h->lpc, saved_lpc, sizeof saved_lpc);
     std::memcpy(h->blk, saved_blk, sizeof saved_blk);
     std::memcpy(h->lpl, saved_lpl, sizeof saved_lpl);
+    h->tuned = saved_tuned;
     return rc ? rc : rc2;
   }
   std::memcpy(h->lpc, best_l, sizeof best_l);
