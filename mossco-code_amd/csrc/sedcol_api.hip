@@ -5,11 +5,13 @@
 // validates its arguments, returns a sedcol_status code and records a message
 // for sedcol_last_error(); nothing aborts the process.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "sedcol_kernels.hpp"
@@ -38,6 +40,11 @@ constexpr int kLpc[3] = {16, 32, 64};
 // steps per launch of the one-workgroup adaptive Euler (at most
 // kAeFusedMaxAttempts attempts per launch, i.e. about 1000 per step)
 constexpr int kAeFusedSteps = 4096;
+
+// largest pinned staging of one sedcol_step (state, top fluxes, flags): the
+// device reads it over the link, which up to this size is quicker than the
+// copies' own waits
+constexpr size_t kStageBytes = size_t(512) << 10;
 
 // Workspace of sedcol_rhs_noalloc: staging of its input state, its
 // right-hand side and top fluxes, and (Fortran layout) of the caller's
@@ -97,11 +104,15 @@ struct sedcol_handle {
   sedcol_coldiag *d_diag = nullptr;
   double *d_scr = nullptr;  // NV*ncell scratch (rhs in/out, adaptive Euler rates)
   double *d_scr2 = nullptr; // NV*ncell scratch
+  double *d_scr3 = nullptr; // NV*ncell: packed state of sedcol_rhs, Fortran layout
   double *d_small = nullptr;  // NV*ncol + ncol scratch
   double *d_warm = nullptr;   // scale, offset (NV*kWarmMaxNodes each) and eps (NV) of a warm start
   double *d_noalloc = nullptr;  // this device's sedcol_rhs_noalloc workspace (not owned)
-  int *d_flag = nullptr;     // [0] error flags, [1..3] work-queue counters per bin, [4] windowed columns pending
+  int *d_flag = nullptr;     // [0] error flags, [1..3] work-queue counters per bin, [4] windowed columns pending,
+                             // [5], [6] votes of adaptive Euler attempts
   int *h_flag = nullptr;     // pinned host copy of d_flag[0..4]
+  bool piped = false;        // counts as a user of the pinned blocks (copy_large)
+  double *h_stage = nullptr; // pinned: state, top fluxes and flags of sedcol_step, small domains only
   int *d_work = nullptr;     // ncol: attempts of each column in the last adaptive launch
   int *d_wrec = nullptr;     // ncol: adaptive position between windows (record, time left, attempts)
   double *d_wrem = nullptr;
@@ -188,33 +199,6 @@ void pack_cells(const sedcol_handle *h, const double *src, std::vector<double> &
   }
   for (int c = 0; c < h->ncol; ++c)
     for (int k = 0; k < h->kmax; ++k) dst[(long long)c * h->kmax + k] = src[fidx(h, c, k)];
-}
-
-void pack_state(const sedcol_handle *h, const double *src, std::vector<double> &dst)
-{
-  dst.resize((size_t)NV * h->ncell);
-  if (h->layout == SEDCOL_LAYOUT_PACKED) {
-    std::memcpy(dst.data(), src, sizeof(double) * NV * h->ncell);
-    return;
-  }
-  const long long plane = (long long)h->ncol * h->kmax;
-  for (int n = 0; n < NV; ++n)
-    for (int k = 0; k < h->kmax; ++k)
-      for (int c = 0; c < h->ncol; ++c)
-        dst[n * h->ncell + (long long)c * h->kmax + k] = src[n * plane + fidx(h, c, k)];
-}
-
-void unpack_state(const sedcol_handle *h, const std::vector<double> &src, double *dst)
-{
-  if (h->layout == SEDCOL_LAYOUT_PACKED) {
-    std::memcpy(dst, src.data(), sizeof(double) * NV * h->ncell);
-    return;
-  }
-  const long long plane = (long long)h->ncol * h->kmax;
-  for (int n = 0; n < NV; ++n)
-    for (int k = 0; k < h->kmax; ++k)
-      for (int c = 0; c < h->ncol; ++c)
-        dst[n * plane + fidx(h, c, k)] = src[n * h->ncell + (long long)c * h->kmax + k];
 }
 
 // Makes the handle's device current for the duration of one entry point and
@@ -501,6 +485,133 @@ int ensure_scratch(sedcol_handle *h)
   return SEDCOL_OK;
 }
 
+// The caller's state arrays go to and from the device as they are, without a
+// copy in host memory: packed ones directly, Fortran ones through d_scr and
+// k_layout.  (A packed copy first, or the transposition on the host, took 59
+// of the 62 ms of setting and 63 of the 76 ms of reading 238 MB.)
+//
+// Large copies go through pinned blocks that several threads fill or empty: the
+// link takes pinned memory at 55 GB/s, where one thread of the runtime moves
+// pageable memory at 28 GB/s in and 17 GB/s out, or 4 GB/s into an array whose
+// pages are still to be made.  The blocks belong to the process and are shared
+// by the handles of large domains, freed with the last of them; one copy at a
+// time uses them, another one goes the runtime's way.
+constexpr size_t kBlock = size_t(2) << 20, kBlocks = 8, kPipeMin = size_t(8) << 20;
+struct Pipe {
+  std::mutex users_mu, mu;
+  int users = 0;
+  char *mem = nullptr;
+} g_pipe;
+
+void pipe_acquire()
+{
+  std::lock_guard<std::mutex> lk(g_pipe.users_mu);
+  if (g_pipe.users++ > 0) return;
+  std::lock_guard<std::mutex> use(g_pipe.mu);
+  if (hipHostMalloc((void **)&g_pipe.mem, kBlock * kBlocks, hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();
+    g_pipe.mem = nullptr;  // copies go the runtime's way
+  }
+}
+
+void pipe_release()
+{
+  std::lock_guard<std::mutex> lk(g_pipe.users_mu);
+  if (--g_pipe.users > 0) return;
+  std::lock_guard<std::mutex> use(g_pipe.mu);
+  if (g_pipe.mem) (void)hipHostFree(g_pipe.mem);
+  g_pipe.mem = nullptr;
+}
+
+// bytes between the caller's memory and the device, in stream order; on return
+// the caller's memory has been read or written unless the copy was small (then
+// it is queued).  to_device: from `in` to `dev`, else from `dev` to `out`.
+int copy_large(sedcol_handle *h, void *dev, const void *in, void *out, size_t bytes, bool to_device)
+{
+  std::unique_lock<std::mutex> use(g_pipe.mu, std::defer_lock);
+  if (bytes < kPipeMin || !h->piped || !use.try_lock() || !g_pipe.mem) {
+    if (to_device) HIPOK(hipMemcpyAsync(dev, in, bytes, hipMemcpyHostToDevice, h->stream));
+    else HIPOK(hipMemcpyAsync(out, dev, bytes, hipMemcpyDeviceToHost, h->stream));
+    return SEDCOL_OK;
+  }
+  const size_t n = (bytes + kBlock - 1) / kBlock;
+  std::atomic<size_t> next{0};
+  std::atomic<int> err{0};
+  // one block, one event per worker: it takes the next part of the array,
+  // fills its block and queues the copy, or queues it, waits and empties it
+  auto work = [&](size_t w) {
+    char *const blk = g_pipe.mem + w * kBlock;
+    hipError_t e = hipSetDevice(h->device);
+    hipEvent_t ev = nullptr;
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    bool pending = false;
+    while (e == hipSuccess && err.load(std::memory_order_relaxed) == 0) {
+      const size_t i = next.fetch_add(1, std::memory_order_relaxed);
+      if (i >= n) break;
+      const size_t o = i * kBlock, len = std::min(kBlock, bytes - o);
+      if (to_device) {
+        if (pending) e = hipEventSynchronize(ev);  // the block's last copy has been read
+        if (e != hipSuccess) break;
+        std::memcpy(blk, static_cast<const char *>(in) + o, len);
+        e = hipMemcpyAsync(static_cast<char *>(dev) + o, blk, len, hipMemcpyHostToDevice, h->stream);
+        if (e == hipSuccess) e = hipEventRecord(ev, h->stream);
+        pending = true;
+      } else {
+        e = hipMemcpyAsync(blk, static_cast<char *>(dev) + o, len, hipMemcpyDeviceToHost, h->stream);
+        if (e == hipSuccess) e = hipEventRecord(ev, h->stream);
+        if (e == hipSuccess) e = hipEventSynchronize(ev);
+        if (e == hipSuccess) std::memcpy(static_cast<char *>(out) + o, blk, len);
+      }
+    }
+    // the block is free for the next user of the pipe once its copy is done
+    if (pending) {
+      const hipError_t e2 = hipEventSynchronize(ev);
+      if (e == hipSuccess) e = e2;
+    }
+    if (ev) (void)hipEventDestroy(ev);
+    if (e != hipSuccess) err.store((int)e, std::memory_order_relaxed);
+  };
+  std::vector<std::thread> team;
+  try {
+    team.reserve(kBlocks);
+    for (size_t w = 1; w < std::min(n, kBlocks); ++w) team.emplace_back(work, w);
+  } catch (...) {  // fewer threads: the others take their parts
+  }
+  work(0);
+  for (auto &t : team) t.join();
+  if (err.load() != 0) {
+    (void)hipStreamSynchronize(h->stream);  // no copy into or out of a block is left
+    return fail(SEDCOL_EHIP, std::string("copy of the state: ") + hipGetErrorString((hipError_t)err.load()));
+  }
+  return SEDCOL_OK;
+}
+
+// caller's state (NV planes) -> packed device array dst (not d_scr)
+int put_state(sedcol_handle *h, const double *conc, double *dst)
+{
+  const size_t bytes = sizeof(double) * NV * (size_t)h->ncell;
+  if (h->layout == SEDCOL_LAYOUT_PACKED) return copy_large(h, dst, conc, nullptr, bytes, true);
+  if (!h->d_scr) HIPOK(hipMalloc(&h->d_scr, bytes));
+  const int rc = copy_large(h, h->d_scr, conc, nullptr, bytes, true);
+  if (rc) return rc;
+  sc::launch_layout(h->stream, h->d_scr, dst, h->ncol, h->kmax, NV, true);
+  HIPOK(hipGetLastError());
+  return SEDCOL_OK;
+}
+
+// packed device array src -> caller's state (queued; src not d_scr)
+int take_state(sedcol_handle *h, double *src, double *conc)
+{
+  const size_t bytes = sizeof(double) * NV * (size_t)h->ncell;
+  if (h->layout != SEDCOL_LAYOUT_PACKED) {
+    if (!h->d_scr) HIPOK(hipMalloc(&h->d_scr, bytes));
+    sc::launch_layout(h->stream, src, h->d_scr, h->ncol, h->kmax, NV, false);
+    HIPOK(hipGetLastError());
+    src = h->d_scr;
+  }
+  return copy_large(h, src, nullptr, conc, bytes, false);
+}
+
 // upload the current bins as the work lists (after a change of the active set)
 int upload_bins(sedcol_handle *h)
 {
@@ -633,6 +744,13 @@ int sedcol_create(const sedcol_desc *desc, sedcol_handle **out)
   HIPOK_C(hipMalloc(&h->d_flag, sizeof(int) * 8));  // error flag, one work-queue counter per bin, pending
   HIPOK_C(hipMemset(h->d_flag, 0, sizeof(int) * 8));
   HIPOK_C(hipHostMalloc((void **)&h->h_flag, sizeof(int) * 8, hipHostMallocDefault));
+  if (sizeof(double) * NV * (size_t)h->ncell >= kPipeMin) {
+    pipe_acquire();
+    h->piped = true;
+  }
+  const size_t stage = sizeof(double) * (NV * ((size_t)h->ncell + (size_t)h->ncol) + 2) + sizeof(sedcol_params) +
+                       sizeof(Dev);  // step_small's layout
+  if (stage <= kStageBytes) HIPOK_C(hipHostMalloc((void **)&h->h_stage, stage, hipHostMallocDefault));
   HIPOK_C(hipMalloc(&h->d_work, sizeof(int) * h->ncol));
   HIPOK_C(hipMalloc(&h->d_wrec, sizeof(int) * h->ncol));
   HIPOK_C(hipMalloc(&h->d_wrem, sizeof(double) * h->ncol));
@@ -664,12 +782,14 @@ int sedcol_destroy(sedcol_handle *h)
   if (h->stream) (void)hipStreamSynchronize(h->stream);
   void *ptrs[] = {h->d_off, h->d_list[0], h->d_list[1], h->d_list[2], h->d_dz, h->d_dzc, h->d_phi, h->d_phiI,
                   h->d_bfac, h->d_biot, h->d_temp, h->d_cbw, h->d_fup, h->d_conc, h->d_cellacc, h->d_colacc,
-                  h->d_flux, h->d_diag, h->d_scr, h->d_scr2, h->d_small, h->d_flag, h->d_work,
+                  h->d_flux, h->d_diag, h->d_scr, h->d_scr2, h->d_scr3, h->d_small, h->d_flag, h->d_work,
                   h->d_devview, h->d_params, h->d_wrec, h->d_wrem, h->d_watt, h->d_ctl, h->d_fcap,
                   h->d_ze1, h->d_ze2, h->d_zcum, h->d_warm};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   if (h->h_flag) (void)hipHostFree(h->h_flag);
+  if (h->h_stage) (void)hipHostFree(h->h_stage);
+  if (h->piped) pipe_release();
   drop_graph(h);
   for (int a = 0; a < 2; ++a) {
     if (h->aux[a]) (void)hipStreamDestroy(h->aux[a]);
@@ -916,9 +1036,8 @@ int sedcol_set_state(sedcol_handle *h, const double *conc)
 {
   if (!h || !conc) return fail(SEDCOL_EINVAL, "null argument");
   const DeviceScope dscope(h->device);
-  std::vector<double> buf;
-  pack_state(h, conc, buf);
-  HIPOK(hipMemcpyAsync(h->d_conc, buf.data(), sizeof(double) * buf.size(), hipMemcpyHostToDevice, h->stream));
+  int rc = put_state(h, conc, h->d_conc);
+  if (rc) return rc;
   HIPOK(hipStreamSynchronize(h->stream));
   return SEDCOL_OK;
 }
@@ -962,13 +1081,11 @@ int sedcol_get_state(sedcol_handle *h, double *conc)
 {
   if (!h || !conc) return fail(SEDCOL_EINVAL, "null argument");
   const DeviceScope dscope(h->device);
-  std::vector<double> buf((size_t)NV * h->ncell);
-  HIPOK(hipMemcpyAsync(buf.data(), h->d_conc, sizeof(double) * buf.size(), hipMemcpyDeviceToHost, h->stream));
+  int rc = take_state(h, h->d_conc, conc);
+  if (rc) return rc;
   HIPOK(hipStreamSynchronize(h->stream));
-  unpack_state(h, buf, conc);
   return SEDCOL_OK;
 }
-
 
 int sedcol_rhs(sedcol_handle *h, const double *conc, double *rhs, double *flux_top_out)
 {
@@ -978,23 +1095,23 @@ int sedcol_rhs(sedcol_handle *h, const double *conc, double *rhs, double *flux_t
   if (!conc || !rhs) return fail(SEDCOL_EINVAL, "null argument");
   if (h->nrec > 1) return fail(SEDCOL_EINVAL, "a forcing series is active; get_rhs uses one record (sedcol_set_forcing)");
   if ((rc = ensure_scratch(h))) return rc;
-  std::vector<double> buf;
-  pack_state(h, conc, buf);
-  HIPOK(hipMemcpyAsync(h->d_scr, buf.data(), sizeof(double) * buf.size(), hipMemcpyHostToDevice, h->stream));
-  HIPOK(hipMemsetAsync(h->d_scr2, 0, sizeof(double) * buf.size(), h->stream));
-  HIPOK(hipMemsetAsync(h->d_small, 0, sizeof(double) * NV * h->ncol, h->stream));
+  // packed: state in d_scr, rhs in d_scr2.  Fortran: d_scr takes the caller's
+  // arrays on both ways, so the packed state is a third array
+  const bool fortran = h->layout == SEDCOL_LAYOUT_FORTRAN;
+  if (fortran && !h->d_scr3) HIPOK(hipMalloc(&h->d_scr3, sizeof(double) * NV * (size_t)h->ncell));
+  double *in = fortran ? h->d_scr3 : h->d_scr;
+  const size_t fl = sizeof(double) * NV * (size_t)h->ncol;
+  if ((rc = put_state(h, conc, in))) return rc;
+  HIPOK(hipMemsetAsync(h->d_scr2, 0, sizeof(double) * NV * (size_t)h->ncell, h->stream));
+  HIPOK(hipMemsetAsync(h->d_small, 0, fl, h->stream));
   const Dev d = h->dev();
   for (int b = 0; b < 3; ++b)
     if (!h->bins[b].empty())
-      sc::launch_rhs(kLpc[b], h->stream, d, h->d_list[b], (int)h->bins[b].size(), h->p, 0, h->d_scr, h->d_scr2,
-                     h->d_small);
+      sc::launch_rhs(kLpc[b], h->stream, d, h->d_list[b], (int)h->bins[b].size(), h->p, 0, in, h->d_scr2, h->d_small);
   HIPOK(hipGetLastError());
-  HIPOK(hipMemcpyAsync(buf.data(), h->d_scr2, sizeof(double) * buf.size(), hipMemcpyDeviceToHost, h->stream));
-  std::vector<double> fl((size_t)NV * h->ncol);
-  HIPOK(hipMemcpyAsync(fl.data(), h->d_small, sizeof(double) * fl.size(), hipMemcpyDeviceToHost, h->stream));
+  if ((rc = take_state(h, h->d_scr2, rhs))) return rc;
+  if (flux_top_out) HIPOK(hipMemcpyAsync(flux_top_out, h->d_small, fl, hipMemcpyDeviceToHost, h->stream));
   HIPOK(hipStreamSynchronize(h->stream));
-  unpack_state(h, buf, rhs);
-  if (flux_top_out) std::memcpy(flux_top_out, fl.data(), sizeof(double) * fl.size());
   return SEDCOL_OK;
 }
 
@@ -1016,7 +1133,7 @@ int sedcol_rhs_noalloc(sedcol_handle *h, const double *conc, double *rhs, double
   std::lock_guard<std::mutex> lk(g_noalloc_mu[h->device]);
   double *in = h->d_noalloc, *out = in + cells, *flux = out + cells, *raw = flux + fl;
   HIPOK(hipMemcpyAsync(fortran ? raw : in, conc, sizeof(double) * cells, hipMemcpyHostToDevice, h->stream));
-  if (fortran) sc::launch_layout(h->stream, raw, in, h->ncol, h->kmax, true);
+  if (fortran) sc::launch_layout(h->stream, raw, in, h->ncol, h->kmax, NV, true);
   // land columns keep rhs = 0 and no top flux; fill kernels, not memsets
   sc::launch_fill_dbl(h->stream, out, (long long)cells, 0.0);
   sc::launch_fill_dbl(h->stream, flux, (long long)fl, 0.0);
@@ -1024,7 +1141,7 @@ int sedcol_rhs_noalloc(sedcol_handle *h, const double *conc, double *rhs, double
   for (int b = 0; b < 3; ++b)
     if (!h->bins[b].empty())
       sc::launch_rhs(kLpc[b], h->stream, d, h->d_list[b], (int)h->bins[b].size(), h->p, 0, in, out, flux);
-  if (fortran) sc::launch_layout(h->stream, out, raw, h->ncol, h->kmax, false);
+  if (fortran) sc::launch_layout(h->stream, out, raw, h->ncol, h->kmax, NV, false);
   HIPOK(hipGetLastError());
   HIPOK(hipMemcpyAsync(rhs, fortran ? raw : out, sizeof(double) * cells, hipMemcpyDeviceToHost, h->stream));
   if (flux_top_out)
@@ -1065,50 +1182,63 @@ int sedcol_rates(sedcol_handle *h, double *dic_release, double *n2_release)
   return SEDCOL_OK;
 }
 
-// ADAPTIVE_EULER over dt on the resident state (solver_library.F90:104-140)
-static int adaptive_euler(sedcol_handle *h, double dt, int rec, int *launches)
+// ADAPTIVE_EULER over dt on the resident state (solver_library.F90:104-140),
+// with the caller's clamp after it.  The votes are flags 5 and 6 in turn
+// (*attempt counts over a run); flag 0 collects NaN.
+static int adaptive_euler(sedcol_handle *h, double dt, int rec, int *attempt, int *launches)
 {
   int rc = ensure_scratch(h);
   if (rc) return rc;
   const Dev d = h->dev();
   double dt_int = 0.0, dt_red = dt;
   bool need_rhs = true;
+  int last = -1;
+  for (int b = 0; b < 3; ++b)
+    if (!h->bins[b].empty()) last = b;
   while (dt_int < dt) {
-    if (need_rhs) {
-      for (int b = 0; b < 3; ++b)
-        if (!h->bins[b].empty()) {
-          sc::launch_rhs_store(kLpc[b], h->stream, d, h->d_list[b], (int)h->bins[b].size(), h->p, rec, h->d_scr,
-                               h->d_scr2);
-          ++*launches;
-        }
-      need_rhs = false;
-    }
-    HIPOK(hipMemsetAsync(h->d_flag, 0, sizeof(int), h->stream));
+    int *viol = h->d_flag + 5 + (*attempt & 1), *clear = h->d_flag + 5 + ((*attempt + 1) & 1);
+    ++*attempt;
     for (int b = 0; b < 3; ++b)
       if (!h->bins[b].empty()) {
-        sc::launch_ae_check(kLpc[b], h->stream, d, h->d_list[b], (int)h->bins[b].size(), dt_red,
-                            h->p.relative_change_min, h->d_scr, h->d_flag);
+        const int n = (int)h->bins[b].size();
+        if (need_rhs)
+          sc::launch_ae_rhs(kLpc[b], h->stream, d, h->d_list[b], n, h->p, rec, dt_red, h->d_scr, h->d_scr2, viol);
+        else
+          sc::launch_ae_check(kLpc[b], h->stream, d, h->d_list[b], n, dt_red, h->p.relative_change_min, h->d_scr, viol);
+        ++*launches;
+      }
+    const bool whole = !(dt_int + dt_red < dt);  // the step that reaches dt
+    for (int b = 0; b < 3; ++b)
+      if (!h->bins[b].empty()) {
+        sc::launch_ae_commit(kLpc[b], h->stream, d, h->d_list[b], (int)h->bins[b].size(), dt_red, h->p.dt_min,
+                             whole && h->p.clamp, h->d_scr, h->d_scr2, viol, b == last ? clear : nullptr, h->d_flag);
         ++*launches;
       }
     HIPOK(hipGetLastError());
-    int viol = 0;
-    if ((rc = read_flag(h, &viol))) return rc;
-    if (viol && dt_red > h->p.dt_min) {
+    HIPOK(hipMemcpyAsync(h->h_flag, viol, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+    HIPOK(hipStreamSynchronize(h->stream));
+    need_rhs = !(h->h_flag[0] && dt_red > h->p.dt_min);
+    if (!need_rhs) {
       dt_red = dt_red * 0.25;  // the state is unchanged: the right-hand side is reused
     } else {
       if (dt_red < h->last_min_dt) h->last_min_dt = dt_red;
-      for (int b = 0; b < 3; ++b)
-        if (!h->bins[b].empty()) {
-          sc::launch_ae_commit(kLpc[b], h->stream, d, h->d_list[b], (int)h->bins[b].size(), dt_red, h->d_scr,
-                               h->d_scr2);
-          ++*launches;
-        }
       dt_int = dt_int + dt_red;
-      need_rhs = true;
     }
   }
-  HIPOK(hipGetLastError());
   return SEDCOL_OK;
+}
+
+// the only non-empty bin if its columns fit the one-workgroup adaptive Euler,
+// else -1
+static int ae_fused_bin(const sedcol_handle *h)
+{
+  int one = -1, nbins = 0;
+  for (int b = 0; b < 3; ++b)
+    if (!h->bins[b].empty()) {
+      ++nbins;
+      one = b;
+    }
+  return nbins == 1 && (int)h->bins[one].size() <= sc::kAeFusedBlock / kLpc[one] ? one : -1;
 }
 
 static int run_fixed(sedcol_handle *h, double dt, int nsteps, int method, int steps_per_launch, int *launches)
@@ -1141,17 +1271,11 @@ int sedcol_run(sedcol_handle *h, double dt, int32_t nsteps, int32_t method, int3
   if (method < SEDCOL_EULER || method > SEDCOL_EMP2)
     return fail(SEDCOL_EINVAL, "sedcol_run takes methods 0..5 (use sedcol_integrate for method 6)");
   if (h->nrec > 1) return fail(SEDCOL_EINVAL, "fixed-step runs use a single forcing record (sedcol_set_forcing)");
-  HIPOK(hipMemsetAsync(h->d_flag, 0, sizeof(int), h->stream));
+  HIPOK(hipMemsetAsync(h->d_flag, 0, sizeof(int) * 8, h->stream));
   int launches = 0;
   HIPOK(hipEventRecord(h->ev0, h->stream));
-  int one_bin = -1, nbins = 0;
-  for (int b = 0; b < 3; ++b)
-    if (!h->bins[b].empty()) {
-      ++nbins;
-      one_bin = b;
-    }
-  if (method == SEDCOL_ADAPTIVE_EULER && nbins == 1 &&
-      (int)h->bins[one_bin].size() <= sc::kAeFusedBlock / kLpc[one_bin]) {
+  const int one_bin = method == SEDCOL_ADAPTIVE_EULER ? ae_fused_bin(h) : -1;
+  if (one_bin >= 0) {
     // every wet column in one workgroup: the steps run without a host round
     // trip per attempt, in launches of kAeFusedSteps steps
     h->h_devview = h->dev();
@@ -1173,17 +1297,9 @@ int sedcol_run(sedcol_handle *h, double dt, int32_t nsteps, int32_t method, int3
       if (flag) break;
     }
   } else if (method == SEDCOL_ADAPTIVE_EULER) {
-    for (int s = 0; s < nsteps; ++s) {
-      if ((rc = adaptive_euler(h, dt, 0, &launches))) return rc;
-      if (h->p.clamp) {
-        const Dev d = h->dev();
-        for (int b = 0; b < 3; ++b)
-          if (!h->bins[b].empty()) {
-            sc::launch_clamp(kLpc[b], h->stream, d, h->d_list[b], (int)h->bins[b].size(), h->d_flag);
-            ++launches;
-          }
-      }
-    }
+    int attempt = 0;
+    for (int s = 0; s < nsteps; ++s)
+      if ((rc = adaptive_euler(h, dt, 0, &attempt, &launches))) return rc;
   } else {
     if ((rc = run_fixed(h, dt, nsteps, method, steps_per_launch, &launches))) return rc;
   }
@@ -1395,6 +1511,59 @@ int sedcol_autotune(sedcol_handle *h, double t_start, double t_span, int32_t rep
   return sedcol_get_tuning(h, best);
 }
 
+// One fixed step of a small domain (h_stage): the state goes through pinned
+// memory that the kernels read and write in place, so the call queues its
+// launches and waits once.  (Copies of their own, each with its wait, took 80
+// of the 104 us of an RK4 step of 16 columns.)
+static int step_small(sedcol_handle *h, double dt, int method, double *conc, double *flux_top_out)
+{
+  const size_t cells = NV * (size_t)h->ncell, fl = NV * (size_t)h->ncol;
+  double *st_conc = h->h_stage, *st_flux = st_conc + cells, *st_mind = st_flux + fl;
+  int *st_flag = reinterpret_cast<int *>(st_mind + 1);
+  const bool fortran = h->layout == SEDCOL_LAYOUT_FORTRAN;
+  const int ae_bin = method == SEDCOL_ADAPTIVE_EULER ? ae_fused_bin(h) : -1;
+  std::memcpy(st_conc, conc, sizeof(double) * cells);
+  if (fortran) sc::launch_layout(h->stream, st_conc, h->d_conc, h->ncol, h->kmax, NV, true);
+  // the views of the one-workgroup kernel travel in the same way
+  static_assert(sizeof(Dev) % sizeof(int) == 0 && sizeof(sedcol_params) % sizeof(double) == 0, "staged as words");
+  double *st_par = reinterpret_cast<double *>(st_flag + 2);
+  int *st_dev = reinterpret_cast<int *>(st_par + sizeof(sedcol_params) / sizeof(double));
+  if (ae_bin >= 0) {
+    const Dev view = h->dev();
+    std::memcpy(st_par, &h->p, sizeof(sedcol_params));
+    std::memcpy(st_dev, &view, sizeof(Dev));
+  }
+  sc::launch_stage(h->stream, st_conc, h->d_conc, fortran ? 0 : (long long)cells, st_par,
+                   reinterpret_cast<double *>(h->d_params), ae_bin >= 0 ? (int)(sizeof(sedcol_params) / 8) : 0, st_dev,
+                   reinterpret_cast<int *>(h->d_devview), ae_bin >= 0 ? (int)(sizeof(Dev) / 4) : 0, h->d_flag);
+  int rc, launches = 0;
+  HIPOK(hipEventRecord(h->ev0, h->stream));
+  if (ae_bin >= 0) {
+    sc::launch_ae_fused(kLpc[ae_bin], h->stream, h->d_devview, h->d_list[ae_bin], (int)h->bins[ae_bin].size(), h->p,
+                        h->d_params, 0, dt, 1, h->d_flag, h->d_small);
+    ++launches;
+  } else if ((rc = run_fixed(h, dt, 1, method, 0, &launches))) {
+    return rc;
+  }
+  HIPOK(hipEventRecord(h->ev1, h->stream));
+  if (fortran) sc::launch_layout(h->stream, h->d_conc, st_conc, h->ncol, h->kmax, NV, false);
+  sc::launch_stage(h->stream, h->d_conc, st_conc, fortran ? 0 : (long long)cells, h->d_flux, st_flux, (int)fl,
+                   h->d_flag, st_flag, 1, nullptr);
+  if (ae_bin >= 0)
+    sc::launch_stage(h->stream, h->d_small, st_mind, 1, nullptr, nullptr, 0, nullptr, nullptr, 0, nullptr);
+  HIPOK(hipGetLastError());
+  HIPOK(hipStreamSynchronize(h->stream));
+  float ms = 0.f;
+  HIPOK(hipEventElapsedTime(&ms, h->ev0, h->ev1));
+  h->last_ms = ms;
+  h->last_launches = launches;
+  if (ae_bin >= 0 && *st_mind < h->last_min_dt) h->last_min_dt = *st_mind;
+  std::memcpy(conc, st_conc, sizeof(double) * cells);
+  rc = flag_status(st_flag[0]);
+  if (!rc && flux_top_out) std::memcpy(flux_top_out, st_flux, sizeof(double) * fl);
+  return rc;
+}
+
 int sedcol_step(sedcol_handle *h, double dt, int32_t method, double *conc_inout, double *flux_top_out)
 {
   int rc = check_handle(h, true);
@@ -1402,6 +1571,9 @@ int sedcol_step(sedcol_handle *h, double dt, int32_t method, double *conc_inout,
   const DeviceScope dscope(h->device);
   if (!conc_inout) return fail(SEDCOL_EINVAL, "null argument");
   if (method < SEDCOL_EULER || method > SEDCOL_ROS2_ADAPTIVE) return fail(SEDCOL_EINVAL, "unknown method");
+  if (h->h_stage && method <= SEDCOL_EMP2 && (method != SEDCOL_ADAPTIVE_EULER || ae_fused_bin(h) >= 0) &&
+      h->nrec <= 1 && dt > 0.0 && std::isfinite(dt))
+    return step_small(h, dt, method, conc_inout, flux_top_out);
   if ((rc = sedcol_set_state(h, conc_inout))) return rc;
   if (method == SEDCOL_EMP_ADAPTIVE || method == SEDCOL_ROS2_ADAPTIVE) {
     if (h->nrec > 1) return fail(SEDCOL_EINVAL, "sedcol_step uses a single forcing record");
@@ -1522,7 +1694,8 @@ int sedcol_save_checkpoint(sedcol_handle *h, void *buf, int64_t bytes)
   std::memcpy(buf, &hd, sizeof hd);
   char *p = static_cast<char *>(buf) + sizeof hd;
   for (auto &q : ck_parts(h)) {
-    HIPOK(hipMemcpyAsync(p, q.first, q.second, hipMemcpyDeviceToHost, h->stream));
+    const int rc = copy_large(h, q.first, nullptr, p, q.second, false);
+    if (rc) return rc;
     p += q.second;
   }
   HIPOK(hipStreamSynchronize(h->stream));
@@ -1543,7 +1716,8 @@ int sedcol_load_checkpoint(sedcol_handle *h, const void *buf, int64_t bytes)
   if (bytes < ck_bytes(h)) return fail(SEDCOL_EINVAL, "checkpoint too short");
   const char *p = static_cast<const char *>(buf) + sizeof hd;
   for (auto &q : ck_parts(h)) {
-    HIPOK(hipMemcpyAsync(q.first, p, q.second, hipMemcpyHostToDevice, h->stream));
+    const int rc = copy_large(h, q.first, p, nullptr, q.second, true);
+    if (rc) return rc;
     p += q.second;
   }
   HIPOK(hipStreamSynchronize(h->stream));

@@ -1615,9 +1615,23 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
 // each sub-step is a right-hand side, a domain-wide check and a commit
 // ---------------------------------------------------------------------------
 
+// Per attempt: the right-hand side with the relative-change test (k_ae_rhs; or
+// the test alone, k_ae_check, when the step was quartered and the rates are
+// still those of the state), then k_ae_commit, which looks at the vote and
+// leaves the state alone if the step has to be quartered.  The host reads the
+// vote behind the commit and does the same comparison, so a step that is not
+// quartered costs two launches and one wait (four launches, a memset and a
+// wait between them before).  The votes alternate between two flags: a commit
+// clears the next attempt's.
+__device__ __forceinline__ bool ae_violates(double x, double r, double dt_red, double rcm)
+{
+  const double c1 = x + dt_red * r;
+  return (c1 - (1.0 + rcm) * x) < 0.0;
+}
+
 template <int LPC, int ARITH>
-__global__ __launch_bounds__(BLOCK) void k_rhs_store(Dev d, const int *list, int nlist, sedcol_params p, int rec,
-                                                     double *r_out, double *s_out)
+__global__ __launch_bounds__(BLOCK) void k_ae_rhs(Dev d, const int *list, int nlist, sedcol_params p, int rec,
+                                                  double dt_red, double *r_out, double *s_out, int *viol)
 {
   constexpr int G = BLOCK / LPC;
   __shared__ double sbc[G][2 * NV];
@@ -1638,14 +1652,18 @@ __global__ __launch_bounds__(BLOCK) void k_rhs_store(Dev d, const int *list, int
 #pragma unroll
   for (int n = 0; n < NV; ++n) x[n] = L.active ? d.conc[n * d.ncell + cell] : 0.0;
   double sC, sN;
+  bool v = false;
+  const double rcm = p.relative_change_min;
   column_rhs<LPC, ARITH>(p, L, sbc[g], x, sC, sN, [&](int n, double r, double F) {
     if (L.active) r_out[n * d.ncell + cell] = r;
     if (l == 0) d.flux[(long long)n * d.ncol + c] = F;
+    v |= L.active && ae_violates(x[n], r, dt_red, rcm);
   }, &d.zw);
   if (L.active) {
     s_out[cell] = sC;
     s_out[d.ncell + cell] = sN;
   }
+  if (v) atomicOr(viol, 1);
 }
 
 template <int LPC>
@@ -1662,19 +1680,33 @@ __global__ __launch_bounds__(BLOCK) void k_ae_check(Dev d, const int *list, int 
   const long long cell = (long long)o + l;
   bool v = false;
 #pragma unroll
-  for (int n = 0; n < NV; ++n) {
-    const double x = d.conc[n * d.ncell + cell];
-    const double c1 = x + dt_red * r_in[n * d.ncell + cell];
-    v |= (c1 - (1.0 + rcm) * x) < 0.0;
-  }
+  for (int n = 0; n < NV; ++n) v |= ae_violates(d.conc[n * d.ncell + cell], r_in[n * d.ncell + cell], dt_red, rcm);
   if (v) atomicOr(viol, 1);
 }
 
+// minimum clamp of one cell after an ode_solver call (fabm_sediment_component.F90:1726-1731):
+// the clamped value; mass to the budget array
+__device__ __forceinline__ double clamp_cell(const Dev &d, int n, long long cell, double x)
+{
+  if (x < 0.0) {
+    if (elem(n) >= 0)
+      kadd(d.cellacc[(2 + elem(n)) * d.ncell + cell], d.cellacc[(7 + elem(n)) * d.ncell + cell], 0.0 - x);
+    x = 0.0;
+  }
+  return x;
+}
+
+// the step dt_red, unless the vote *viol asks for a smaller one and dt_red is
+// above dt_min; clamp: also the minimum clamp and the NaN test (errflag bit 1)
+// that follow a whole step; *clear (or null) is set to 0
 template <int LPC>
-__global__ __launch_bounds__(BLOCK) void k_ae_commit(Dev d, const int *list, int nlist, double dt_red,
-                                                     const double *r_in, const double *s_in)
+__global__ __launch_bounds__(BLOCK) void k_ae_commit(Dev d, const int *list, int nlist, double dt_red, double dt_min,
+                                                     int clamp, const double *r_in, const double *s_in,
+                                                     const int *viol, int *clear, int *errflag)
 {
   constexpr int G = BLOCK / LPC;
+  if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
+  if (*viol && dt_red > dt_min) return;
   const int g = threadIdx.x / LPC, l = threadIdx.x % LPC;
   const int slot = blockIdx.x * G + g;
   if (slot >= nlist) return;
@@ -1692,10 +1724,19 @@ __global__ __launch_bounds__(BLOCK) void k_ae_commit(Dev d, const int *list, int
   }
   if (l >= K) return;
   const long long cell = (long long)o + l;
+  bool nan = false;
 #pragma unroll
-  for (int n = 0; n < NV; ++n) d.conc[n * d.ncell + cell] = d.conc[n * d.ncell + cell] + dt_red * r_in[n * d.ncell + cell];
+  for (int n = 0; n < NV; ++n) {
+    double x = d.conc[n * d.ncell + cell] + dt_red * r_in[n * d.ncell + cell];
+    if (clamp) {
+      nan |= x != x;
+      x = clamp_cell(d, n, cell, x);
+    }
+    d.conc[n * d.ncell + cell] = x;
+  }
   kadd(d.cellacc[cell], d.cellacc[5 * d.ncell + cell], dt_red * s_in[cell]);
   kadd(d.cellacc[d.ncell + cell], d.cellacc[6 * d.ncell + cell], dt_red * s_in[d.ncell + cell]);
+  if (nan) atomicOr(errflag, 1);
 }
 
 // ADAPTIVE_EULER steps of a small domain in one workgroup: every wet column
@@ -1703,8 +1744,7 @@ __global__ __launch_bounds__(BLOCK) void k_ae_commit(Dev d, const int *list, int
 // (the step is quartered while any cell of the domain fails the
 // relative-change test, solver_library.F90:100-140) is a block-wide vote
 // instead of a flag read by the host.  Per attempt the same operations as
-// k_rhs_store, k_ae_check and k_ae_commit, and k_clamp after each step, so
-// the results are those of the multi-launch path bit for bit.  The state
+// k_ae_rhs and k_ae_commit, so the results are those of the multi-launch path bit for bit.  The state
 // stays in registers; the top fluxes of the last right-hand side go to LDS
 // for the lanes that accumulate them.  *min_dt receives the smallest step
 // taken.  A launch stops after kAeFusedMaxAttempts attempts (errflag bit 2).
@@ -1804,10 +1844,7 @@ __global__ __launch_bounds__(BLK) void k_ae_fused(const Dev *dptr, const int *li
       bool v = false;
       if (act) {
 #pragma unroll
-        for (int n = 0; n < NV; ++n) {
-          const double c1 = x[n] + dt_red * r[n];
-          v |= (c1 - (1.0 + rcm) * x[n]) < 0.0;
-        }
+        for (int n = 0; n < NV; ++n) v |= ae_violates(x[n], r[n], dt_red, rcm);
       }
       const int viol = ONE ? __any(v) : __syncthreads_or(v);
       if (viol && dt_red > p.dt_min) {
@@ -1870,32 +1907,6 @@ __global__ __launch_bounds__(BLK) void k_ae_fused(const Dev *dptr, const int *li
     d.diag[c] = dg;
   }
   if (threadIdx.x == 0) *min_dt = mind;
-}
-
-// minimum clamp after an ode_solver call (fabm_sediment_component.F90:1726-1731)
-template <int LPC>
-__global__ __launch_bounds__(BLOCK) void k_clamp(Dev d, const int *list, int nlist, int *errflag)
-{
-  constexpr int G = BLOCK / LPC;
-  const int g = threadIdx.x / LPC, l = threadIdx.x % LPC;
-  const int slot = blockIdx.x * G + g;
-  if (slot >= nlist) return;
-  const int c = list[slot];
-  const int o = d.off[c], K = d.off[c + 1] - o;
-  if (l >= K) return;
-  const long long cell = (long long)o + l;
-  bool nan = false;
-#pragma unroll
-  for (int n = 0; n < NV; ++n) {
-    const double x = d.conc[n * d.ncell + cell];
-    nan |= x != x;
-    if (x < 0.0) {
-      if (elem(n) >= 0)
-        kadd(d.cellacc[(2 + elem(n)) * d.ncell + cell], d.cellacc[(7 + elem(n)) * d.ncell + cell], 0.0 - x);
-      d.conc[n * d.ncell + cell] = 0.0;
-    }
-  }
-  if (nan) atomicOr(errflag, 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -2372,36 +2383,77 @@ void launch_fill_dbl(hipStream_t st, double *p, long long n, double v)
   hipLaunchKernelGGL(k_fill_dbl, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p, n, v);
 }
 
-// Fortran state conc(i,j,k,n) = f[(n K + k) ncol + c] against the packed
-// state x[n ncell + c K + k] of a uniform grid (ncell = ncol K); one thread
-// per element, in Fortran order (reads or writes of f coalesced).
-__global__ void k_layout(const double *src, double *dst, int ncol, int K, int to_packed)
+// Fortran arrays f[(n K + k) ncol + c] against packed ones x[(n ncol + c) K + k]
+// of a uniform grid, nvar planes: a transposition of ncol x K per plane.  64
+// columns per block go through LDS, so that both sides are read and written in
+// whole lines: rows of 64 columns of f, and one run of 64 K values of x (one
+// thread per element, in Fortran order, wrote or read x with a stride of K:
+// 32 us for 11 planes of 8000 columns of 30 layers, this 14 us; 90000 columns
+// take 121 us, 3.9 TB/s).
+constexpr int kLayoutCols = 64;
+__global__ __launch_bounds__(256) void k_layout(const double *__restrict__ src, double *__restrict__ dst, int ncol,
+                                                int K, int to_packed)
+{
+  __shared__ double tile[SEDCOL_KMAX][kLayoutCols + 1];
+  const int c0 = blockIdx.x * kLayoutCols;
+  const int nc = ncol - c0 < kLayoutCols ? ncol - c0 : kLayoutCols;
+  const long long plane = (long long)ncol * K;
+  const long long f0 = (long long)blockIdx.y * plane + c0;               // f of (k = 0, c0)
+  const long long x0 = (long long)blockIdx.y * plane + (long long)c0 * K;  // x of (c0, k = 0)
+  const int cc = threadIdx.x % kLayoutCols, kq = threadIdx.x / kLayoutCols;
+  if (to_packed) {
+    if (cc < nc)
+      for (int k = kq; k < K; k += 256 / kLayoutCols) tile[k][cc] = src[f0 + (long long)k * ncol + cc];
+    __syncthreads();
+    for (int i = threadIdx.x; i < nc * K; i += 256) {
+      const int c = i / K;
+      dst[x0 + i] = tile[i - c * K][c];
+    }
+  } else {
+    for (int i = threadIdx.x; i < nc * K; i += 256) {
+      const int c = i / K;
+      tile[i - c * K][c] = src[x0 + i];
+    }
+    __syncthreads();
+    if (cc < nc)
+      for (int k = kq; k < K; k += 256 / kLayoutCols) dst[f0 + (long long)k * ncol + cc] = tile[k][cc];
+  }
+}
+
+void launch_layout(hipStream_t st, const double *src, double *dst, int ncol, int K, int nvar, bool to_packed)
+{
+  if (ncol <= 0 || K <= 0 || nvar <= 0) return;
+  hipLaunchKernelGGL(k_layout, dim3((unsigned)((ncol + kLayoutCols - 1) / kLayoutCols), (unsigned)nvar), dim3(256), 0,
+                     st, src, dst, ncol, K, to_packed ? 1 : 0);
+}
+
+// n doubles, and up to three small copies on the way: from, or to, pinned host
+// memory that the device reads and writes in place
+__global__ void k_stage(const double *__restrict__ src, double *__restrict__ dst, long long n, const double *s1,
+                        double *d1, int n1, const int *s2, int *d2, int n2, int *zero)
 {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long plane = (long long)ncol * K;
-  if (i >= (long long)NV * plane) return;
-  const long long n = i / plane;
-  const long long r = i - n * plane;
-  const long long k = r / ncol;
-  const long long c = r - k * ncol;
-  const long long j = n * plane + c * K + k;
-  if (to_packed) dst[j] = src[i];
-  else dst[i] = src[j];
+  if (i < n) dst[i] = src[i];
+  if (i < n1) d1[i] = s1[i];
+  if (i < n2) d2[i] = s2[i];
+  if (zero && i == 0) *zero = 0;
 }
 
-void launch_layout(hipStream_t st, const double *src, double *dst, int ncol, int K, bool to_packed)
+void launch_stage(hipStream_t st, const double *src, double *dst, long long n, const double *s1, double *d1, int n1,
+                  const int *s2, int *d2, int n2, int *zero)
 {
-  const long long n = (long long)NV * ncol * K;
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_layout, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, src, dst, ncol, K,
-                     to_packed ? 1 : 0);
+  long long m = n > n1 ? n : n1;
+  m = m > n2 ? m : n2;
+  if (m < 1) m = 1;
+  hipLaunchKernelGGL(k_stage, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, st, src, dst, n, s1, d1, n1, s2, d2,
+                     n2, zero);
 }
 
-void launch_rhs_store(int lpc, hipStream_t st, const Dev &d, const int *list, int n, const sedcol_params &p, int rec,
-                      double *r_out, double *s_out)
+void launch_ae_rhs(int lpc, hipStream_t st, const Dev &d, const int *list, int n, const sedcol_params &p, int rec,
+                   double dt_red, double *r_out, double *s_out, int *viol)
 {
-  SC_DISPATCH_ARITH(p, SC_DISPATCH_LPC(lpc, hipLaunchKernelGGL((k_rhs_store<LPC, AR>), grid_for<LPC>(n), dim3(BLOCK),
-                                                               0, st, d, list, n, p, rec, r_out, s_out)));
+  SC_DISPATCH_ARITH(p, SC_DISPATCH_LPC(lpc, hipLaunchKernelGGL((k_ae_rhs<LPC, AR>), grid_for<LPC>(n), dim3(BLOCK), 0,
+                                                               st, d, list, n, p, rec, dt_red, r_out, s_out, viol)));
 }
 
 void launch_ae_check(int lpc, hipStream_t st, const Dev &d, const int *list, int n, double dt_red, double rcm,
@@ -2411,11 +2463,11 @@ void launch_ae_check(int lpc, hipStream_t st, const Dev &d, const int *list, int
                                           dt_red, rcm, r_in, viol));
 }
 
-void launch_ae_commit(int lpc, hipStream_t st, const Dev &d, const int *list, int n, double dt_red,
-                      const double *r_in, const double *s_in)
+void launch_ae_commit(int lpc, hipStream_t st, const Dev &d, const int *list, int n, double dt_red, double dt_min,
+                      bool clamp, const double *r_in, const double *s_in, const int *viol, int *clear, int *errflag)
 {
   SC_DISPATCH_LPC(lpc, hipLaunchKernelGGL((k_ae_commit<LPC>), grid_for<LPC>(n), dim3(BLOCK), 0, st, d, list, n,
-                                          dt_red, r_in, s_in));
+                                          dt_red, dt_min, clamp ? 1 : 0, r_in, s_in, viol, clear, errflag));
 }
 
 void launch_ae_fused(int lpc, hipStream_t st, const Dev *d_dev, const int *list, int n, const sedcol_params &p,
@@ -2435,12 +2487,6 @@ void launch_ae_fused(int lpc, hipStream_t st, const Dev *d_dev, const int *list,
     SC_AE_FUSED(kAeFusedBlock);
   }
 #undef SC_AE_FUSED
-}
-
-void launch_clamp(int lpc, hipStream_t st, const Dev &d, const int *list, int n, int *errflag)
-{
-  SC_DISPATCH_LPC(lpc, hipLaunchKernelGGL((k_clamp<LPC>), grid_for<LPC>(n), dim3(BLOCK), 0, st, d, list, n,
-                                          errflag));
 }
 
 void launch_budget(int lpc, hipStream_t st, const Dev &d, const int *list, int n, double *budget)

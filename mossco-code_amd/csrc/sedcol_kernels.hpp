@@ -94,21 +94,28 @@ void launch_warm_profiles(int lpc, hipStream_t st, const Dev &d, const int *list
 // v into p[0..n-1] (a kernel, so that it can be captured in a graph)
 void launch_fill_int(hipStream_t st, int *p, int n, int v);
 void launch_fill_dbl(hipStream_t st, double *p, long long n, double v);
-// state of a uniform grid between the Fortran layout (ncol, K, NV) and the
-// packed one (NV, ncol*K): src Fortran -> dst packed when to_packed, else
-// src packed -> dst Fortran
-void launch_layout(hipStream_t st, const double *src, double *dst, int ncol, int K, bool to_packed);
+// nvar planes of a uniform grid between the Fortran layout (ncol, K, nvar) and
+// the packed one (nvar, ncol*K): src Fortran -> dst packed when to_packed, else
+// src packed -> dst Fortran; not in place
+void launch_layout(hipStream_t st, const double *src, double *dst, int ncol, int K, int nvar, bool to_packed);
 // boundary conditions of the listed columns from the fields at the soil
 // surface into forcing record 0 (present: bit n set when variable n's
 // field exists)
 void launch_assemble(hipStream_t st, const Dev &d, const int *list, int n, const sedcol_params &p, unsigned present,
                      const double *ts, const double *cs, const double *ws, double *temp, double *cbw, double *fup);
-void launch_rhs_store(int lpc, hipStream_t st, const Dev &d, const int *list, int n, const sedcol_params &p, int rec,
-                      double *r_out, double *s_out);
+// dst[0..n-1] = src, d1[0..n1-1] = s1, d2[0..n2-1] = s2, *zero = 0 (zero may be
+// null), in one launch; host sides are pinned memory
+void launch_stage(hipStream_t st, const double *src, double *dst, long long n, const double *s1, double *d1, int n1,
+                  const int *s2, int *d2, int n2, int *zero);
+// ADAPTIVE_EULER attempts of any domain: rates into r_out (NV*ncell) and sinks
+// into s_out, or'ing the relative-change test of step dt_red into *viol; the
+// test alone on stored rates; the step, if the vote or dt_min allows it
+void launch_ae_rhs(int lpc, hipStream_t st, const Dev &d, const int *list, int n, const sedcol_params &p, int rec,
+                   double dt_red, double *r_out, double *s_out, int *viol);
 void launch_ae_check(int lpc, hipStream_t st, const Dev &d, const int *list, int n, double dt_red, double rcm,
                      const double *r_in, int *viol);
-void launch_ae_commit(int lpc, hipStream_t st, const Dev &d, const int *list, int n, double dt_red,
-                      const double *r_in, const double *s_in);
+void launch_ae_commit(int lpc, hipStream_t st, const Dev &d, const int *list, int n, double dt_red, double dt_min,
+                      bool clamp, const double *r_in, const double *s_in, const int *viol, int *clear, int *errflag);
 // ADAPTIVE_EULER steps of a domain whose wet columns all sit in one bin of
 // at most kAeFusedBlock / lpc columns, in one workgroup (no host round trip
 // per attempt); errflag bit 1 NaN, bit 2 attempt limit; *min_dt (device) the
@@ -118,7 +125,6 @@ constexpr int kAeFusedMaxAttempts = 1 << 22;
 // (d_dev, d_params: device copies of the domain view and of p)
 void launch_ae_fused(int lpc, hipStream_t st, const Dev *d_dev, const int *list, int n, const sedcol_params &p,
                      const sedcol_params *d_params, int rec, double dt, int nsteps, int *errflag, double *min_dt);
-void launch_clamp(int lpc, hipStream_t st, const Dev &d, const int *list, int n, int *errflag);
 void launch_budget(int lpc, hipStream_t st, const Dev &d, const int *list, int n, double *budget);
 void launch_inventory(int lpc, hipStream_t st, const Dev &d, const int *list, int n, double *inv);
 void launch_residual(int lpc, hipStream_t st, const Dev &d, const int *list, int n, const sedcol_params &p, int rec,
