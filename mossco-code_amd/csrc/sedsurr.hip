@@ -3,19 +3,18 @@
 // A multilayer perceptron trained and evaluated with hand-written kernels:
 //   k_gemm     bf16 x bf16 -> fp32 on the MFMA units (v_mfma_f32_32x32x16
 //              bf16), 64 x 64 block tiles, four waves of 32 x 32, operands
-//              staged through LDS; the three products of training (forward
-//              H W, data gradient dZ W^T, weight gradient H^T dZ) are the
-//              transpose variants of one kernel, with fused epilogues (bias
-//              + GELU storing the pre-activation, bias only, GELU'
-//              product, plain fp32)
-//   k_loss     squared error, its gradient in bf16, per-block loss sums
-//   k_sum_slices  the split-k weight gradients, summed in a fixed order
-//              (for the gradient query; in training k_adam sums them);
-//              the bias gradients (column sums of dZ) come out of the
-//              weight-gradient product as the row of a ones column
-//              appended to its left operand
-//   k_adam     Adam on the fp32 master parameters, writing the bf16 copy
+//              staged through LDS: the forward product H W with its epilogues
+//              (bias + GELU storing the pre-activation; bias only; bias, the
+//              squared error and its gradient in bf16)
+//   k_bwd      the data gradient dZ W^T (with the GELU' product) and the weight
+//              gradient H^T dZ of a layer in one launch, by the same tiles; the
+//              bias gradients (column sums of dZ) are the row of a ones column
+//              appended to the left operand, and a product over many rows is
+//              split into slices, summed in a fixed order by their reader
+//   k_adam     Adam on the fp32 master parameters, writing the bf16 copy, with
+//              the next step's gather and the step's loss in blocks of its own
 //   k_gather   minibatch rows of the resident training set, bf16 inputs
+//   k_set_params, k_get_params  between the caller's and the padded layout
 // Layer widths are padded on the device (inputs to 32, outputs to a
 // multiple of 64) with zero weights, which keeps the products exact and the
 // padded parameters at zero through training.
@@ -60,34 +59,30 @@ __device__ inline float gelu_grad(float z)
 }
 
 constexpr int BM = 64, BN = 64, BK = 64;
-enum { EPI_F32 = 0, EPI_BIAS = 1, EPI_BIAS_GELU = 2, EPI_GELU_GRAD = 3 };
+enum { EPI_F32 = 0, EPI_BIAS = 1, EPI_BIAS_GELU = 2, EPI_GELU_GRAD = 3, EPI_LOSS = 4 };
 
 struct Epi {
-  float *out_f;       // fp32 output (EPI_F32, EPI_BIAS; pre-activation for EPI_BIAS_GELU)
+  float *out_f;       // fp32 output (EPI_F32, EPI_BIAS; pre-activation for EPI_BIAS_GELU; squared
+                      // errors per block for EPI_LOSS)
   int ldo;
   long long zstride;  // EPI_F32 with split k: distance between the slices' outputs
-  bf16 *out_h;        // bf16 output (EPI_BIAS_GELU activation, EPI_GELU_GRAD dZ)
+  bf16 *out_h;        // bf16 output (EPI_BIAS_GELU activation, EPI_GELU_GRAD and EPI_LOSS dZ)
   int ldh;
   const float *bias;  // EPI_BIAS, EPI_BIAS_GELU
-  const float *zin;   // EPI_GELU_GRAD: pre-activation of the layer below
+  const float *zin;   // EPI_GELU_GRAD: pre-activation of the layer below; EPI_LOSS: targets
   int ldz;
+  float scale;        // EPI_LOSS: dZ = scale (output - target) over the first n_out columns
+  int n_out;
 };
 
-// eight consecutive bf16 (16 bytes) of a row-major array, zero outside
-// [0, lim) of the fastest index; one 16-byte load when all eight are inside
-// and the address is aligned
-__device__ inline uint4 load8(const bf16 *__restrict__ p, int i0, int lim, bool row_ok)
+// eight consecutive bf16 of a row-major array, or zeros.  Every leading
+// dimension is a multiple of 32 and every array starts on a 16-byte boundary, so
+// a group of eight is inside or outside as a whole and its load is aligned.
+__device__ __forceinline__ uint4 load8(const bf16 *__restrict__ p, bool ok)
 {
-  if (row_ok && i0 + 7 < lim && ((reinterpret_cast<uintptr_t>(p + i0) & 15u) == 0))
-    return *reinterpret_cast<const uint4 *>(p + i0);
-  unsigned w[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const unsigned lo = (row_ok && i0 + 2 * j < lim) ? p[i0 + 2 * j] : 0u;
-    const unsigned hi = (row_ok && i0 + 2 * j + 1 < lim) ? p[i0 + 2 * j + 1] : 0u;
-    w[j] = lo | (hi << 16);
-  }
-  return make_uint4(w[0], w[1], w[2], w[3]);
+  uint4 v = make_uint4(0u, 0u, 0u, 0u);
+  if (ok) v = *reinterpret_cast<const uint4 *>(p);
+  return v;
 }
 __device__ inline bf16 elem8(const uint4 &w, int j)
 {
@@ -95,201 +90,264 @@ __device__ inline bf16 elem8(const uint4 &w, int j)
   return (bf16)((j & 1) ? (u >> 16) : (u & 0xffffu));
 }
 
-// C (M x N) = op(A) (M x K) op(B) (K x N); op(A)(m,k) = TA ? A[k lda + m] :
-// A[m lda + k], op(B)(k,n) = TB ? B[n ldb + k] : B[k ldb + n].  Out-of-range
-// rows, columns and k are loaded as zero and not stored.  Block z of the
-// grid takes k in [z kchunk, (z+1) kchunk) and (EPI_F32) writes its partial
-// product at out_f + z zstride.
-//
-// Both tiles sit in LDS with k contiguous (A as [m][k], B as [n][k]), so a
-// lane's MFMA operand (8 consecutive k of one row or column) is one 16-byte
-// LDS read.  v_mfma_f32_32x32x16_bf16: lane l supplies row (A) / column (B)
-// l % 32 at k = 8 (l / 32) + 0..7.  The k loop is software pipelined: the
-// next 64-wide k tile is loaded from global memory into registers while the
-// MFMAs run on the current one, and the LDS tiles are double buffered, so
-// one barrier per k tile suffices.  The MFMAs accumulate k in increasing
-// order of 16-wide steps, as for any tile width.
-template <bool TA, bool TB, int EPI>
-__global__ __launch_bounds__(256) void k_gemm(int M, int N, int K, int kchunk, const bf16 *__restrict__ A, int lda,
-                                              const bf16 *__restrict__ B, int ldb, Epi e, int ones_row)
+// Tiles of both operands in LDS with k contiguous (A as [m][k], B as [n][k]),
+// double buffered.  Rows of 128 bytes without padding; the 16-byte chunk c of
+// row r sits at c ^ swz(r), so that the lanes of an operand read (32
+// consecutive rows, one chunk) and of a transposing write (rows 8 apart) meet
+// different banks: with rows padded to 144 bytes those writes met in fours.
+struct Tiles {
+  bf16 a[2][BM][BK], b[2][BN][BK];
+};
+__device__ __forceinline__ int swz(int r) { return ((r >> 3) ^ (r >> 1)) & 7; }
+// the element at (r, k) of a tile
+__device__ __forceinline__ bf16 *at(bf16 (&t)[64][BK], int r, int k)
 {
-  constexpr int LDK = BK + 8;  // row pitch of the tiles: 144 bytes, 16-byte aligned rows
-  __shared__ __attribute__((aligned(16))) bf16 sA[2][BM][LDK];
-  __shared__ __attribute__((aligned(16))) bf16 sB[2][BN][LDK];
+  return &t[r][((((k >> 3) ^ swz(r)) << 3)) | (k & 7)];
+}
+
+// One 64 x 64 tile (bx, by) of C (M x N) = op(A) (M x K) op(B) (K x N);
+// op(A)(m,k) = TA ? A[k lda + m] : A[m lda + k], op(B)(k,n) = TB ? B[n ldb + k] :
+// B[k ldb + n].  Out-of-range rows, columns and k are loaded as zero and not
+// stored.  Slice z takes k in [z kchunk, (z+1) kchunk) and (EPI_F32) writes its
+// partial product at out_f + z zstride.
+//
+// With k contiguous in LDS a lane's MFMA operand (8 consecutive k of one row or
+// column) is one 16-byte LDS read.  v_mfma_f32_32x32x16_bf16: lane l supplies
+// row (A) / column (B) l % 32 at k = 8 (l / 32) + 0..7.  A tile is four MFMAs per
+// wave, so the products here are bound by the latency of their loads and by what
+// surrounds the k loop: kDepth tiles are in flight in registers, the double buffer
+// leaves one barrier per tile, and the code is kept short.  The MFMAs accumulate k
+// in increasing order of 16-wide steps, whatever the depth.  Mean time of the
+// three hidden layers' forward products of 4096 rows (32, 512, 512 -> 512) and of
+// a hidden layer's backward pass (2 x 2.1 GFLOP):
+//   one tile in flight, rows padded to 144 bytes         13.9 us   34.6 us (two launches)
+//   four tiles, the backward pass in one launch          14.2      29.6
+//   ... chunks exchanged instead of padding              13.5      26.3
+//   ... two tiles (106 instead of 134 registers)         13.2      23.7
+//   ... whole 16-byte loads, rolled epilogue, XCD order  10.6      19.0
+constexpr int kDepth = 2;
+static_assert(kDepth % 2 == 0, "the two buffers alternate");
+template <bool TA, bool TB, int EPI>
+__device__ __forceinline__ void gemm_tile(Tiles &S, int bx, int by, int z, int M, int N, int K, int kchunk,
+                                          const bf16 *__restrict__ A, int lda, const bf16 *__restrict__ B, int ldb,
+                                          const Epi &e, int ones_row)
+{
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int bm = blockIdx.y * BM, bn = blockIdx.x * BN;
+  const int bm = by * BM, bn = bx * BN;
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  const int kb0 = blockIdx.z * kchunk;
+  const int kb0 = z * kchunk;
   const int kend = min(K, kb0 + kchunk);
   f32x16 acc;
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
   const int r = lane & 31, q8 = (lane >> 5) * 8;
 
-  // this thread's share of a 64 x 64 tile of each operand: eight
-  // consecutive elements at idx = 8 tid + 2048 h, h = 0, 1
-  uint4 ra[2], rb[2];
-  // Operands stored k-major (TA for A, !TB for B) are transposed into the
-  // k-contiguous LDS tiles: a thread loads the same eight m (or n) at two
-  // consecutive k (k even), so every tile element pair (m, k..k+1) is one
-  // 4-byte LDS write.
-  const int tm = (tid % 8) * 8, tk = 2 * (tid / 8);
-  auto fetch = [&](int k0) {
+  // This thread's share of a 64 x 64 tile of each operand: eight consecutive k
+  // of the rows tid / 8 + 32 h, h = 0, 1, or, for an operand stored k-major (TA
+  // for A, !TB for B), which is transposed on its way into LDS, the same eight m
+  // (or n) at two consecutive k (k even), so that every tile element pair
+  // (m, k..k+1) is one 4-byte LDS write.
+  uint4 ra[kDepth][2], rb[kDepth][2];
+  const int c8 = (tid % 8) * 8, r8 = tid / 8;
+  auto fetch = [&](uint4 (&va)[2], uint4 (&vb)[2], int k0) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int idx = tid * 8 + 2048 * h;
-      if (TA) {  // A stored k-major: m fastest
-        const int m = tm, k = tk + h;
-        // row ones_row of op(A) is all ones (read nothing there): the
-        // product's row ones_row is then the column sums of op(B)
-        const int lim = ones_row >= 0 ? ones_row : M;
-        ra[h] = load8(A + (size_t)(k0 + k) * lda, bm + m, lim, k0 + k < kend);
-        const int j1 = ones_row - (bm + m);
-        if (j1 >= 0 && j1 < 8 && k0 + k < kend) {
-          const unsigned one = 0x3F80u;  // bf16 1.0
-          if (j1 == 0) ra[h].x = (ra[h].x & 0xffff0000u) | one;
-          else if (j1 == 1) ra[h].x = (ra[h].x & 0xffffu) | (one << 16);
-          else if (j1 == 2) ra[h].y = (ra[h].y & 0xffff0000u) | one;
-          else if (j1 == 3) ra[h].y = (ra[h].y & 0xffffu) | (one << 16);
-          else if (j1 == 4) ra[h].z = (ra[h].z & 0xffff0000u) | one;
-          else if (j1 == 5) ra[h].z = (ra[h].z & 0xffffu) | (one << 16);
-          else if (j1 == 6) ra[h].w = (ra[h].w & 0xffff0000u) | one;
-          else ra[h].w = (ra[h].w & 0xffffu) | (one << 16);
-        }
+      if (TA) {
+        const int m = bm + c8, k = k0 + 2 * r8 + h;
+        // row ones_row of op(A) is all ones: the product's row ones_row is then
+        // the column sums of op(B)
+        va[h] = load8(A + (size_t)k * lda + m, k < kend && m < ones_row);
+        if (m == ones_row && k < kend) va[h].x = 0x3F80u;  // bf16 1.0
       } else {
-        const int m = idx / BK, k = idx % BK;
-        ra[h] = load8(A + (size_t)(bm + m) * lda, k0 + k, kend, bm + m < M);
+        const int m = bm + r8 + 32 * h, k = k0 + c8;
+        va[h] = load8(A + (size_t)m * lda + k, k < kend && m < M);
       }
-      if (TB) {  // B stored n-major: k fastest
-        const int n = idx / BK, kb = idx % BK;
-        rb[h] = load8(B + (size_t)(bn + n) * ldb, k0 + kb, kend, bn + n < N);
+      if (TB) {
+        const int n = bn + r8 + 32 * h, k = k0 + c8;
+        vb[h] = load8(B + (size_t)n * ldb + k, k < kend && n < N);
       } else {
-        const int kb = tk + h, n = tm;
-        rb[h] = load8(B + (size_t)(k0 + kb) * ldb, bn + n, N, k0 + kb < kend);
+        const int n = bn + c8, k = k0 + 2 * r8 + h;
+        vb[h] = load8(B + (size_t)k * ldb + n, k < kend && n < ldb);
       }
     }
   };
   auto pair = [](const uint4 &lo, const uint4 &hi, int j) {
     return (unsigned)elem8(lo, j) | ((unsigned)elem8(hi, j) << 16);
   };
-  auto stage = [&](int buf) {
+  auto stage = [&](int buf, const uint4 (&va)[2], const uint4 (&vb)[2]) {
     if (TA) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) *reinterpret_cast<unsigned *>(&sA[buf][tm + j][tk]) = pair(ra[0], ra[1], j);
+      for (int j = 0; j < 8; ++j) *reinterpret_cast<unsigned *>(at(S.a[buf], c8 + j, 2 * r8)) = pair(va[0], va[1], j);
     } else {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int idx = tid * 8 + 2048 * h;
-        const int m = idx / BK, k = idx % BK;
-        *reinterpret_cast<uint4 *>(&sA[buf][m][k]) = ra[h];
-      }
+      for (int h = 0; h < 2; ++h) *reinterpret_cast<uint4 *>(at(S.a[buf], r8 + 32 * h, c8)) = va[h];
     }
     if (TB) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int idx = tid * 8 + 2048 * h;
-        const int n = idx / BK, kb = idx % BK;
-        *reinterpret_cast<uint4 *>(&sB[buf][n][kb]) = rb[h];
-      }
+      for (int h = 0; h < 2; ++h) *reinterpret_cast<uint4 *>(at(S.b[buf], r8 + 32 * h, c8)) = vb[h];
     } else {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) *reinterpret_cast<unsigned *>(&sB[buf][tm + j][tk]) = pair(rb[0], rb[1], j);
+      for (int j = 0; j < 8; ++j) *reinterpret_cast<unsigned *>(at(S.b[buf], c8 + j, 2 * r8)) = pair(vb[0], vb[1], j);
     }
   };
 
-  int buf = 0;
-  if (kb0 < kend) fetch(kb0);
-  for (int k0 = kb0; k0 < kend; k0 += BK) {
-    stage(buf);
-    __syncthreads();
-    if (k0 + BK < kend) fetch(k0 + BK);
 #pragma unroll
-    for (int kk = 0; kk < BK; kk += 16) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8 *>(&sA[buf][wm + r][kk + q8]);
-      const bf16x8 b = *reinterpret_cast<const bf16x8 *>(&sB[buf][wn + r][kk + q8]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+  for (int u = 0; u < kDepth; ++u)
+    if (kb0 + u * BK < kend) fetch(ra[u], rb[u], kb0 + u * BK);
+  for (int k0 = kb0; k0 < kend; k0 += kDepth * BK) {
+#pragma unroll
+    for (int u = 0; u < kDepth; ++u) {
+      const int ku = k0 + u * BK;
+      if (ku < kend) {
+        const int buf = u & 1;
+        stage(buf, ra[u], rb[u]);
+        __syncthreads();
+        if (ku + kDepth * BK < kend) fetch(ra[u], rb[u], ku + kDepth * BK);
+#pragma unroll
+        for (int kk = 0; kk < BK; kk += 16) {
+          const bf16x8 a = *reinterpret_cast<const bf16x8 *>(at(S.a[buf], wm + r, kk + q8));
+          const bf16x8 b = *reinterpret_cast<const bf16x8 *>(at(S.b[buf], wn + r, kk + q8));
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+        }
+      }
     }
-    buf ^= 1;
   }
-  // accumulator layout of the 32 x 32 result: lane holds column (lane & 31),
-  // register v holds row 8 (v / 4) + 4 (lane / 32) + v % 4
-  const int col = bn + wn + r;
-  if (col >= N) return;
-  const int q = (lane >> 5) * 4;
+  // The result goes through LDS, so that the epilogue is one rolled loop over
+  // four columns per thread with 16-byte loads and stores.  In the accumulator of
+  // the 32 x 32 product a lane holds column (lane & 31), register v holds row
+  // 8 (v / 4) + 4 (lane / 32) + v % 4.
+  __syncthreads();  // the tiles are done with
+  float (*C)[BN + 4] = reinterpret_cast<float (*)[BN + 4]>(&S);
 #pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int row = bm + wm + 8 * (v >> 2) + q + (v & 3);
-    if (row >= M) continue;
-    const float x = acc[v];
-    if constexpr (EPI == EPI_F32) {
-      e.out_f[blockIdx.z * e.zstride + (size_t)row * e.ldo + col] = x;
-    } else if constexpr (EPI == EPI_BIAS) {
-      e.out_f[(size_t)row * e.ldo + col] = x + e.bias[col];
-    } else if constexpr (EPI == EPI_BIAS_GELU) {
-      const float z = x + e.bias[col];
-      e.out_f[(size_t)row * e.ldo + col] = z;
-      e.out_h[(size_t)row * e.ldh + col] = to_bf16(gelu(z));
-    } else {
-      const float z = e.zin[(size_t)row * e.ldz + col];
-      e.out_h[(size_t)row * e.ldh + col] = to_bf16(x * gelu_grad(z));
+  for (int v = 0; v < 16; ++v) C[wm + 8 * (v >> 2) + (lane >> 5) * 4 + (v & 3)][wn + r] = acc[v];
+  __syncthreads();
+  float sq = 0.0f;  // EPI_LOSS: the thread's squared errors
+  if constexpr (EPI == EPI_BIAS) {
+    // any width and any alignment of the output
+    const int col = bn + lane;
+    const float bias = col < N ? e.bias[col] : 0.0f;
+    for (int row = wave; row < BM; row += 4)
+      if (bm + row < M && col < N) e.out_f[(size_t)(bm + row) * e.ldo + col] = C[row][lane] + bias;
+  } else {
+    const int c4 = (tid % 16) * 4, col = bn + c4;
+    float4 bias = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if constexpr (EPI == EPI_BIAS_GELU || EPI == EPI_LOSS)
+      if (col < N) bias = *reinterpret_cast<const float4 *>(e.bias + col);
+#pragma unroll 1
+    for (int t = tid / 16; t < BM; t += 16) {
+      const int row = bm + t;
+      if (row >= M || col >= N) break;
+      const float4 x4 = *reinterpret_cast<const float4 *>(&C[t][c4]);
+      float x[4] = {x4.x + bias.x, x4.y + bias.y, x4.z + bias.z, x4.w + bias.w};
+      if constexpr (EPI == EPI_F32) {
+        *reinterpret_cast<float4 *>(e.out_f + z * e.zstride + (size_t)row * e.ldo + col) = x4;
+      } else {
+        if constexpr (EPI == EPI_BIAS_GELU) {
+          *reinterpret_cast<float4 *>(e.out_f + (size_t)row * e.ldo + col) = make_float4(x[0], x[1], x[2], x[3]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) x[j] = gelu(x[j]);
+        } else {
+          const float4 z4 = *reinterpret_cast<const float4 *>(e.zin + (size_t)row * e.ldz + col);
+          const float zs[4] = {z4.x, z4.y, z4.z, z4.w};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            if constexpr (EPI == EPI_GELU_GRAD) {
+              x[j] *= gelu_grad(zs[j]);
+            } else {
+              const float d = col + j < e.n_out ? x[j] - zs[j] : 0.0f;
+              sq += d * d;
+              x[j] = e.scale * d;
+            }
+          }
+        }
+        const unsigned lo = to_bf16(x[0]) | ((unsigned)to_bf16(x[1]) << 16);
+        const unsigned hi = to_bf16(x[2]) | ((unsigned)to_bf16(x[3]) << 16);
+        *reinterpret_cast<uint2 *>(e.out_h + (size_t)row * e.ldh + col) = make_uint2(lo, hi);
+      }
     }
+  }
+  if constexpr (EPI == EPI_LOSS) {
+    // the block's squared errors, in a fixed order: lanes by halves, then the
+    // four waves
+    __syncthreads();  // the results are done with
+    float *red = reinterpret_cast<float *>(&S);
+    red[tid] = sq;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+      if (tid < w) red[tid] += red[tid + w];
+      __syncthreads();
+    }
+    if (tid == 0) e.out_f[by * ((N + BN - 1) / BN) + bx] = red[0];
   }
 }
 
-// out[i] = sum over s < S of part[s stride + i], in order of s
-__global__ void k_sum_slices(const float *part, int S, long long stride, long long n, float *out)
+// Blocks go to the eight XCDs in turn, each with an L2 of its own: block i of n
+// takes tile xcd_order(i, n), which hands every XCD one run of consecutive tiles.
+// With the column tiles counted fastest, a run shares its rows of the left
+// operand, and in k_bwd the gradients' slices of the batch.
+__device__ __forceinline__ int xcd_order(int i, int n)
 {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    float a = 0.0f;
-    for (int sl = 0; sl < S; ++sl) a += part[sl * stride + i];
-    out[i] = a;
+  const int x = i & 7, q = n >> 3, rest = n & 7;
+  return x * q + min(x, rest) + (i >> 3);
+}
+
+template <int EPI>
+__global__ __launch_bounds__(256) void k_gemm(int M, int N, int K, const bf16 *__restrict__ A, int lda,
+                                              const bf16 *__restrict__ B, int ldb, Epi e)
+{
+  __shared__ __attribute__((aligned(16))) Tiles S;
+  const int nx = gridDim.x, t = xcd_order(blockIdx.y * nx + blockIdx.x, nx * gridDim.y);
+  gemm_tile<false, false, EPI>(S, t % nx, t / nx, 0, M, N, K, K, A, lda, B, ldb, e, -1);
+}
+
+// Both products of a layer's backward pass, which need the same dZ and not each
+// other: the first nd blocks make tiles of dZ W^T (with GELU'), the others those
+// of [H_in, 1]^T dZ.  Neither product fills the device to its end alone.
+struct Bwd {
+  const bf16 *dz, *w, *hin;
+  int b, win, wout, kchunk, ndx, nd, nwx, nwy, ng;  // ndx, nwx, nwy: tiles per row / column; nd, ng: blocks
+  Epi d, g;
+};
+__global__ __launch_bounds__(256) void k_bwd(Bwd p)
+{
+  __shared__ __attribute__((aligned(16))) Tiles S;
+  int i = blockIdx.x;
+  if (i < p.nd) {
+    i = xcd_order(i, p.nd);
+    gemm_tile<false, true, EPI_GELU_GRAD>(S, i % p.ndx, i / p.ndx, 0, p.b, p.win, p.wout, p.wout, p.dz, p.wout, p.w,
+                                          p.wout, p.d, -1);
+  } else {
+    i = xcd_order(i - p.nd, p.ng);
+    const int z = i / (p.nwx * p.nwy), t = i % (p.nwx * p.nwy);
+    gemm_tile<true, false, EPI_F32>(S, t % p.nwx, t / p.nwx, z, p.win + 1, p.wout, p.b, p.kchunk, p.hin, p.win, p.dz,
+                                    p.wout, p.g, p.win);
   }
 }
 
 // rows of the fp32 sets (or of X itself when rows is null) into padded
-// batch buffers: Xb bf16 (b x kin, zero beyond n_in), Yb fp32 (b x nout_p)
-__global__ void k_gather(const float *X, int n_in, const float *Y, int n_out, const int *rows, int b, int kin,
-                         int nout_p, bf16 *Xb, float *Yb)
+// batch buffers: Xb bf16 (b x kin, zero beyond n_in), Yb fp32 (b x nout_p);
+// one wave per row, block blk of 256 threads
+struct Gather {
+  const float *X, *Y;
+  const int *rows;
+  int n_in, n_out, b, kin, nout_p;
+  bf16 *Xb;
+  float *Yb;
+};
+__device__ __forceinline__ void gather_rows(const Gather &q, int blk)
 {
-  const int i = blockIdx.x;
-  if (i >= b) return;
-  const long long src = rows ? rows[i] : i;
-  for (int j = threadIdx.x; j < kin; j += blockDim.x)
-    Xb[(size_t)i * kin + j] = j < n_in ? to_bf16(X[src * n_in + j]) : (bf16)0;
-  if (Yb)
-    for (int j = threadIdx.x; j < nout_p; j += blockDim.x)
-      Yb[(size_t)i * nout_p + j] = j < n_out ? Y[src * n_out + j] : 0.0f;
+  const int i = blk * 4 + (int)(threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (i >= q.b) return;
+  const long long src = q.rows ? q.rows[i] : i;
+  for (int j = l; j < q.kin; j += 64) q.Xb[(size_t)i * q.kin + j] = j < q.n_in ? to_bf16(q.X[src * q.n_in + j]) : (bf16)0;
+  if (q.Yb)
+    for (int j = l; j < q.nout_p; j += 64)
+      q.Yb[(size_t)i * q.nout_p + j] = j < q.n_out ? q.Y[src * q.n_out + j] : 0.0f;
 }
-
-// squared error over the first n_out columns; dZ = bf16(scale (yh - y));
-// one partial sum of squared errors per block
-__global__ __launch_bounds__(256) void k_loss(const float *Yh, const float *Y, int b, int n_out, int ld, float scale,
-                                              bf16 *dZ, float *part)
-{
-  __shared__ float red[256];
-  float s = 0.0f;
-  const long long total = (long long)b * ld;
-  for (long long i = blockIdx.x * 256ll + threadIdx.x; i < total; i += (long long)gridDim.x * 256) {
-    const int col = (int)(i % ld);
-    float g = 0.0f;
-    if (col < n_out) {
-      const float d = Yh[i] - Y[i];
-      s += d * d;
-      g = scale * d;
-    }
-    dZ[i] = to_bf16(g);
-  }
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
+__global__ __launch_bounds__(256) void k_gather(Gather q) { gather_rows(q, blockIdx.x); }
 
 // out[0] = sum(part[0..n-1]) * scale (one block)
-__global__ __launch_bounds__(256) void k_sum(const float *part, int n, float scale, float *out)
+__device__ __forceinline__ void sum_parts(const float *part, int n, float scale, float *out)
 {
   __shared__ float red[256];
   float s = 0.0f;
@@ -302,9 +360,7 @@ __global__ __launch_bounds__(256) void k_sum(const float *part, int n, float sca
   }
   if (threadIdx.x == 0) out[0] = red[0] * scale;
 }
-
-// Adam on the flat parameter vector; wb receives the bf16 copy
-// Split-k slices of the weight gradients that Adam sums itself: layer l's
+// Split-k slices of the weight gradients, summed by their reader: layer l's
 // parameters [woff, woff + welems) take their gradient from nz slices at
 // part + pofs (slice z at + z welems) when nz > 1, else from g
 constexpr int kMaxLayers = 17;  // n_layers <= 16 hidden layers + the output layer
@@ -314,34 +370,126 @@ struct Slices {
   int nz[kMaxLayers];
 };
 
-__global__ void k_adam(float *w, const float *g, float *m, float *v, bf16 *wb, long long n, float lr, float b1,
-                       float b2, float eps, float bc1, float bc2, const float *part, Slices sl)
+// The end of a training step in one launch: Adam in the first na blocks, four
+// parameters per thread (every layer's part starts and ends at a multiple of 64
+// floats), the next step's batch in the blocks after them, and the loss of this
+// step in the last one (13.4 + 5.6 + 4.4 us in launches of their own, 11.2 us
+// together; the parameters, moments and slices are 40 MB).
+struct Step {
+  float *w;
+  const float *g;
+  float *m, *v;
+  bf16 *wb;
+  long long n;
+  float lr, b1, b2, eps, bc1, bc2;
+  const float *part;  // split-k slices
+  int na, ng;         // blocks of Adam and of the gather (0: none)
+  const float *lpart;
+  int nlpart;
+  float lscale;
+  float *loss;
+  Gather next;
+};
+__global__ __launch_bounds__(256) void k_adam(Step p, Slices sl)
 {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x) {
-    float gi = g[i];
-    for (int l = 0; l < sl.nl; ++l) {
-      const long long j = i - sl.woff[l];
-      if (j >= 0 && j < sl.welems[l] && sl.nz[l] > 1) {
-        // the slices in order, as k_sum_slices adds them
-        float a = 0.0f;
-        for (int z = 0; z < sl.nz[l]; ++z) a += part[sl.pofs[l] + z * sl.welems[l] + j];
-        gi = a;
-      }
-    }
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float wi = w[i] - lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
-    w[i] = wi;
-    wb[i] = to_bf16(wi);
+  if ((int)blockIdx.x >= p.na) {
+    const int i = (int)blockIdx.x - p.na;
+    if (i < p.ng) gather_rows(p.next, i);
+    else sum_parts(p.lpart, p.nlpart, p.lscale, p.loss);
+    return;
   }
+  const long long i = 4 * (blockIdx.x * 256ll + threadIdx.x);
+  if (i >= p.n) return;
+  int l = 0;
+  while (l + 1 < sl.nl && i >= sl.woff[l + 1]) ++l;
+  float4 gi;
+  if (sl.nz[l] > 1) {
+    // the slices in order
+    gi = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const float *q = p.part + sl.pofs[l] + (i - sl.woff[l]);
+    const long long step = sl.welems[l];
+    const int nz = sl.nz[l];
+#pragma unroll 8
+    for (int z = 0; z < nz; ++z) {
+      const float4 t = *reinterpret_cast<const float4 *>(q + z * step);
+      gi.x += t.x;
+      gi.y += t.y;
+      gi.z += t.z;
+      gi.w += t.w;
+    }
+  } else {
+    gi = *reinterpret_cast<const float4 *>(p.g + i);
+  }
+  const float4 m4 = *reinterpret_cast<const float4 *>(p.m + i), v4 = *reinterpret_cast<const float4 *>(p.v + i);
+  const float4 w4 = *reinterpret_cast<const float4 *>(p.w + i);
+  float gs[4] = {gi.x, gi.y, gi.z, gi.w}, ms[4] = {m4.x, m4.y, m4.z, m4.w}, vs[4] = {v4.x, v4.y, v4.z, v4.w};
+  float ws[4] = {w4.x, w4.y, w4.z, w4.w};
+  unsigned hb[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    ms[k] = p.b1 * ms[k] + (1.0f - p.b1) * gs[k];
+    vs[k] = p.b2 * vs[k] + (1.0f - p.b2) * gs[k] * gs[k];
+    ws[k] = ws[k] - p.lr * (ms[k] / p.bc1) / (sqrtf(vs[k] / p.bc2) + p.eps);
+    hb[k] = to_bf16(ws[k]);
+  }
+  *reinterpret_cast<float4 *>(p.m + i) = make_float4(ms[0], ms[1], ms[2], ms[3]);
+  *reinterpret_cast<float4 *>(p.v + i) = make_float4(vs[0], vs[1], vs[2], vs[3]);
+  *reinterpret_cast<float4 *>(p.w + i) = make_float4(ws[0], ws[1], ws[2], ws[3]);
+  *reinterpret_cast<uint2 *>(p.wb + i) = make_uint2(hb[0] | (hb[1] << 16), hb[2] | (hb[3] << 16));
 }
 
-__global__ void k_to_bf16(const float *w, bf16 *wb, long long n)
+// The caller's parameter vector (layers' W and b without padding) to the padded
+// device layout with its bf16 copy, or back.  Layer l's entries are fi rows of
+// fo weights and the row of biases, at flat + fofs, on the device rows of fop
+// at woff (fip rows, then the biases); the rest of a padded layer stays zero.
+struct Layers {
+  int nl;
+  int fi[kMaxLayers], fo[kMaxLayers], fip[kMaxLayers], fop[kMaxLayers];
+  long long fofs[kMaxLayers], woff[kMaxLayers];
+};
+__global__ __launch_bounds__(256) void k_set_params(Layers L, const float *__restrict__ flat, float *w, bf16 *wb,
+                                                    float *m, float *v)
 {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
-    wb[i] = to_bf16(w[i]);
+  const int l = blockIdx.y;
+  const int fop = L.fop[l];
+  const int n = (L.fip[l] + 1) * fop;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+    const int r = i / fop, c = i - r * fop;
+    const int src = r < L.fi[l] ? r : r == L.fip[l] ? L.fi[l] : -1;  // the biases follow the padded rows
+    const float x = src >= 0 && c < L.fo[l] ? flat[L.fofs[l] + (long long)src * L.fo[l] + c] : 0.0f;
+    const long long o = L.woff[l] + i;
+    w[o] = x;
+    wb[o] = to_bf16(x);
+    m[o] = 0.0f;
+    v[o] = 0.0f;
+  }
+}
+// sl (or null): the gradient instead, layers split over k as the sum of their
+// slices in order; the last block then sums the loss
+__global__ __launch_bounds__(256) void k_get_params(Layers L, const float *__restrict__ w, float *__restrict__ flat,
+                                                    int grad, Slices sl, const float *__restrict__ part,
+                                                    const float *lpart, int nlpart, float lscale, float *loss)
+{
+  const int l = blockIdx.y;
+  if (l == L.nl) {
+    if (blockIdx.x == 0) sum_parts(lpart, nlpart, lscale, loss);
+    return;
+  }
+  const int fo = L.fo[l], n = (L.fi[l] + 1) * fo;
+  const int nz = grad ? sl.nz[l] : 1;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+    const int r = i / fo, c = i - r * fo;
+    const long long j = (long long)(r < L.fi[l] ? r : L.fip[l]) * L.fop[l] + c;
+    float x;
+    if (nz > 1) {
+      x = 0.0f;
+#pragma unroll 8
+      for (int z = 0; z < nz; ++z) x += part[sl.pofs[l] + z * sl.welems[l] + j];
+    } else {
+      x = w[L.woff[l] + j];
+    }
+    flat[L.fofs[l] + i] = x;
+  }
 }
 
 }  // namespace ss
@@ -399,13 +547,15 @@ struct sedsurr_handle {
   bf16 *xb = nullptr;                   // max_batch x kin
   std::vector<bf16 *> hs;               // hidden activations, max_batch x n_hidden
   std::vector<float *> zs;              // pre-activations
-  float *yh = nullptr, *yb = nullptr;   // max_batch x nout_p
+  float *yb = nullptr;                  // max_batch x nout_p
   bf16 *dz0 = nullptr, *dz1 = nullptr;  // max_batch x max(n_hidden, nout_p)
-  float *part = nullptr;                // loss partial sums
-  float *kpart = nullptr;               // split-k partial weight gradients
-  float *kpart_all = nullptr;           // the same, one region per layer (training: summed by Adam)
+  float *part = nullptr;                // squared errors per block, then the loss of sedsurr_loss_grad
+  float *kpart_all = nullptr;           // split-k partial weight gradients, one region per layer
   std::vector<long long> kpofs;         // offset of layer l's region in kpart_all
-  ss::Slices slices{};                  // the last training step's deferred slices
+  ss::Slices slices{};                  // the slices of the last backward pass
+  ss::Layers layers{};                  // padded and caller's layouts of the parameters
+  float *flat = nullptr;                // np: parameters or gradient in the caller's layout
+  float *h_loss = nullptr;              // pinned: the loss of sedsurr_loss_grad
   float *loss = nullptr;                // per-step losses of a train call
   int loss_cap = 0;
   float *X = nullptr, *Y = nullptr;     // training set
@@ -424,20 +574,15 @@ struct sedsurr_handle {
 
 namespace {
 
-constexpr int kLossBlocks = 256;
-
 constexpr int kMaxSplit = 8;     // k slices of a weight-gradient product
+constexpr int kParamBlocks = 256;  // blocks per layer of the parameter copies
 
-template <bool TA, bool TB, int EPI>
+template <int EPI>
 void gemm(sedsurr_handle *h, int M, int N, int K, const bf16 *A, int lda, const bf16 *B, int ldb, ss::Epi e,
-          int *launches, int split = 1, int ones_row = -1)
+          int *launches)
 {
-  const int kchunk = (K + split - 1) / split;
-  const int kc = (kchunk + ss::BK - 1) / ss::BK * ss::BK;
-  const int nz = (K + kc - 1) / kc;
-  dim3 grid((N + ss::BN - 1) / ss::BN, (M + ss::BM - 1) / ss::BM, nz > 0 ? nz : 1);
-  hipLaunchKernelGGL((ss::k_gemm<TA, TB, EPI>), grid, dim3(256), 0, h->st, M, N, K, kc, A, lda, B, ldb, e,
-                     ones_row);
+  dim3 grid((N + ss::BN - 1) / ss::BN, (M + ss::BM - 1) / ss::BM);
+  hipLaunchKernelGGL(ss::k_gemm<EPI>, grid, dim3(256), 0, h->st, M, N, K, A, lda, B, ldb, e);
   ++*launches;
 }
 
@@ -454,8 +599,14 @@ int split_for(int M, int N, int b)
 // width of the activation entering layer l (padded)
 inline int in_width(const sedsurr_handle *h, int l) { return h->fip[l]; }
 
-// forward pass of b rows from h->xb; output h->yh (b x nout_p), or, with
-// out, the n_out real columns only, compact (b x n_out)
+inline int tiles(int n, int t) { return (n + t - 1) / t; }
+
+// blocks of the output layer's product for b rows, each with a partial loss
+inline int loss_parts(const sedsurr_handle *h, int b) { return tiles(b, ss::BM) * tiles(h->nout_p, ss::BN); }
+
+// forward pass of b rows from h->xb; the n_out real columns, compact, to out,
+// or, without out, the loss against h->yb: squared errors per block to h->part
+// and dZ of the output layer to h->dz0
 void forward(sedsurr_handle *h, int b, int *launches, float *out = nullptr)
 {
   const int L = h->nl;
@@ -463,39 +614,37 @@ void forward(sedsurr_handle *h, int b, int *launches, float *out = nullptr)
     const bf16 *A = l == 0 ? h->xb : h->hs[l - 1];
     const int lda = in_width(h, l);
     ss::Epi e{};
+    e.bias = h->w + h->boff[l];
     if (l < L - 1) {
       e.out_f = h->zs[l];
       e.ldo = h->fop[l];
       e.out_h = h->hs[l];
       e.ldh = h->fop[l];
-      e.bias = h->w + h->boff[l];
-      gemm<false, false, ss::EPI_BIAS_GELU>(h, b, h->fop[l], h->fip[l], A, lda, h->wb + h->woff[l], h->fop[l], e,
+      gemm<ss::EPI_BIAS_GELU>(h, b, h->fop[l], h->fip[l], A, lda, h->wb + h->woff[l], h->fop[l], e,
                                             launches);
+    } else if (out) {
+      e.out_f = out;
+      e.ldo = h->s.n_out;
+      gemm<ss::EPI_BIAS>(h, b, h->s.n_out, h->fip[l], A, lda, h->wb + h->woff[l], h->fop[l], e, launches);
     } else {
-      e.out_f = out ? out : h->yh;
-      e.ldo = out ? h->s.n_out : h->nout_p;
-      e.bias = h->w + h->boff[l];
-      gemm<false, false, ss::EPI_BIAS>(h, b, out ? h->s.n_out : h->fop[l], h->fip[l], A, lda, h->wb + h->woff[l],
-                                       h->fop[l], e, launches);
+      e.out_f = h->part;
+      e.out_h = h->dz0;
+      e.ldh = h->nout_p;
+      e.zin = h->yb;
+      e.ldz = h->nout_p;
+      e.scale = 2.0f / ((float)b * (float)h->s.n_out);
+      e.n_out = h->s.n_out;
+      gemm<ss::EPI_LOSS>(h, b, h->nout_p, h->fip[l], A, lda, h->wb + h->woff[l], h->fop[l], e, launches);
     }
   }
 }
 
-// loss of the forward output against h->yb, gradient into h->g; loss value
-// to *loss_dev.  defer: split weight gradients stay as slices in
-// h->kpart_all (described in h->slices) for k_adam to sum
-void loss_backward(sedsurr_handle *h, int b, float *loss_dev, int *launches, bool defer = false)
+// gradient of the loss of forward(): into h->g, or as slices in h->kpart_all
+// for the layers whose product over the batch is split (h->slices)
+void backward(sedsurr_handle *h, int b, int *launches)
 {
-  const int L = h->nl;
-  const float scale = 2.0f / ((float)b * (float)h->s.n_out);
-  hipLaunchKernelGGL(ss::k_loss, dim3(kLossBlocks), dim3(256), 0, h->st, h->yh, h->yb, b, h->s.n_out, h->nout_p,
-                     scale, h->dz0, h->part);
-  hipLaunchKernelGGL(ss::k_sum, dim3(1), dim3(256), 0, h->st, h->part, kLossBlocks,
-                     1.0f / ((float)b * (float)h->s.n_out), loss_dev);
-  *launches += 2;
   bf16 *dz = h->dz0, *dzn = h->dz1;
-  for (int l = L - 1; l >= 0; --l) {
-    const bf16 *Hin = l == 0 ? h->xb : h->hs[l - 1];
+  for (int l = h->nl - 1; l >= 0; --l) {
     const int win = in_width(h, l), wout = h->fop[l];
     // [dW_l; db_l] = [H_in, 1]^T dZ_l in one product: the bias gradient
     // (the column sums of dZ_l) is the row of a ones column appended to
@@ -505,54 +654,46 @@ void loss_backward(sedsurr_handle *h, int b, float *loss_dev, int *launches, boo
     const long long welems = (long long)(win + 1) * wout;
     const int kc = ((b + split - 1) / split + ss::BK - 1) / ss::BK * ss::BK;
     const int nz = (b + kc - 1) / kc;
-    float *part = defer ? h->kpart_all + h->kpofs[l] : h->kpart;
-    ss::Epi e{};
-    e.out_f = nz > 1 ? part : h->g + h->woff[l];
-    e.ldo = wout;
-    e.zstride = welems;
-    gemm<true, false, ss::EPI_F32>(h, win + 1, wout, b, Hin, win, dz, wout, e, launches, split, win);
+    ss::Bwd p{};
+    p.dz = dz;
+    p.w = h->wb + h->woff[l];
+    p.hin = l == 0 ? h->xb : h->hs[l - 1];
+    p.b = b;
+    p.win = win;
+    p.wout = wout;
+    p.kchunk = kc;
+    p.ndx = tiles(win, ss::BN);
+    p.nd = l > 0 ? p.ndx * tiles(b, ss::BM) : 0;  // the input needs no gradient
+    p.nwx = tiles(wout, ss::BN);
+    p.nwy = tiles(win + 1, ss::BM);
+    p.ng = p.nwx * p.nwy * nz;
+    // dZ_{l-1} = GELU'(Z_{l-1}) * (dZ_l W_l^T)
+    p.d.out_h = dzn;
+    p.d.ldh = win;
+    p.d.zin = l > 0 ? h->zs[l - 1] : nullptr;
+    p.d.ldz = win;
+    p.g.out_f = nz > 1 ? h->kpart_all + h->kpofs[l] : h->g + h->woff[l];
+    p.g.ldo = wout;
+    p.g.zstride = welems;
+    hipLaunchKernelGGL(ss::k_bwd, dim3(p.nd + p.ng), dim3(256), 0, h->st, p);
+    ++*launches;
     h->slices.woff[l] = h->woff[l];
     h->slices.welems[l] = welems;
     h->slices.pofs[l] = h->kpofs[l];
-    h->slices.nz[l] = defer ? nz : 1;
-    if (nz > 1 && !defer) {
-      hipLaunchKernelGGL(ss::k_sum_slices, dim3(512), dim3(256), 0, h->st, h->kpart, nz, welems, welems,
-                         h->g + h->woff[l]);
-      ++*launches;
-    }
-    if (l > 0) {
-      // dZ_{l-1} = GELU'(Z_{l-1}) * (dZ_l W_l^T)
-      ss::Epi d{};
-      d.out_h = dzn;
-      d.ldh = win;
-      d.zin = h->zs[l - 1];
-      d.ldz = win;
-      gemm<false, true, ss::EPI_GELU_GRAD>(h, b, win, wout, dz, wout, h->wb + h->woff[l], wout, d, launches);
-      std::swap(dz, dzn);
-    }
+    h->slices.nz[l] = nz;
+    std::swap(dz, dzn);
   }
 }
 
-// host logical flat vector <-> padded device layout
-void pad_params(const sedsurr_handle *h, const float *src, std::vector<float> &dst)
+ss::Gather gather_of(const sedsurr_handle *h, const float *X, const float *Y, const int *rows, int b)
 {
-  dst.assign(h->np_pad, 0.0f);
-  long long o = 0;
-  for (int l = 0; l < h->nl; ++l) {
-    for (int i = 0; i < h->fi[l]; ++i)
-      for (int j = 0; j < h->fo[l]; ++j) dst[h->woff[l] + (long long)i * h->fop[l] + j] = src[o++];
-    for (int j = 0; j < h->fo[l]; ++j) dst[h->boff[l] + j] = src[o++];
-  }
+  return ss::Gather{X, Y, rows, h->s.n_in, h->s.n_out, b, h->kin, h->nout_p, h->xb, Y ? h->yb : nullptr};
 }
 
-void unpad_params(const sedsurr_handle *h, const std::vector<float> &src, float *dst)
+void gather(sedsurr_handle *h, const ss::Gather &q, int *launches)
 {
-  long long o = 0;
-  for (int l = 0; l < h->nl; ++l) {
-    for (int i = 0; i < h->fi[l]; ++i)
-      for (int j = 0; j < h->fo[l]; ++j) dst[o++] = src[h->woff[l] + (long long)i * h->fop[l] + j];
-    for (int j = 0; j < h->fo[l]; ++j) dst[o++] = src[h->boff[l] + j];
-  }
+  hipLaunchKernelGGL(ss::k_gather, dim3((q.b + 3) / 4), dim3(256), 0, h->st, q);
+  ++*launches;
 }
 
 }  // namespace
@@ -625,14 +766,12 @@ int sedsurr_create(const sedsurr_shape *shape, sedsurr_handle **out)
     h->zs.push_back(zb);
   }
   const size_t wmax = (size_t)std::max(s.n_hidden, h->nout_p);
-  HIPOK_C(hipMalloc(&h->yh, sizeof(float) * B * h->nout_p));
   HIPOK_C(hipMalloc(&h->yb, sizeof(float) * B * h->nout_p));
   HIPOK_C(hipMalloc(&h->dz0, sizeof(bf16) * B * wmax));
   HIPOK_C(hipMalloc(&h->dz1, sizeof(bf16) * B * wmax));
-  HIPOK_C(hipMalloc(&h->part, sizeof(float) * (kLossBlocks + 1)));  // + the loss of sedsurr_loss_grad
-  long long wmax_el = 0;
-  for (int l = 0; l < h->nl; ++l) wmax_el = std::max(wmax_el, (long long)(h->fip[l] + 1) * h->fop[l]);
-  HIPOK_C(hipMalloc(&h->kpart, sizeof(float) * kMaxSplit * wmax_el));
+  HIPOK_C(hipMalloc(&h->part, sizeof(float) * (loss_parts(h, s.max_batch) + 1)));  // + the loss of sedsurr_loss_grad
+  HIPOK_C(hipMalloc(&h->flat, sizeof(float) * (size_t)h->np));
+  HIPOK_C(hipHostMalloc((void **)&h->h_loss, sizeof(float), hipHostMallocDefault));
   if (h->nl > ss::kMaxLayers) return cleanup(fail(SEDCOL_EINVAL, "too many layers"));
   long long kall = 0;
   for (int l = 0; l < h->nl; ++l) {
@@ -641,6 +780,17 @@ int sedsurr_create(const sedsurr_shape *shape, sedsurr_handle **out)
   }
   HIPOK_C(hipMalloc(&h->kpart_all, sizeof(float) * kall));
   h->slices.nl = h->nl;
+  h->layers.nl = h->nl;
+  long long fofs = 0;
+  for (int l = 0; l < h->nl; ++l) {
+    h->layers.fi[l] = h->fi[l];
+    h->layers.fo[l] = h->fo[l];
+    h->layers.fip[l] = h->fip[l];
+    h->layers.fop[l] = h->fop[l];
+    h->layers.woff[l] = h->woff[l];
+    h->layers.fofs[l] = fofs;
+    fofs += (long long)(h->fi[l] + 1) * h->fo[l];
+  }
   HIPOK_C(hipMalloc(&h->xin, sizeof(float) * B * s.n_in));
   HIPOK_C(hipMalloc(&h->yin, sizeof(float) * B * s.n_out));
 #undef HIPOK_C
@@ -653,13 +803,14 @@ int sedsurr_destroy(sedsurr_handle *h)
   if (!h) return SEDCOL_OK;
   const DeviceScope dscope(h->device);
   if (h->st) (void)hipStreamSynchronize(h->st);
-  std::vector<void *> ptrs = {h->w, h->g, h->m, h->v, h->wb, h->xb, h->yh, h->yb, h->dz0, h->dz1,
-                              h->part, h->loss, h->X, h->Y, h->rows, h->xin, h->yin, h->kpart, h->kpart_all,
-                              h->ydev};
+  std::vector<void *> ptrs = {h->w, h->g, h->m, h->v, h->wb, h->xb, h->yb, h->dz0, h->dz1,
+                              h->part, h->loss, h->X, h->Y, h->rows, h->xin, h->yin, h->kpart_all,
+                              h->ydev, h->flat};
   for (auto *q : h->hs) ptrs.push_back(q);
   for (auto *q : h->zs) ptrs.push_back(q);
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
+  if (h->h_loss) (void)hipHostFree(h->h_loss);
   if (h->e0) (void)hipEventDestroy(h->e0);
   if (h->e1) (void)hipEventDestroy(h->e1);
   if (h->st) (void)hipStreamDestroy(h->st);
@@ -681,13 +832,9 @@ int sedsurr_set_params(sedsurr_handle *h, const float *params)
   const DeviceScope dscope(h->device);
   for (long long i = 0; i < h->np; ++i)
     if (!std::isfinite(params[i])) return fail(SEDCOL_EDOMAIN, "non-finite parameter");
-  std::vector<float> buf;
-  pad_params(h, params, buf);
-  const size_t P = (size_t)h->np_pad;
-  HIPOK(hipMemcpyAsync(h->w, buf.data(), sizeof(float) * P, hipMemcpyHostToDevice, h->st));
-  HIPOK(hipMemsetAsync(h->m, 0, sizeof(float) * P, h->st));
-  HIPOK(hipMemsetAsync(h->v, 0, sizeof(float) * P, h->st));
-  hipLaunchKernelGGL(ss::k_to_bf16, dim3(1024), dim3(256), 0, h->st, h->w, h->wb, (long long)P);
+  HIPOK(hipMemcpyAsync(h->flat, params, sizeof(float) * (size_t)h->np, hipMemcpyHostToDevice, h->st));
+  hipLaunchKernelGGL(ss::k_set_params, dim3(kParamBlocks, h->nl), dim3(256), 0, h->st, h->layers, h->flat, h->w, h->wb,
+                     h->m, h->v);
   HIPOK(hipGetLastError());
   HIPOK(hipStreamSynchronize(h->st));
   h->step = 0;
@@ -698,10 +845,11 @@ int sedsurr_get_params(sedsurr_handle *h, float *params)
 {
   if (!h || !params) return fail(SEDCOL_EINVAL, "null argument");
   const DeviceScope dscope(h->device);
-  std::vector<float> buf(h->np_pad);
-  HIPOK(hipMemcpyAsync(buf.data(), h->w, sizeof(float) * h->np_pad, hipMemcpyDeviceToHost, h->st));
+  hipLaunchKernelGGL(ss::k_get_params, dim3(kParamBlocks, h->nl), dim3(256), 0, h->st, h->layers, h->w, h->flat, 0,
+                     h->slices, (const float *)nullptr, (const float *)nullptr, 0, 0.0f, (float *)nullptr);
+  HIPOK(hipGetLastError());
+  HIPOK(hipMemcpyAsync(params, h->flat, sizeof(float) * (size_t)h->np, hipMemcpyDeviceToHost, h->st));
   HIPOK(hipStreamSynchronize(h->st));
-  unpad_params(h, buf, params);
   return SEDCOL_OK;
 }
 
@@ -754,17 +902,33 @@ int sedsurr_train(sedsurr_handle *h, int32_t steps, int32_t batch, const int32_t
   HIPOK(hipMemcpyAsync(h->rows, rows, sizeof(int) * nr, hipMemcpyHostToDevice, h->st));
   int launches = 0;
   HIPOK(hipEventRecord(h->e0, h->st));
+  gather(h, gather_of(h, h->X, h->Y, h->rows, batch), &launches);
   for (int s = 0; s < steps; ++s) {
-    hipLaunchKernelGGL(ss::k_gather, dim3(batch), dim3(64), 0, h->st, h->X, h->s.n_in, h->Y, h->s.n_out,
-                       h->rows + (long long)s * batch, batch, h->kin, h->nout_p, h->xb, h->yb);
-    ++launches;
     forward(h, batch, &launches);
-    loss_backward(h, batch, h->loss + s, &launches, true);
+    backward(h, batch, &launches);
     ++h->step;
-    const float bc1 = 1.0f - std::pow(adam->beta1, (float)h->step);
-    const float bc2 = 1.0f - std::pow(adam->beta2, (float)h->step);
-    hipLaunchKernelGGL(ss::k_adam, dim3(1024), dim3(256), 0, h->st, h->w, h->g, h->m, h->v, h->wb, h->np_pad,
-                       adam->lr, adam->beta1, adam->beta2, adam->eps, bc1, bc2, h->kpart_all, h->slices);
+    ss::Step p{};
+    p.w = h->w;
+    p.g = h->g;
+    p.m = h->m;
+    p.v = h->v;
+    p.wb = h->wb;
+    p.n = h->np_pad;
+    p.lr = adam->lr;
+    p.b1 = adam->beta1;
+    p.b2 = adam->beta2;
+    p.eps = adam->eps;
+    p.bc1 = 1.0f - std::pow(adam->beta1, (float)h->step);
+    p.bc2 = 1.0f - std::pow(adam->beta2, (float)h->step);
+    p.part = h->kpart_all;
+    p.na = (int)((h->np_pad / 4 + 255) / 256);
+    p.ng = s + 1 < steps ? (batch + 3) / 4 : 0;
+    p.lpart = h->part;
+    p.nlpart = loss_parts(h, batch);
+    p.lscale = 1.0f / ((float)batch * (float)h->s.n_out);
+    p.loss = h->loss + s;
+    if (p.ng) p.next = gather_of(h, h->X, h->Y, h->rows + (long long)(s + 1) * batch, batch);
+    hipLaunchKernelGGL(ss::k_adam, dim3(p.na + p.ng + 1), dim3(256), 0, h->st, p, h->slices);
     ++launches;
   }
   HIPOK(hipGetLastError());
@@ -789,16 +953,19 @@ int sedsurr_loss_grad(sedsurr_handle *h, const float *X, const float *Y, int32_t
   HIPOK(hipMemcpyAsync(h->xin, X, sizeof(float) * (size_t)n * h->s.n_in, hipMemcpyHostToDevice, h->st));
   HIPOK(hipMemcpyAsync(h->yin, Y, sizeof(float) * (size_t)n * h->s.n_out, hipMemcpyHostToDevice, h->st));
   int launches = 0;
-  hipLaunchKernelGGL(ss::k_gather, dim3(n), dim3(64), 0, h->st, h->xin, h->s.n_in, h->yin, h->s.n_out,
-                     (const int *)nullptr, n, h->kin, h->nout_p, h->xb, h->yb);
+  gather(h, gather_of(h, h->xin, h->yin, nullptr, n), &launches);
   forward(h, n, &launches);
-  loss_backward(h, n, h->part + kLossBlocks, &launches);
+  backward(h, n, &launches);
+  const int np = loss_parts(h, n);
+  float *loss_dev = h->part + np;
+  // the gradient straight into the caller's layout, slices summed on the way
+  hipLaunchKernelGGL(ss::k_get_params, dim3(kParamBlocks, h->nl + 1), dim3(256), 0, h->st, h->layers, h->g, h->flat, 1,
+                     h->slices, h->kpart_all, h->part, np, 1.0f / ((float)n * (float)h->s.n_out), loss_dev);
   HIPOK(hipGetLastError());
-  std::vector<float> buf(h->np_pad);
-  HIPOK(hipMemcpyAsync(buf.data(), h->g, sizeof(float) * h->np_pad, hipMemcpyDeviceToHost, h->st));
-  HIPOK(hipMemcpyAsync(loss, h->part + kLossBlocks, sizeof(float), hipMemcpyDeviceToHost, h->st));
+  HIPOK(hipMemcpyAsync(h->h_loss, loss_dev, sizeof(float), hipMemcpyDeviceToHost, h->st));
+  HIPOK(hipMemcpyAsync(grad, h->flat, sizeof(float) * (size_t)h->np, hipMemcpyDeviceToHost, h->st));
   HIPOK(hipStreamSynchronize(h->st));
-  unpad_params(h, buf, grad);
+  *loss = *h->h_loss;
   return SEDCOL_OK;
 }
 
@@ -813,9 +980,7 @@ static int predict_rows(sedsurr_handle *h, const float *X, int64_t n, float *Y, 
     const int b = (int)std::min<int64_t>(B, n - r0);
     HIPOK(hipMemcpyAsync(h->xin, X + r0 * h->s.n_in, sizeof(float) * (size_t)b * h->s.n_in, hipMemcpyHostToDevice,
                          h->st));
-    hipLaunchKernelGGL(ss::k_gather, dim3(b), dim3(64), 0, h->st, h->xin, h->s.n_in, (const float *)nullptr, no,
-                       (const int *)nullptr, b, h->kin, h->nout_p, h->xb, (float *)nullptr);
-    ++launches;
+    gather(h, gather_of(h, h->xin, nullptr, nullptr, b), &launches);
     // compact b x n_out output, in place on the device or staged for the host
     forward(h, b, &launches, y_on_device ? Y + r0 * no : h->yb);
     HIPOK(hipGetLastError());
