@@ -487,8 +487,8 @@ int ensure_scratch(sedcol_handle *h)
 
 // The caller's state arrays go to and from the device as they are, without a
 // copy in host memory: packed ones directly, Fortran ones through d_scr and
-// k_layout.  (A packed copy first, or the transposition on the host, took 59
-// of the 62 ms of setting and 63 of the 76 ms of reading 238 MB.)
+// k_layout.  (With the transposition on the host and pageable copies, setting
+// 238 MB took 59 ms and reading them 76 ms.)
 //
 // Large copies go through pinned blocks that several threads fill or empty: the
 // link takes pinned memory at 55 GB/s, where one thread of the runtime moves
@@ -1513,8 +1513,8 @@ int sedcol_autotune(sedcol_handle *h, double t_start, double t_span, int32_t rep
 
 // One fixed step of a small domain (h_stage): the state goes through pinned
 // memory that the kernels read and write in place, so the call queues its
-// launches and waits once.  (Copies of their own, each with its wait, took 80
-// of the 104 us of an RK4 step of 16 columns.)
+// launches and waits once.  (With copies of their own, each with its wait, an
+// RK4 step of 16 columns took 104 us, so 43.)
 static int step_small(sedcol_handle *h, double dt, int method, double *conc, double *flux_top_out)
 {
   const size_t cells = NV * (size_t)h->ncell, fl = NV * (size_t)h->ncol;

@@ -652,9 +652,10 @@ __device__ __forceinline__ bool state_ok(const double (&c)[NV])
   return e > kStateLo && m < 0x1p500;
 }
 
-// One get_rhs evaluation for the lane's layer.  sbc[0..NV) bottom-water
-// concentrations, sbc[NV..2NV) top fluxes (LDS, per group; load_forcing puts
-// 0 for a closed top).
+// One get_rhs evaluation for the lane's layer.  sbc[n] is the bottom-water
+// concentration of variable n, sbc[TF + n] its top flux (0 for a closed top):
+// TF = NV in a group's LDS slot, TF = 0 with the one of the two that the
+// boundary condition uses (the flux computed from a given flux is not used).
 // For each variable n the callback receives (n, rhs_n, F) where F is the flux
 // through the lane's upper interface (lane 0: the top flux intFlux(:,:,1)).
 // Transport: diff3d (fabm_sediment_driver.F90:739-825) with the particulate
@@ -664,7 +665,7 @@ __device__ __forceinline__ bool state_ok(const double (&c)[NV])
 // the same expression as the interior's against the bottom water: a select,
 // so that the evaluation is one stretch of code over all variables.
 // FD: divisions by reciprocals (reference form).
-template <int LPC, int ARITH, bool FD, class CB>
+template <int LPC, int ARITH, int TF, bool FD, class CB>
 __device__ __forceinline__ void column_terms(const sedcol_params &p, const Lane &L, const double *sbc,
                                              const double (&c)[NV], double &sC, double &sN, CB &&cb, const ZwDev *zw)
 {
@@ -700,13 +701,13 @@ __device__ __forceinline__ void column_terms(const sedcol_params &p, const Lane 
       const double D = pt ? Dbio : Ddis;
       const double num = D * (x - xo);
       const double Fd = -(FD ? div_by(num, L.dzc, L.ydzc) : num / L.dzc);
-      F = (pt ? givenp : givend) ? sbc[NV + n] : Fd;
+      F = (pt ? givenp : givend) ? sbc[TF + n] : Fd;
       if (ARITH == ARITH_EXT && pt && p.bcup_part == 4) {
         // diff3d BcUp = 4 (fabm_sediment_driver.F90:791-802): the top flux
         // beyond the first layer's cap is added to the interfaces below,
         // each layer's cap taken off in turn, sequentially as written there;
         // every lane of the group runs the same loop on broadcast caps
-        double rest = sbc[NV + n] - __shfl(L.cap, 0, LPC);
+        double rest = sbc[TF + n] - __shfl(L.cap, 0, LPC);
         bool running = true;  // every check so far passed
 #pragma unroll 1
         for (int k = 1; k < LPC; ++k) {
@@ -734,7 +735,7 @@ __device__ __forceinline__ void column_terms(const sedcol_params &p, const Lane 
     } else {
       const double G = pt ? L.Gb : L.Gd;
       const double Fd = -(G * (x - xo));
-      F = (pt ? givenp : givend) ? sbc[NV + n] : Fd;
+      F = (pt ? givenp : givend) ? sbc[TF + n] : Fd;
       // the lane exchange runs on every lane (a lane outside the exec mask
       // reads as 0 to the lane above it), then the bottom value replaces it;
       // written as a select on lg_dn's result it would only be evaluated
@@ -747,7 +748,7 @@ __device__ __forceinline__ void column_terms(const sedcol_params &p, const Lane 
   }
 }
 
-template <int LPC, int ARITH, class CB>
+template <int LPC, int ARITH, int TF = NV, class CB>
 __device__ __forceinline__ void column_rhs(const sedcol_params &p, const Lane &L, const double *sbc,
                                            const double (&c)[NV], double &sC, double &sN, CB &&cb,
                                            const ZwDev *zw = nullptr)
@@ -756,10 +757,10 @@ __device__ __forceinline__ void column_rhs(const sedcol_params &p, const Lane &L
   // wave barriers keep those accesses ordered around the evaluation.
   __builtin_amdgcn_wave_barrier();
   if constexpr (ARITH == ARITH_REF) {
-    if (__any(L.active && (L.wide || !state_ok(c)))) column_terms<LPC, ARITH, false>(p, L, sbc, c, sC, sN, cb, zw);
-    else column_terms<LPC, ARITH, true>(p, L, sbc, c, sC, sN, cb, zw);
+    if (__any(L.active && (L.wide || !state_ok(c)))) column_terms<LPC, ARITH, TF, false>(p, L, sbc, c, sC, sN, cb, zw);
+    else column_terms<LPC, ARITH, TF, true>(p, L, sbc, c, sC, sN, cb, zw);
   } else {
-    column_terms<LPC, ARITH, false>(p, L, sbc, c, sC, sN, cb, zw);
+    column_terms<LPC, ARITH, TF, false>(p, L, sbc, c, sC, sN, cb, zw);
   }
   __builtin_amdgcn_wave_barrier();
 }
@@ -866,12 +867,9 @@ __device__ __forceinline__ double psolve(const double (&c)[NV], const double (&g
 // (b_j + d) s, s = 1/(qmin + d0) <= 1, are multiplied with their
 // derivative; L and dL/dw = d sum 1/(b_j + d) come from one log and one
 // division per lane.
-// The b_j live in LDS (bs[j * RS], the lane's slots): they are read once per
-// iteration and would otherwise hold 22 VGPRs through the loop.
-template <int LPC, bool STAGE2, int RS>
+template <int LPC, bool STAGE2>
 __device__ __forceinline__ double psolve_geo(const double (&c)[NV], const double (&g)[NV], const double (&den)[NV],
-                                             double h, bool active, int64_t &zero_sink, int64_t &newton,
-                                             double *bs)
+                                             double h, bool active, int64_t &zero_sink, int64_t &newton)
 {
   double b[NV];
   double Sl = 1.0, nl = 0.0, am = 0.0;
@@ -895,20 +893,17 @@ __device__ __forceinline__ double psolve_geo(const double (&c)[NV], const double
   const double lnS = STAGE2 ? lg_sum<LPC>(active ? dlog(Sl) : 0.0) : 0.0;
   const double qmin = lg_max<LPC>(am);
 #pragma unroll
-  for (int n = 0; n < NV; ++n) bs[n * RS] = b[n] > 0.0 ? -1.0 : qmin + b[n];  // b < 0: not destroyed
+  for (int n = 0; n < NV; ++n) b[n] = b[n] > 0.0 ? -1.0 : qmin + b[n];  // b < 0: not destroyed
   double d = STAGE2 ? dexp((0.0 - lnS) / N) : 1.0;
   const double sc = 1.0 / (qmin + d);
   const double lsc = dlog(sc);
   for (int it = 0; it < 60; ++it) {
     newton += 1;
-    // the slots are re-read in every iteration, not held in registers
-    __asm__ volatile("" ::: "memory");
     double P = 1.0, D = 0.0;
 #pragma unroll
     for (int n = 0; n < NV; ++n) {
-      const double bn = bs[n * RS];
-      const bool on = bn >= 0.0;
-      const double f = on ? (bn + d) * sc : 1.0;
+      const bool on = b[n] >= 0.0;
+      const double f = on ? (b[n] + d) * sc : 1.0;
       D = fma(D, f, on ? P * sc : 0.0);
       P = P * f;
     }
@@ -931,11 +926,11 @@ __device__ __forceinline__ double psolve_geo(const double (&c)[NV], const double
 // The Patankar factor of a weighting (sedcol_params.emp_weights), fixed per
 // kernel instance: PW = 0 the product over the destroyed components, PW = 1
 // their geometric mean.
-template <int LPC, bool STAGE2, int PW, int RS>
+template <int LPC, bool STAGE2, int PW>
 __device__ __forceinline__ double pfactor(const double (&c)[NV], const double (&g)[NV], const double (&den)[NV],
-                                          double h, bool active, int64_t &zero_sink, int64_t &newton, double *bs)
+                                          double h, bool active, int64_t &zero_sink, int64_t &newton)
 {
-  if constexpr (PW == 1) return psolve_geo<LPC, STAGE2, RS>(c, g, den, h, active, zero_sink, newton, bs);
+  if constexpr (PW == 1) return psolve_geo<LPC, STAGE2>(c, g, den, h, active, zero_sink, newton);
   else return psolve<LPC, STAGE2>(c, g, den, h, active, zero_sink, newton);
 }
 

@@ -89,6 +89,14 @@ __device__ __forceinline__ void load_forcing(const Dev &d, const sedcol_params &
   }
 }
 
+// The boundary values of a group's slot in registers: of each variable the one
+// that its boundary condition uses (column_terms with TF = 0).
+__device__ __forceinline__ void take_top(const sedcol_params &p, const double *sbc, double (&bc)[NV])
+{
+#pragma unroll
+  for (int n = 0; n < NV; ++n) bc[n] = sbc[(part(n) ? p.bcup_part : p.bcup_dis) != 2 ? NV + n : n];
+}
+
 // top fluxes of one right-hand side, held by the group's first lane, into the
 // group's LDS slot: one branch for all variables
 __device__ __forceinline__ void store_top(bool first, const double (&Ft)[NV], double *F)
@@ -148,8 +156,6 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
   constexpr int G = BLOCK / LPC;
   __shared__ double sbc[G][2 * NV];
   __shared__ double sF[G][4][NV];
-  // coefficients of the geometric-mean Patankar solve (one slot otherwise)
-  __shared__ double sgeo[PW == 1 ? NV : 1][BLOCK];
   const int g = threadIdx.x / LPC, l = threadIdx.x % LPC;
   const int slot = blockIdx.x * G + g;
   const bool valid = slot < nlist;
@@ -165,9 +171,8 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
   if (!valid) return;
   // the boundary values stay in registers for the whole run: read from LDS in
   // every right-hand side, they cost a lone wave 1600 of 4900 cycles
-  double bc[2 * NV];
-#pragma unroll
-  for (int n = 0; n < 2 * NV; ++n) bc[n] = sbc[g][n];
+  double bc[NV];
+  take_top(p, sbc[g], bc);
   double(*F)[NV] = sF[g];
   const bool act = L.active;
   const bool own = l < NV;  // lane l accumulates the top flux of variable l
@@ -192,7 +197,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
     double sC, sN, Ft[NV];
     if (METHOD == SEDCOL_EULER) {
       double r0[NV];
-      column_rhs<LPC, ARITH>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, 0>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
         r0[n] = r;
         Ft[n] = Fv;
       }, &d.zw);
@@ -209,7 +214,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       // solver_library.F90:142-163
       double cs[NV], k[NV];
       double aC, aN;
-      column_rhs<LPC, ARITH>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, 0>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
         k[n] = 0.5 * r;
         cs[n] = x[n] + (0.5 * dt) * r;
         Ft[n] = Fv;
@@ -217,7 +222,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       store_top(l == 0, Ft, F[0]);
       aC = 0.5 * sC;
       aN = 0.5 * sN;
-      column_rhs<LPC, ARITH>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, 0>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k[n] = k[n] + r;
         cs[n] = x[n] + (0.5 * dt) * r;
         Ft[n] = Fv;
@@ -225,7 +230,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       store_top(l == 0, Ft, F[1]);
       aC = aC + sC;
       aN = aN + sN;
-      column_rhs<LPC, ARITH>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, 0>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k[n] = k[n] + r;
         cs[n] = x[n] + dt * r;
         Ft[n] = Fv;
@@ -233,7 +238,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       store_top(l == 0, Ft, F[2]);
       aC = aC + sC;
       aN = aN + sN;
-      column_rhs<LPC, ARITH>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, 0>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k[n] = k[n] + 0.5 * r;
         Ft[n] = Fv;
       }, &d.zw);
@@ -253,7 +258,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       // solver_library.F90:164-185
       double cs[NV], k1[NV], k2[NV];
       double s1C, s1N, s2C, s2N;
-      column_rhs<LPC, ARITH>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, 0>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
         k1[n] = r;
         cs[n] = x[n] + (third * dt) * r;
         Ft[n] = Fv;
@@ -261,7 +266,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       store_top(l == 0, Ft, F[0]);
       s1C = sC;
       s1N = sN;
-      column_rhs<LPC, ARITH>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, 0>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k2[n] = r;
         cs[n] = x[n] + dt * (r - third * k1[n]);
         Ft[n] = Fv;
@@ -269,7 +274,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       store_top(l == 0, Ft, F[1]);
       s2C = sC;
       s2N = sN;
-      column_rhs<LPC, ARITH>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, 0>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         cs[n] = x[n] + dt * ((k1[n] - k2[n]) + r);
         k1[n] = (k1[n] + 3.0 * k2[n]) + 3.0 * r;
         Ft[n] = Fv;
@@ -277,7 +282,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       store_top(l == 0, Ft, F[2]);
       double aC = (s1C + 3.0 * s2C) + 3.0 * sC;
       double aN = (s1N + 3.0 * s2N) + 3.0 * sN;
-      column_rhs<LPC, ARITH>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, 0>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k1[n] = k1[n] + r;
         Ft[n] = Fv;
       }, &d.zw);
@@ -295,12 +300,12 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       kadd(acc[1], accc[1], w * aN);
     } else {  // EMP-1 / EMP-2 with a fixed step
       double f0[NV];
-      column_rhs<LPC, ARITH>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, 0>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
         f0[n] = r;
         Ft[n] = Fv;
       }, &d.zw);
       store_top(l == 0, Ft, F[0]);
-      const double p1 = pfactor<LPC, false, PW, BLOCK>(x, f0, x, dt, act, zs, dg.newton, &sgeo[0][threadIdx.x]);
+      const double p1 = pfactor<LPC, false, PW>(x, f0, x, dt, act, zs, dg.newton);
       if (p1 < dg.p_min) dg.p_min = p1;
       if (METHOD == SEDCOL_EMP1) {
 #pragma unroll
@@ -319,12 +324,12 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
           c1[n] = y < 0.0 ? 0.0 : y;
         }
         const double s0C = sC, s0N = sN;
-        column_rhs<LPC, ARITH>(p, L, bc, c1, sC, sN, [&](int n, double r, double Fv) {
+        column_rhs<LPC, ARITH, 0>(p, L, bc, c1, sC, sN, [&](int n, double r, double Fv) {
           f0[n] = (f0[n] + r) * 0.5;
           Ft[n] = Fv;
         }, &d.zw);
       store_top(l == 0, Ft, F[1]);
-        const double p2 = pfactor<LPC, true, PW, BLOCK>(x, f0, c1, dt, act, zs, dg.newton, &sgeo[0][threadIdx.x]);
+        const double p2 = pfactor<LPC, true, PW>(x, f0, c1, dt, act, zs, dg.newton);
         if (p2 < dg.p_min) dg.p_min = p2;
 #pragma unroll
         for (int n = 0; n < NV; ++n) x[n] = x[n] + (dt * p2) * f0[n];
@@ -394,7 +399,9 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
 // 3 spills about 340 bytes per lane).  With geometric weights the step does not
 // fit (130 to 190 bytes of scratch per lane) and one wave is faster at every
 // size, reference form, 1 h: 1201 columns of 30 to 60 layers 157 -> 104 ms,
-// 9000 columns of 10 to 60 layers 300 -> 235 ms.
+// 9000 columns of 10 to 60 layers 300 -> 235 ms.  It then has room for the
+// boundary values and the solve's coefficients, which were read from LDS in
+// every evaluation (3 h of the 1201 columns 273 -> 264 ms).
 #ifndef SEDCOL_EMP_MIN_WAVES
 #define SEDCOL_EMP_MIN_WAVES 2
 #endif
@@ -436,7 +443,15 @@ __global__ __launch_bounds__(BLK, PW == 1 ? SEDCOL_GEO_MIN_WAVES : SEDCOL_EMP_MI
   const int g = threadIdx.x / LPC, l = threadIdx.x % LPC;
   const bool own = l < NV;  // lane l accumulates the top flux of variable l
   double(*F)[NV] = sF[g];
+  // one wave per SIMD (PW == 1) has room for the boundary values in registers
+  constexpr int TF = PW == 1 ? 0 : NV;
+  double bcr[NV];
   const double *bc = sbc[g];
+  if constexpr (PW == 1) bc = bcr;
+  auto boundary = [&]() {
+    __builtin_amdgcn_wave_barrier();
+    if constexpr (PW == 1) take_top(p, sbc[g], bcr);
+  };
   const int r1 = ctl.r1;
 
   // state of the group's current column
@@ -449,8 +464,6 @@ __global__ __launch_bounds__(BLK, PW == 1 ? SEDCOL_GEO_MIN_WAVES : SEDCOL_EMP_MI
   // touched only when an attempt is accepted, so they live in LDS and leave
   // the registers to the right-hand side.
   __shared__ double sacc[7][BLK];
-  // coefficients of the geometric-mean Patankar solve (one slot otherwise)
-  __shared__ double sgeo[PW == 1 ? NV : 1][BLK];
   double &sinkC = sacc[0][threadIdx.x], &sinkN = sacc[1][threadIdx.x], &fint = sacc[2][threadIdx.x];
   double &sinkCc = sacc[3][threadIdx.x], &sinkNc = sacc[4][threadIdx.x], &fintc = sacc[5][threadIdx.x];
   double &flast = sacc[6][threadIdx.x];
@@ -499,7 +512,7 @@ __global__ __launch_bounds__(BLK, PW == 1 ? SEDCOL_GEO_MIN_WAVES : SEDCOL_EMP_MI
       if (rem > 0.0) {
         // resumed inside record r
         load_forcing<LPC, ARITH>(d, p, c, r, Gm, L, sbc[g]);
-        __builtin_amdgcn_wave_barrier();
+        boundary();
       }
     }
     bool finish = false;
@@ -515,7 +528,7 @@ __global__ __launch_bounds__(BLK, PW == 1 ? SEDCOL_GEO_MIN_WAVES : SEDCOL_EMP_MI
         const double b = ctl.t_end < hi ? ctl.t_end : hi;
         rem = b - a;
         load_forcing<LPC, ARITH>(d, p, c, r, Gm, L, sbc[g]);
-        __builtin_amdgcn_wave_barrier();
+        boundary();
         continue;
       }
     }
@@ -536,21 +549,21 @@ __global__ __launch_bounds__(BLK, PW == 1 ? SEDCOL_GEO_MIN_WAVES : SEDCOL_EMP_MI
       const double h = clipped ? rem : dt;
       double f0[NV], c1[NV];
       double s0C, s0N, s1C, s1N;
-      column_rhs<LPC, ARITH>(p, L, bc, x, s0C, s0N, [&](int n, double rr, double Fv) {
+      column_rhs<LPC, ARITH, TF>(p, L, bc, x, s0C, s0N, [&](int n, double rr, double Fv) {
         f0[n] = rr;
         if (l == 0) F[0][n] = Fv;
       }, &d.zw);
-      const double p1 = pfactor<LPC, false, PW, BLK>(x, f0, x, h, act, zs, dg.newton, &sgeo[0][threadIdx.x]);
+      const double p1 = pfactor<LPC, false, PW>(x, f0, x, h, act, zs, dg.newton);
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
         const double y = x[n] + (h * p1) * f0[n];
         c1[n] = y < 0.0 ? 0.0 : y;
       }
-      column_rhs<LPC, ARITH>(p, L, bc, c1, s1C, s1N, [&](int n, double rr, double Fv) {
+      column_rhs<LPC, ARITH, TF>(p, L, bc, c1, s1C, s1N, [&](int n, double rr, double Fv) {
         f0[n] = (f0[n] + rr) * 0.5;
         if (l == 0) F[1][n] = Fv;
       }, &d.zw);
-      const double p2 = pfactor<LPC, true, PW, BLK>(x, f0, c1, h, act, zs, dg.newton, &sgeo[0][threadIdx.x]);
+      const double p2 = pfactor<LPC, true, PW>(x, f0, c1, h, act, zs, dg.newton);
       // err = max |c2 - c1| / sc: the lane's largest ratio by
       // cross-multiplication over the variables, one division, then the
       // maximum over the layers
@@ -1001,8 +1014,8 @@ __device__ __forceinline__ void ros_rows(RosShared<LPC> &R, const RosLane &C, in
 // factor in registers: LDS traffic bounds the LDS form, because an access by
 // 11 lanes costs a full wave's (68 cycles a layer against a chain of 24).
 // A factor with its first sweep went from 6700 to 3300 cycles (24 layers), a
-// sweep down from 2200 to 930 and up from 2700 to 850; half a day of 3000
-// columns of 20 to 40 layers, a spin-up's chunk, from 222 to 122 ms.
+// sweep down from 2200 to 930 and up from 2700 to 850; a day of 3000
+// columns of 20 to 40 layers, a spin-up's two chunks, from 445 to 243 ms.
 
 // Thomas factor of species l's class and forward sweep of the first solve
 template <int LPC>
@@ -1348,7 +1361,11 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
   const int g = threadIdx.x / LPC, l = threadIdx.x % LPC;
   const bool own = l < NV;
   double(*F)[NV] = sF[g];
-  const double *bc = sbc[g];
+  double bc[NV];
+  auto boundary = [&]() {
+    __builtin_amdgcn_wave_barrier();
+    take_top(p, sbc[g], bc);
+  };
   RosShared<LPC> &R = sR[g];
   const int r1 = ctl.r1;
   const unsigned dirmask = (p.bcup_part == 2 ? 0x41Fu : 0u) | (p.bcup_dis == 2 ? 0x3E0u : 0u);
@@ -1419,6 +1436,7 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
       have = true;
       if (rem > 0.0) {
         load_forcing<LPC, ARITH>(d, p, c, r, Gm, L, sbc[g]);
+        boundary();
         coefficients();
       }
     }
@@ -1434,6 +1452,7 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
         const double b = ctl.t_end < hi ? ctl.t_end : hi;
         rem = b - a;
         load_forcing<LPC, ARITH>(d, p, c, r, Gm, L, sbc[g]);
+        boundary();
         coefficients();
         continue;
       }
@@ -1459,23 +1478,20 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
       double f[NV], k1[NV], k2[NV];
       double s0C, s0N, s1C = 0.0, s1N = 0.0;
       double Ft[NV];
-      column_rhs<LPC, ARITH>(p, L, bc, x, s0C, s0N, [&](int n, double rr, double Fv) {
+      column_rhs<LPC, ARITH, 0>(p, L, bc, x, s0C, s0N, [&](int n, double rr, double Fv) {
         f[n] = rr;
         Ft[n] = Fv;
       });
       store_top(l == 0, Ft, F[0]);
       ros_rows<LPC>(R, C, l, K, act, L.phi, gh, dirmask);
-      // the Jacobian is evaluated again for the second stage (same values)
-      // rather than kept live across the second right-hand side
-      double gC = 0.0, gN = 0.0;
-      bool ok;
-      {
-        KJac J;
-        kin_jac(p, L.fT, x, J);
-        ok = ros_wsolve<LPC, true>(R, S, J, C, l, K, kw, act, gh, dirmask, L.phi, f, k1, R.top[0]);
-        gC = kjac_sinkC(J, k1);
-        gN = kjac_sinkN(J, k1);
-      }
+      // The Jacobian stays live for the second stage, and with it the local
+      // solves' pivots: a spin-up of 3000 columns takes 165 ms against 171 with
+      // a second evaluation, though 64 lanes pay 168 bytes of scratch.
+      KJac J;
+      kin_jac(p, L.fT, x, J);
+      bool ok = ros_wsolve<LPC, true>(R, S, J, C, l, K, kw, act, gh, dirmask, L.phi, f, k1, R.top[0]);
+      double gC = kjac_sinkC(J, k1);
+      double gN = kjac_sinkN(J, k1);
       bool fail = group_any<LPC>(!ok);
       if (!fail) {
 #pragma unroll
@@ -1486,13 +1502,11 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
         double c1[NV];
 #pragma unroll
         for (int n = 0; n < NV; ++n) c1[n] = f[n];
-        column_rhs<LPC, ARITH>(p, L, bc, c1, s1C, s1N, [&](int n, double rr, double Fv) {
+        column_rhs<LPC, ARITH, 0>(p, L, bc, c1, s1C, s1N, [&](int n, double rr, double Fv) {
           f[n] = rr - 2.0 * k1[n];
           Ft[n] = Fv;
         });
         store_top(l == 0, Ft, F[1]);
-        KJac J;
-        kin_jac(p, L.fT, x, J);
         ok = ros_wsolve<LPC, false>(R, S, J, C, l, K, kw, act, gh, dirmask, L.phi, f, k2, R.top[1]);
         fail = group_any<LPC>(!ok);
         gC = gC + kjac_sinkC(J, k2);
@@ -1786,11 +1800,9 @@ __global__ __launch_bounds__(BLK) void k_ae_fused(const Dev *dptr, const int *li
   const bool act = valid && L.active;
   const bool own = valid && l < NV;
   // boundary values: in registers for one wave, as in k_fixed
-  double rbc[2 * NV];
-  if constexpr (ONE) {
-#pragma unroll
-    for (int n = 0; n < 2 * NV; ++n) rbc[n] = sbc[g][n];
-  }
+  constexpr int TF = ONE ? 0 : NV;
+  double rbc[NV];
+  if constexpr (ONE) take_top(p, sbc[g], rbc);
   const double *bc = ONE ? rbc : sbc[g];
   double x[NV], r[NV];
 #pragma unroll
@@ -1832,7 +1844,7 @@ __global__ __launch_bounds__(BLK) void k_ae_fused(const Dev *dptr, const int *li
       if (need) {
         if (valid) {
           double Ft[NV];
-          column_rhs<LPC, ARITH>(p, L, bc, x, sC, sN, [&](int n, double rr, double F) {
+          column_rhs<LPC, ARITH, TF>(p, L, bc, x, sC, sN, [&](int n, double rr, double F) {
             r[n] = rr;
             Ft[n] = F;
           }, &d.zw);
