@@ -178,8 +178,9 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
   const bool own = l < NV;  // lane l accumulates the top flux of variable l
 
   double x[NV];
+  const double *from = d.hconc ? d.hconc : d.conc;
 #pragma unroll
-  for (int n = 0; n < NV; ++n) x[n] = act ? d.conc[n * d.ncell + cell] : 0.0;
+  for (int n = 0; n < NV; ++n) x[n] = act ? from[n * d.ncell + cell] : 0.0;
   double fint = own ? d.colacc[(long long)l * d.ncol + c] : 0.0;
   double fintc = own ? d.colacc[(long long)(NV + l) * d.ncol + c] : 0.0;
   double flast = own ? d.flux[(long long)l * d.ncol + c] : 0.0;
@@ -363,7 +364,10 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       for (int n = 0; n < NV; ++n) nan |= act && (x[n] != x[n]);
       if (group_any<LPC>(nan)) {
         dg.status = 1;
-        if (l == 0) atomicOr(errflag, 1);
+        if (l == 0) {
+          atomicOr(errflag, 1);
+          if (d.hflag) *d.hflag = 1;
+        }
         break;
       }
     }
@@ -376,6 +380,12 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
     d.colacc[(long long)l * d.ncol + c] = fint;
     d.colacc[(long long)(NV + l) * d.ncol + c] = fintc;
     d.flux[(long long)l * d.ncol + c] = flast;
+  }
+  if (d.hconc) {
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+      if (act) d.hconc[n * d.ncell + cell] = x[n];
+    if (own) d.hflux[(long long)l * d.ncol + c] = flast;
   }
 #pragma unroll
   for (int a = 0; a < 5; ++a)

@@ -32,6 +32,11 @@ struct Dev {
   int *wrec;        // ncol: current forcing record (past the last one: done)
   double *wrem;     // ncol: time left in that record
   long long *watt;  // ncol: attempts since the start of the span
+  // pinned host memory of sedcol_step, or null: k_fixed takes the state from hconc
+  // and leaves the new one there too, the top fluxes in hflux and 1 in *hflag if
+  // a column has a NaN
+  double *hconc, *hflux;
+  int *hflag;
 };
 
 // Span of one adaptive integration, read by the kernel through a pointer
