@@ -1097,7 +1097,8 @@ __device__ __forceinline__ double row_bcast(double v)
 // broadcast, one VALU move each.  A species' right-hand side is read from
 // LDS once, swept down and up in registers and written back.  Layers beyond
 // the column are identity rows with right-hand side 0, so a finite last value
-// leaves T_{K-1} as it is; ok() is false when it is not finite.
+// leaves T_{K-1} as it is; solve() leaves a column whose last value is not
+// finite to the LDS form.
 template <int LPC>
 struct RosSweep {
   static constexpr int R16 = LPC / 16;
@@ -1231,9 +1232,20 @@ struct RosSweep {
     }
   }
 
+  // the factor to where the LDS form reads it
+  __device__ __forceinline__ void store_factor(RosShared<LPC> &R) const
+  {
+#pragma unroll
+    for (int i = 0; i < R16; ++i) {
+      R.AI[m][16 * i + j].y = iv[i];
+      R.E[m][16 * i + j] = E[i];
+    }
+  }
+
   // B z = T for the group's species; FACTOR makes the factor first.  False
-  // (with T untouched) when a pivot is outside the range of rcp_exact or a
-  // value is not finite in any active group: the LDS form then takes over.
+  // (with T untouched) when a pivot of the group is outside the range of
+  // rcp_exact or a value is not finite: the LDS form then takes over, for this
+  // group alone, so that a column does not depend on its neighbour in the wave.
   template <bool FACTOR>
   __device__ __forceinline__ bool solve(RosShared<LPC> &R, int kw)
   {
@@ -1258,10 +1270,12 @@ struct RosSweep {
     } else {
       forward(t, d, kw);
     }
-    if (__any(!(ok && fabs(d) < INFINITY))) return false;
-    backward(t, d, kw);
-    store_all(t, kw);
-    return true;
+    const bool good = !group_any<LPC>(!(ok && fabs(d) < INFINITY));
+    if (good) {
+      backward(t, d, kw);
+      store_all(t, kw);
+    }
+    return good;
   }
 };
 
@@ -1292,6 +1306,10 @@ __device__ __forceinline__ void ros_bsolve(RosShared<LPC> &R, RosSweep<LPC> &S, 
   bool done = false;
   if constexpr (LPC > 16) done = S.template solve<FACTOR>(R, kw);
   if (!done) {
+    if constexpr (LPC > 16 && !FACTOR) {
+      S.store_factor(R);  // it may have been made in registers
+      __builtin_amdgcn_wave_barrier();
+    }
     if (FACTOR) ros_factor_lds<LPC>(R, l, K);
     else ros_forward_lds<LPC>(R, l, K);
     __builtin_amdgcn_wave_barrier();
