@@ -1114,14 +1114,18 @@ struct RosSweep {
     own = l < 32 && j < (m == 0 ? 6 : 5);
     T = R.T[m == 0 ? (j < 5 ? j : 10) : (j < 5 ? 5 + j : 5)];
   }
-  __device__ __forceinline__ void load_factor(const RosShared<LPC> &R)
+  // the factor that the LDS form made: it has the rows of the column, the rest
+  // are identity rows
+  __device__ __forceinline__ void load_factor(const RosShared<LPC> &R, int K)
   {
 #pragma unroll
     for (int i = 0; i < R16; ++i) {
       const dbl2 ai = R.AI[m][16 * i + j];
+      const double e = R.E[m][16 * i + j];
+      const bool in = 16 * i + j < K;
       a[i] = ai.x;
-      iv[i] = ai.y;
-      E[i] = R.E[m][16 * i + j];
+      iv[i] = in ? ai.y : 1.0;
+      E[i] = in ? e : 0.0;
     }
   }
   template <int B>
@@ -1316,7 +1320,7 @@ __device__ __forceinline__ void ros_bsolve(RosShared<LPC> &R, RosSweep<LPC> &S, 
     ros_backward_lds<LPC>(R, l, K);
     if constexpr (LPC > 16) {
       __builtin_amdgcn_wave_barrier();
-      if (FACTOR) S.load_factor(R);
+      if (FACTOR) S.load_factor(R, K);
     }
   }
   __builtin_amdgcn_wave_barrier();

@@ -1,7 +1,8 @@
 """The sweeps of the linearly implicit stepper leave their registers for the
 general form when a value is not finite or a pivot is out of range.  A column
-that does so must not change the column that shares its wave; bitwise against
-the oracle."""
+that does so must not change the column that shares its wave, nor may what an
+earlier launch left in LDS enter the rows beyond a column; bitwise against the
+oracle."""
 import numpy as np
 import pytest
 
@@ -44,3 +45,28 @@ def test_column_beside_an_overflowing_one(gpu_ready, layers, bad, span, block):
     assert np.array_equal(xg, xo)
     for k in ("accepted", "rejected", "dt_next"):
         assert np.array_equal(dg[k], orc.diag[k]), k
+
+
+def test_rows_beyond_a_column(gpu_ready):
+    """Columns of 32 layers leave a factor that is not a number in row 23 of
+    every place; the columns of 17 layers that follow there have pivots out of
+    range, so they take their factor from LDS and their later solves run over 24
+    rows."""
+    n, m = 4096, 64
+    dom = _domain(np.repeat([32, 17], [n, m]))
+    dom.params.clamp = 0
+    dom.params.D0 = 1.0e283
+    dom.dzc[dom.off[:n] + 24] *= 1.0e-30
+    with capi.SedimentColumns.from_domain(dom) as g:
+        with pytest.raises(capi.SedcolError) as e:
+            g.integrate(0.0, 1800.0)
+        assert e.value.code == capi.SEDCOL_ENAN
+        xg, dg = g.get_state(), g.diagnostics()
+    sub = dom.subset(np.arange(n, n + m))
+    orc = O.Oracle(sub, dom.params.si())
+    xo = sub.conc0.copy()
+    assert orc.emp_integrate(xo, 1800.0, nthreads=4) == 0
+    assert np.all(np.isfinite(xo))
+    assert np.all(dg["status"][:n] == 1) and np.all(dg["status"][n:] == 0)
+    assert np.array_equal(xg[:, dom.off[n]:], xo)
+    assert np.array_equal(dg["accepted"][n:], orc.diag["accepted"])
