@@ -150,11 +150,12 @@ __device__ __forceinline__ double drsqrt(double x)
 // Correctly rounded quotients without the range scaling of the IEEE
 // division: the hardware reciprocal estimate (relative error 2^-24), one
 // third-order step to the last place (rcp_near), and Markstein's correction of
-// the quotient by its residual.  They equal the IEEE division's results while
-// b and 1/b are well inside the normal range, |a| is 0 or at least 2^-970 (so
-// that the residual is exact) and the quotient is normal; callers check the
-// range.  In issue slots of 4 cycles: 10 for a division against 14, 9 for a
-// reciprocal, 3 for a division by a b whose reciprocal is at hand.
+// the quotient by its residual.  They equal the IEEE division's results, the
+// sign of a zero included, while b is positive, b and 1/b are well inside the
+// normal range, |a| is 0 or at least 2^-970 (so that the residual is exact) and
+// the quotient is normal; callers check the range.  In issue slots of 4 cycles:
+// 10 for a division against 14, 9 for a reciprocal, 3 for a division by a b
+// whose reciprocal is at hand.
 __device__ __forceinline__ double rcp_near(double b)
 {
   const double y = __builtin_amdgcn_rcp(b);
@@ -166,11 +167,12 @@ __device__ __forceinline__ double rcp_exact(double b)
   const double y = rcp_near(b);
   return fma(fma(-b, y, 1.0), y, y);
 }
-// a / b with y = 1/b rounded
+// a / b with y = 1/b rounded.  The residual is taken with its sign reversed: for
+// b > 0 a zero quotient then keeps the sign of a (q + -0), which q + 0 loses.
 __device__ __forceinline__ double div_by(double a, double b, double y)
 {
   const double q = a * y;
-  return fma(fma(-b, q, a), y, q);
+  return fma(-fma(b, q, -a), y, q);
 }
 template <bool FD>
 __device__ __forceinline__ double quot(double a, double b)
