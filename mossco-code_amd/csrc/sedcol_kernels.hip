@@ -149,9 +149,31 @@ __global__ __launch_bounds__(BLOCK) void k_rhs(Dev d, const int *list, int nlist
 // fixed-step window: EULER, RK4, RK4 3/8, EMP-1, EMP-2
 // ---------------------------------------------------------------------------
 
-template <int LPC, int METHOD, int ARITH, int PW = 0>
-__global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nlist, sedcol_params p, int rec,
-                                                 double dt, int nsteps, int *errflag)
+// Instances that take a little more than the 256 registers of two waves per
+// SIMD.  A launch of at most one wave per SIMD is a lone chain per wave, which
+// the registers suit best; beyond, the second wave hides more than the few
+// spilled values cost (FULL).  24 steps of 30 layers, one wave and two:
+//                                   600 columns     2200 columns    20000 columns
+//   EMP-2, reference form           210    216 us   381    296 us   1808   1283 us
+//   EMP-1 ext. form                 168    172      296    227      1345    937
+//   EMP-1 geometric, fast form      158    168      279    223      1262    921
+// The Euler step of the extended form gains from two waves at every size (600
+// columns 138 -> 131 us, 20000 columns 1025 -> 699 us).
+constexpr bool fixed_split(int method, int arith, int pw)
+{
+  return method == SEDCOL_EMP2   ? arith == ARITH_REF && pw == 0
+         : method == SEDCOL_EMP1 ? (arith == ARITH_EXT && pw == 0) || (arith == ARITH_FAST && pw == 1)
+                                 : false;
+}
+constexpr int fixed_waves(int method, int arith, bool full)
+{
+  return full || (method == SEDCOL_EULER && arith == ARITH_EXT) ? 2 : 1;
+}
+
+template <int LPC, int METHOD, int ARITH, int PW, bool FULL>
+__global__ __launch_bounds__(BLOCK, fixed_waves(METHOD, ARITH, FULL)) void k_fixed(Dev d, const int *list, int nlist,
+                                                                                 sedcol_params p, int rec, double dt,
+                                                                                 int nsteps, int *errflag)
 {
   constexpr int G = BLOCK / LPC;
   __shared__ double sbc[G][2 * NV];
@@ -170,9 +192,16 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
   __syncthreads();
   if (!valid) return;
   // the boundary values stay in registers for the whole run: read from LDS in
-  // every right-hand side, they cost a lone wave 1600 of 4900 cycles
-  double bc[NV];
-  take_top(p, sbc[g], bc);
+  // every right-hand side, they cost a lone wave 1600 of 4900 cycles.  The two
+  // waves of a full EMP-1 launch read them (in registers, 80 and 156 instead of
+  // 20 and 80 bytes of scratch, and 4 and 16 % more time at 20000 columns)
+  constexpr int TF = FULL && METHOD == SEDCOL_EMP1 ? NV : 0;
+  double bcr[NV];
+  const double *bc = sbc[g];
+  if constexpr (TF == 0) {
+    take_top(p, sbc[g], bcr);
+    bc = bcr;
+  }
   double(*F)[NV] = sF[g];
   const bool act = L.active;
   const bool own = l < NV;  // lane l accumulates the top flux of variable l
@@ -198,7 +227,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
     double sC, sN, Ft[NV];
     if (METHOD == SEDCOL_EULER) {
       double r0[NV];
-      column_rhs<LPC, ARITH, 0>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, TF>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
         r0[n] = r;
         Ft[n] = Fv;
       }, &d.zw);
@@ -215,7 +244,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       // solver_library.F90:142-163
       double cs[NV], k[NV];
       double aC, aN;
-      column_rhs<LPC, ARITH, 0>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, TF>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
         k[n] = 0.5 * r;
         cs[n] = x[n] + (0.5 * dt) * r;
         Ft[n] = Fv;
@@ -223,7 +252,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       store_top(l == 0, Ft, F[0]);
       aC = 0.5 * sC;
       aN = 0.5 * sN;
-      column_rhs<LPC, ARITH, 0>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, TF>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k[n] = k[n] + r;
         cs[n] = x[n] + (0.5 * dt) * r;
         Ft[n] = Fv;
@@ -231,7 +260,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       store_top(l == 0, Ft, F[1]);
       aC = aC + sC;
       aN = aN + sN;
-      column_rhs<LPC, ARITH, 0>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, TF>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k[n] = k[n] + r;
         cs[n] = x[n] + dt * r;
         Ft[n] = Fv;
@@ -239,7 +268,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       store_top(l == 0, Ft, F[2]);
       aC = aC + sC;
       aN = aN + sN;
-      column_rhs<LPC, ARITH, 0>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, TF>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k[n] = k[n] + 0.5 * r;
         Ft[n] = Fv;
       }, &d.zw);
@@ -259,7 +288,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       // solver_library.F90:164-185
       double cs[NV], k1[NV], k2[NV];
       double s1C, s1N, s2C, s2N;
-      column_rhs<LPC, ARITH, 0>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, TF>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
         k1[n] = r;
         cs[n] = x[n] + (third * dt) * r;
         Ft[n] = Fv;
@@ -267,7 +296,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       store_top(l == 0, Ft, F[0]);
       s1C = sC;
       s1N = sN;
-      column_rhs<LPC, ARITH, 0>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, TF>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k2[n] = r;
         cs[n] = x[n] + dt * (r - third * k1[n]);
         Ft[n] = Fv;
@@ -275,7 +304,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       store_top(l == 0, Ft, F[1]);
       s2C = sC;
       s2N = sN;
-      column_rhs<LPC, ARITH, 0>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, TF>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         cs[n] = x[n] + dt * ((k1[n] - k2[n]) + r);
         k1[n] = (k1[n] + 3.0 * k2[n]) + 3.0 * r;
         Ft[n] = Fv;
@@ -283,7 +312,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       store_top(l == 0, Ft, F[2]);
       double aC = (s1C + 3.0 * s2C) + 3.0 * sC;
       double aN = (s1N + 3.0 * s2N) + 3.0 * sN;
-      column_rhs<LPC, ARITH, 0>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, TF>(p, L, bc, cs, sC, sN, [&](int n, double r, double Fv) {
         k1[n] = k1[n] + r;
         Ft[n] = Fv;
       }, &d.zw);
@@ -301,7 +330,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
       kadd(acc[1], accc[1], w * aN);
     } else {  // EMP-1 / EMP-2 with a fixed step
       double f0[NV];
-      column_rhs<LPC, ARITH, 0>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
+      column_rhs<LPC, ARITH, TF>(p, L, bc, x, sC, sN, [&](int n, double r, double Fv) {
         f0[n] = r;
         Ft[n] = Fv;
       }, &d.zw);
@@ -325,7 +354,7 @@ __global__ __launch_bounds__(BLOCK) void k_fixed(Dev d, const int *list, int nli
           c1[n] = y < 0.0 ? 0.0 : y;
         }
         const double s0C = sC, s0N = sN;
-        column_rhs<LPC, ARITH, 0>(p, L, bc, c1, sC, sN, [&](int n, double r, double Fv) {
+        column_rhs<LPC, ARITH, TF>(p, L, bc, c1, sC, sN, [&](int n, double r, double Fv) {
           f0[n] = (f0[n] + r) * 0.5;
           Ft[n] = Fv;
         }, &d.zw);
@@ -2119,13 +2148,20 @@ void launch_rhs(int lpc, hipStream_t st, const Dev &d, const int *list, int n, c
                                                                st, d, list, n, p, rec, conc, rhs, flux, sinks)));
 }
 
+// lanes of one wave on each of the 1024 SIMDs
+constexpr long long kSimdLanes = 1024 * 64;
+
 void launch_fixed(int lpc, int method, hipStream_t st, const Dev &d, const int *list, int n,
                   const sedcol_params &p, int rec, double dt, int nsteps, int *errflag)
 {
+  const bool full = (long long)n * lpc > kSimdLanes;
 #define SC_FIX(M, W)                                                                                             \
-  SC_DISPATCH_ARITH(p, SC_DISPATCH_LPC(lpc, hipLaunchKernelGGL((k_fixed<LPC, M, AR, W>), grid_for<LPC>(n),        \
-                                                               dim3(BLOCK), 0, st, d, list, n, p, rec, dt, nsteps, \
-                                                               errflag)))
+  SC_DISPATCH_ARITH(p, SC_DISPATCH_LPC(lpc, {                                                                      \
+                      auto *k = k_fixed<LPC, M, AR, W, false>;                                                     \
+                      if (full) k = k_fixed<LPC, M, AR, W, fixed_split(M, AR, W)>;                                 \
+                      hipLaunchKernelGGL(k, grid_for<LPC>(n), dim3(BLOCK), 0, st, d, list, n, p, rec, dt, nsteps,  \
+                                         errflag);                                                                 \
+                    }))
   const bool geo = p.emp_weights == 1;
   switch (method) {
     case SEDCOL_EULER: SC_FIX(SEDCOL_EULER, 0); break;
