@@ -22,7 +22,8 @@ def _domain(layers, seed=17):
 
 
 @pytest.mark.parametrize("block", [64, 256])
-@pytest.mark.parametrize("layers,bad", [((24, 20), 0), ((24, 20), 1), ((17, 32), 0), ((32, 25, 18, 31, 17, 20), 3)])
+@pytest.mark.parametrize("layers,bad", [((24, 20), 0), ((24, 20), 1), ((17, 32), 0), ((32, 25, 18, 31, 17, 20), 3),
+                                        ((40, 64, 33), 1)])
 @pytest.mark.parametrize("span", [1.0, 30.0])
 def test_column_beside_an_overflowing_one(gpu_ready, layers, bad, span, block):
     """Bottom water of 1e70 mmol/m3 oxygen: the rates of the first stage are
