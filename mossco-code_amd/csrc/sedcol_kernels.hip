@@ -1866,7 +1866,17 @@ __global__ __launch_bounds__(BLK) void k_ae_fused(const Dev *dptr, const int *li
   double rbc[NV];
   if constexpr (ONE) take_top(p, sbc[g], rbc);
   const double *bc = ONE ? rbc : sbc[g];
-  double x[NV], r[NV];
+  // Two waves per SIMD (BLK = 512) have no registers for the rates between an
+  // evaluation and its step: in LDS 12 to 252 bytes of scratch per lane are left
+  // of 92 to 428, and four calls of 1800 s for 20 columns of 16 layers take 245 us
+  // instead of 360 (fast form 207 for 241, extended form 403 for 762).
+  constexpr bool RLDS = BLK > 256;
+  __shared__ double srate[RLDS ? NV : 1][RLDS ? BLK : 1];
+  double x[NV], rreg[NV];
+  auto r = [&](int n) -> double & {
+    if constexpr (RLDS) return srate[n][threadIdx.x];
+    else return rreg[n];
+  };
 #pragma unroll
   for (int n = 0; n < NV; ++n) x[n] = act ? d.conc[n * d.ncell + cell] : 0.0;
   double sC = 0.0, sN = 0.0;
@@ -1907,7 +1917,7 @@ __global__ __launch_bounds__(BLK) void k_ae_fused(const Dev *dptr, const int *li
         if (valid) {
           double Ft[NV];
           column_rhs<LPC, ARITH, TF>(p, L, bc, x, sC, sN, [&](int n, double rr, double F) {
-            r[n] = rr;
+            r(n) = rr;
             Ft[n] = F;
           }, &d.zw);
           store_top(l == 0, Ft, sF[g]);
@@ -1918,7 +1928,7 @@ __global__ __launch_bounds__(BLK) void k_ae_fused(const Dev *dptr, const int *li
       bool v = false;
       if (act) {
 #pragma unroll
-        for (int n = 0; n < NV; ++n) v |= ae_violates(x[n], r[n], dt_red, rcm);
+        for (int n = 0; n < NV; ++n) v |= ae_violates(x[n], r(n), dt_red, rcm);
       }
       const int viol = ONE ? __any(v) : __syncthreads_or(v);
       if (viol && dt_red > p.dt_min) {
@@ -1930,7 +1940,7 @@ __global__ __launch_bounds__(BLK) void k_ae_fused(const Dev *dptr, const int *li
         dt_last = dt_red;
         if (act) {
 #pragma unroll
-          for (int n = 0; n < NV; ++n) x[n] = x[n] + dt_red * r[n];
+          for (int n = 0; n < NV; ++n) x[n] = x[n] + dt_red * r(n);
           kadd(acc(0), acc(2), dt_red * sC);
           kadd(acc(1), acc(3), dt_red * sN);
         }
