@@ -614,7 +614,8 @@ __global__ __launch_bounds__(BLK, PW == 1 ? SEDCOL_GEO_MIN_WAVES : SEDCOL_EMP_MI
         const double yp = vmax(y, 0.0);
         const double sc = p.emp_atol + p.emp_rtol * vmax(yp, x[n]);
         const double dv = fabs(yp - c1[n]);
-        bad |= (y != y) || (sc != sc);
+        // a NaN in y (vmax drops it) or in dv (two infinities), in one comparison
+        bad |= __builtin_isunordered(y, dv) || (sc != sc);
         if (dv * bd > bn * sc) {
           bn = dv;
           bd = sc;
