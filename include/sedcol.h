@@ -174,7 +174,12 @@ typedef struct {
  * parameter sets run such a bin with one layer per lane); 0 reads as 1.
  * lanes_per_column: 16, 32 or 64, at least the bin's largest K divided by
  * layers_per_lane; workgroup = lanes_per_column * columns_per_group threads,
- * 64, 128 or 256.  Results are identical for every shape. */
+ * 64, 128 or 256.  Until a shape is installed (sedcol_set_tuning,
+ * sedcol_autotune), the bins run with 16, 32 and 64 lanes, one layer per lane,
+ * in workgroups of 256 threads, the linearly implicit stepper (method 7) in
+ * workgroups of 64; sedcol_get_tuning reports what the current parameters run.
+ * An installed shape holds for every method.  Results are identical for every
+ * shape. */
 #define SEDCOL_NBIN 3
 typedef struct {
   int32_t lanes_per_column[SEDCOL_NBIN];

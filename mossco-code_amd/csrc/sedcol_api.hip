@@ -312,11 +312,16 @@ int check_tuning(const sedcol_handle *h, const sedcol_tuning *t)
   return SEDCOL_OK;
 }
 
-// kernel shape bin b runs with under the current parameters.  Unless a shape
-// was installed, the linearly implicit stepper runs in blocks of one wave: a
-// block holds its place until its slowest column is done, and at one wave per
-// SIMD a place is a quarter of a CU (a day of spin-up of 3000 columns 189 ->
-// 175 ms; adaptive EMP does not gain).  An installed
+// workgroup size of bin b.  Unless a shape was installed, the linearly implicit
+// stepper runs in blocks of one wave: a block holds its place until its slowest
+// column is done, and at one wave per SIMD a place is a quarter of a CU (a day of
+// spin-up of 3000 columns 189 -> 175 ms; adaptive EMP does not gain).
+int group_size(const sedcol_handle *h, int b)
+{
+  return !h->tuned && h->p.adaptive_method == SEDCOL_ROS2_ADAPTIVE ? std::max(64, h->lpc[b]) : h->blk[b];
+}
+
+// kernel shape bin b runs with under the current parameters.  An installed
 // two-layers-per-lane shape falls back to one layer per lane (with enough
 // lanes for the bin) where that kernel does not cover the parameters
 // (linearly implicit stepper, geometric-mean weights, bioturbation profile
@@ -324,9 +329,8 @@ int check_tuning(const sedcol_handle *h, const sedcol_tuning *t)
 void effective_shape(const sedcol_handle *h, int b, int *lpc, int *blk, int *lpl)
 {
   *lpc = h->lpc[b];
-  *blk = h->blk[b];
+  *blk = group_size(h, b);
   *lpl = h->lpl[b];
-  if (!h->tuned && h->p.adaptive_method == SEDCOL_ROS2_ADAPTIVE) *blk = std::max(64, *lpc);
   if (*lpl == 2 && !sc::emp2_supported(h->p)) {
     *lpl = 1;
     *lpc = std::max(*lpc, bin_min_lpc(h, b, 1));
@@ -1395,7 +1399,7 @@ int sedcol_get_tuning(sedcol_handle *h, sedcol_tuning *t)
   const DeviceScope dscope(h->device);
   for (int b = 0; b < SEDCOL_NBIN; ++b) {
     t->lanes_per_column[b] = h->lpc[b];
-    t->columns_per_group[b] = h->blk[b] / h->lpc[b];
+    t->columns_per_group[b] = group_size(h, b) / h->lpc[b];
     t->layers_per_lane[b] = h->lpl[b];
   }
   return SEDCOL_OK;
@@ -1447,11 +1451,11 @@ int sedcol_autotune(sedcol_handle *h, double t_start, double t_span, int32_t rep
   std::memcpy(saved_blk, h->blk, sizeof saved_blk);
   std::memcpy(saved_lpl, h->lpl, sizeof saved_lpl);
   h->sched = sedcol_schedule{0, 0, 1, 0};  // one launch per trial
-  const bool saved_tuned = h->tuned;
-  h->tuned = true;
   int best_l[3], best_w[3], best_p[3];
   std::memcpy(best_l, h->lpc, sizeof best_l);
-  std::memcpy(best_w, h->blk, sizeof best_w);
+  for (int b = 0; b < 3; ++b) best_w[b] = group_size(h, b);
+  const bool saved_tuned = h->tuned;
+  h->tuned = true;
   std::memcpy(best_p, h->lpl, sizeof best_p);
   for (int b = 0; b < 3 && rc == SEDCOL_OK; ++b) {
     if (h->bins[b].empty()) continue;
