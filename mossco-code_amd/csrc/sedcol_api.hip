@@ -112,6 +112,7 @@ struct sedcol_handle {
                              // [5], [6] votes of adaptive Euler attempts
   int *h_flag = nullptr;     // pinned host copy of d_flag[0..4]
   bool piped = false;        // counts as a user of the pinned blocks (copy_large)
+  std::vector<double> h_pack;  // small Fortran states, packed
   double *h_stage = nullptr; // pinned: state, top fluxes and flags of sedcol_step, small domains only
   int *d_work = nullptr;     // ncol: attempts of each column in the last adaptive launch
   int *d_wrec = nullptr;     // ncol: adaptive position between windows (record, time left, attempts)
@@ -493,7 +494,7 @@ int ensure_scratch(sedcol_handle *h)
 
 // The caller's state arrays go to and from the device as they are, without a
 // copy in host memory: packed ones directly, Fortran ones through d_scr and
-// k_layout.  (With the transposition on the host and pageable copies, setting
+// k_layout, small ones excepted.  (With the transposition on the host and pageable copies, setting
 // 238 MB took 59 ms and reading them 76 ms.)
 //
 // Large copies go through pinned blocks that several threads fill or empty: the
@@ -592,11 +593,38 @@ int copy_large(sedcol_handle *h, void *dev, const void *in, void *out, size_t by
   return SEDCOL_OK;
 }
 
-// caller's state (NV planes) -> packed device array dst (not d_scr)
-int put_state(sedcol_handle *h, const double *conc, double *dst)
+// A small Fortran state is transposed by the host instead, in h_pack: there a
+// launch costs more than the loop.  In us, host and device: setting and reading
+// 16 columns of 15 layers 11 and 12, 24 and 25; 200 of 25 layers 38 and 40, 37 and
+// 43; 400 of 15 layers 44 and 46, 40 and 45.  The right-hand side, both ways in
+// one call: 63 and 80; 103 and 115; 115 and 123; 500 of 15 layers 135 and 133.
+constexpr long long kHostCells = 5500, kHostCellsRhs = 7000;  // h_pack is made for the larger
+static_assert(kHostCells <= kHostCellsRhs, "h_pack");
+
+void transpose_state(const sedcol_handle *h, const double *src, double *dst, bool to_packed)
+{
+  const long long plane = (long long)h->ncol * h->kmax;
+  for (int n = 0; n < NV; ++n)
+    for (int k = 0; k < h->kmax; ++k) {
+      const long long f = n * plane + fidx(h, 0, k), x = n * plane + k;
+      if (to_packed)
+        for (int c = 0; c < h->ncol; ++c) dst[x + (long long)c * h->kmax] = src[f + c];
+      else
+        for (int c = 0; c < h->ncol; ++c) dst[f + c] = src[x + (long long)c * h->kmax];
+    }
+}
+
+// caller's state (NV planes) -> packed device array dst (not d_scr if the device
+// transposes); a Fortran state of up to host_cells cells is transposed by the host
+int put_state(sedcol_handle *h, const double *conc, double *dst, long long host_cells)
 {
   const size_t bytes = sizeof(double) * NV * (size_t)h->ncell;
   if (h->layout == SEDCOL_LAYOUT_PACKED) return copy_large(h, dst, conc, nullptr, bytes, true);
+  if (h->ncell <= host_cells) {
+    transpose_state(h, conc, h->h_pack.data(), true);
+    HIPOK(hipMemcpyAsync(dst, h->h_pack.data(), bytes, hipMemcpyHostToDevice, h->stream));
+    return SEDCOL_OK;
+  }
   if (!h->d_scr) HIPOK(hipMalloc(&h->d_scr, bytes));
   const int rc = copy_large(h, h->d_scr, conc, nullptr, bytes, true);
   if (rc) return rc;
@@ -605,10 +633,15 @@ int put_state(sedcol_handle *h, const double *conc, double *dst)
   return SEDCOL_OK;
 }
 
-// packed device array src -> caller's state (queued; src not d_scr)
-int take_state(sedcol_handle *h, double *src, double *conc)
+// packed device array src (not d_scr if the device transposes) -> caller's state;
+// complete after a wait and unpack_state
+int take_state(sedcol_handle *h, double *src, double *conc, long long host_cells)
 {
   const size_t bytes = sizeof(double) * NV * (size_t)h->ncell;
+  if (h->layout != SEDCOL_LAYOUT_PACKED && h->ncell <= host_cells) {
+    HIPOK(hipMemcpyAsync(h->h_pack.data(), src, bytes, hipMemcpyDeviceToHost, h->stream));
+    return SEDCOL_OK;
+  }
   if (h->layout != SEDCOL_LAYOUT_PACKED) {
     if (!h->d_scr) HIPOK(hipMalloc(&h->d_scr, bytes));
     sc::launch_layout(h->stream, src, h->d_scr, h->ncol, h->kmax, NV, false);
@@ -616,6 +649,12 @@ int take_state(sedcol_handle *h, double *src, double *conc)
     src = h->d_scr;
   }
   return copy_large(h, src, nullptr, conc, bytes, false);
+}
+
+void unpack_state(sedcol_handle *h, double *conc, long long host_cells)
+{
+  if (h->layout != SEDCOL_LAYOUT_PACKED && h->ncell <= host_cells)
+    transpose_state(h, h->h_pack.data(), conc, false);
 }
 
 // upload the current bins as the work lists (after a change of the active set)
@@ -750,6 +789,7 @@ int sedcol_create(const sedcol_desc *desc, sedcol_handle **out)
   HIPOK_C(hipMalloc(&h->d_flag, sizeof(int) * 8));  // error flag, one work-queue counter per bin, pending
   HIPOK_C(hipMemset(h->d_flag, 0, sizeof(int) * 8));
   HIPOK_C(hipHostMalloc((void **)&h->h_flag, sizeof(int) * 8, hipHostMallocDefault));
+  if (h->layout != SEDCOL_LAYOUT_PACKED && h->ncell <= kHostCellsRhs) h->h_pack.resize(NV * (size_t)h->ncell);
   if (sizeof(double) * NV * (size_t)h->ncell >= kPipeMin) {
     pipe_acquire();
     h->piped = true;
@@ -1042,7 +1082,7 @@ int sedcol_set_state(sedcol_handle *h, const double *conc)
 {
   if (!h || !conc) return fail(SEDCOL_EINVAL, "null argument");
   const DeviceScope dscope(h->device);
-  int rc = put_state(h, conc, h->d_conc);
+  int rc = put_state(h, conc, h->d_conc, kHostCells);
   if (rc) return rc;
   HIPOK(hipStreamSynchronize(h->stream));
   return SEDCOL_OK;
@@ -1087,9 +1127,10 @@ int sedcol_get_state(sedcol_handle *h, double *conc)
 {
   if (!h || !conc) return fail(SEDCOL_EINVAL, "null argument");
   const DeviceScope dscope(h->device);
-  int rc = take_state(h, h->d_conc, conc);
+  int rc = take_state(h, h->d_conc, conc, kHostCells);
   if (rc) return rc;
   HIPOK(hipStreamSynchronize(h->stream));
+  unpack_state(h, conc, kHostCells);
   return SEDCOL_OK;
 }
 
@@ -1101,13 +1142,13 @@ int sedcol_rhs(sedcol_handle *h, const double *conc, double *rhs, double *flux_t
   if (!conc || !rhs) return fail(SEDCOL_EINVAL, "null argument");
   if (h->nrec > 1) return fail(SEDCOL_EINVAL, "a forcing series is active; get_rhs uses one record (sedcol_set_forcing)");
   if ((rc = ensure_scratch(h))) return rc;
-  // packed: state in d_scr, rhs in d_scr2.  Fortran: d_scr takes the caller's
-  // arrays on both ways, so the packed state is a third array
-  const bool fortran = h->layout == SEDCOL_LAYOUT_FORTRAN;
-  if (fortran && !h->d_scr3) HIPOK(hipMalloc(&h->d_scr3, sizeof(double) * NV * (size_t)h->ncell));
-  double *in = fortran ? h->d_scr3 : h->d_scr;
+  // state in d_scr, rhs in d_scr2.  Where k_layout transposes, d_scr takes the
+  // caller's arrays on both ways, so the packed state is a third array
+  const bool third = h->layout == SEDCOL_LAYOUT_FORTRAN && h->ncell > kHostCellsRhs;
+  if (third && !h->d_scr3) HIPOK(hipMalloc(&h->d_scr3, sizeof(double) * NV * (size_t)h->ncell));
+  double *in = third ? h->d_scr3 : h->d_scr;
   const size_t fl = sizeof(double) * NV * (size_t)h->ncol;
-  if ((rc = put_state(h, conc, in))) return rc;
+  if ((rc = put_state(h, conc, in, kHostCellsRhs))) return rc;
   HIPOK(hipMemsetAsync(h->d_scr2, 0, sizeof(double) * NV * (size_t)h->ncell, h->stream));
   HIPOK(hipMemsetAsync(h->d_small, 0, fl, h->stream));
   const Dev d = h->dev();
@@ -1115,9 +1156,10 @@ int sedcol_rhs(sedcol_handle *h, const double *conc, double *rhs, double *flux_t
     if (!h->bins[b].empty())
       sc::launch_rhs(kLpc[b], h->stream, d, h->d_list[b], (int)h->bins[b].size(), h->p, 0, in, h->d_scr2, h->d_small);
   HIPOK(hipGetLastError());
-  if ((rc = take_state(h, h->d_scr2, rhs))) return rc;
+  if ((rc = take_state(h, h->d_scr2, rhs, kHostCellsRhs))) return rc;
   if (flux_top_out) HIPOK(hipMemcpyAsync(flux_top_out, h->d_small, fl, hipMemcpyDeviceToHost, h->stream));
   HIPOK(hipStreamSynchronize(h->stream));
+  unpack_state(h, rhs, kHostCellsRhs);
   return SEDCOL_OK;
 }
 
