@@ -351,28 +351,28 @@ void drop_graph(sedcol_handle *h)
 // Work-queue counters and the pending count must be zero beforehand.
 // Persistent launches always run as branches forked from the handle's stream:
 // each bin ends on a few slow columns that leave most of the device idle, and
-// the next bin's blocks start there.  The bin with the fewest blocks goes
+// the next bin's blocks start there.  The bin with the fewest threads goes
 // first: its columns all start at once, and the bin that has more columns than
 // places, which works off a queue, fills what they leave.  In order, the bins'
 // slowest columns added up (1201 columns of 30 to 60 layers, geometric weights,
 // 3 h: 768 ms in order, 405 ms as branches; 9001 columns of 10 to 60 layers,
-// 6 h: 650 ms in order, 426 ms with the most blocks first, 266 ms with the
+// 6 h: 650 ms in order, 426 ms with the most threads first, 266 ms with the
 // fewest first).  Windowed launches fork as the schedule says.
 int launch_bins(sedcol_handle *h, int only, int *launches)
 {
   int list[3], nb = 0;
-  long long blocks[3] = {0, 0, 0};
+  long long threads[3] = {0, 0, 0};
   for (int b = 0; b < 3; ++b)
     if (!h->bins[b].empty() && (only < 0 || only == b)) {
       int lpc, blk, lpl;
       effective_shape(h, b, &lpc, &blk, &lpl);
-      blocks[b] = ((long long)h->bins[b].size() * lpc + blk - 1) / blk * blk;  // in threads: blocks differ in size
+      threads[b] = ((long long)h->bins[b].size() * lpc + blk - 1) / blk * blk;
       list[nb++] = b;
     }
-  std::stable_sort(list, list + nb, [&](int p, int q) { return blocks[p] < blocks[q]; });
+  std::stable_sort(list, list + nb, [&](int p, int q) { return threads[p] < threads[q]; });
   const bool fork = (h->sched.window <= 0 || h->sched.concurrent_bins) && nb > 1;
   if (fork) HIPOK(hipEventRecord(h->evfork, h->stream));
-  for (int i = 0; i < nb; ++i) {
+  auto branch = [&](int i) -> int {
     const int b = list[i];
     hipStream_t st = h->stream;
     if (fork && i > 0) {
@@ -386,11 +386,16 @@ int launch_bins(sedcol_handle *h, int only, int *launches)
       return fail(SEDCOL_EINVAL, "unsupported lanes per column / workgroup size");
     ++*launches;
     if (fork && i > 0) HIPOK(hipEventRecord(h->evjoin[i - 1], st));
-  }
+    return SEDCOL_OK;
+  };
+  int rc = SEDCOL_OK, done = 0;
+  while (done < nb && (rc = branch(done)) == SEDCOL_OK) ++done;
   // joined after the last launch: a wait between them would order the
-  // handle's own branch behind the others
+  // handle's own branch behind the others.  After a failure, too: the branches
+  // that run are the handle's work
   if (fork)
-    for (int i = 1; i < nb; ++i) HIPOK(hipStreamWaitEvent(h->stream, h->evjoin[i - 1], 0));
+    for (int i = 1; i < done; ++i) HIPOK(hipStreamWaitEvent(h->stream, h->evjoin[i - 1], 0));
+  if (rc) return rc;
   HIPOK(hipGetLastError());
   return SEDCOL_OK;
 }
