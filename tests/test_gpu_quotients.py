@@ -1,5 +1,5 @@
-"""Quotients of the reference form without IEEE divisions, at the operands where
-such sequences go wrong; bit patterns against the oracle."""
+"""Quotients and reciprocals of the reference form without IEEE divisions, at
+the operands where such sequences go wrong; bit patterns against the oracle."""
 import numpy as np
 import pytest
 
@@ -11,6 +11,27 @@ pytestmark = pytest.mark.gpu
 
 def _bits(a):
     return np.ascontiguousarray(a).view(np.int64)
+
+
+def test_reciprocal_of_a_mantissa_of_ones(gpu_ready):
+    """The pathway sum 1 - 2^-53: its reciprocal lies 2^-106 above the middle of
+    two doubles, where a correction by the residual meets a tie."""
+    dom = cases.plain_columns(ni=64, nj=1, K=16, seed=6)
+    dom.params.kin.kinO2anox = 2.0 ** -50
+    dom.params.kin.ksO2oxic = 3.0
+    o2 = 3.0 * 2.0 ** 53
+    assert o2 / (o2 + 3.0) == 1.0 - 2.0 ** -53
+    rng = np.random.default_rng(1)
+    x = dom.conc0.copy()
+    x[:5] = 10.0 ** rng.uniform(0.0, 5.0, size=x[:5].shape)
+    x[5] = o2
+    x[6:9] = 0.0
+    dom.cbw[0, 5] = o2
+    p = dom.params.si()
+    with capi.SedimentColumns.from_domain(dom) as g:
+        rg, fg = g.get_rhs(x)
+    ro, fo = O.Oracle(dom, p).rhs(x)
+    assert np.array_equal(rg, ro) and np.array_equal(fg, fo)
 
 
 @pytest.mark.parametrize("wide", [False, True])
