@@ -172,17 +172,20 @@ __device__ __forceinline__ double rcp_exact(double b)
   const double y = rcp_near(b);
   return fma(fma(-b, y, 1.0), y, y);
 }
-// a / b with y = 1/b rounded.  The residual is taken with its sign reversed: for
-// b > 0 a zero quotient then keeps the sign of a (q + -0), which q + 0 loses.
-__device__ __forceinline__ double div_by(double a, double b, double y)
+// a / b with ny = -1/b rounded.  The residual is taken with its sign reversed: for
+// b > 0 a zero quotient then keeps the sign of a (q + -0), which q + 0 loses.  The
+// reciprocal is negative so that the last step is the short form of the fma,
+// which has no sign modifiers (240 RK4 steps of 16 columns of 15 layers: 1527 ->
+// 1504 us).
+__device__ __forceinline__ double div_by(double a, double b, double ny)
 {
-  const double q = a * y;
-  return fma(-fma(b, q, -a), y, q);
+  const double q = a * -ny;
+  return fma(fma(b, q, -a), ny, q);
 }
 template <bool FD>
 __device__ __forceinline__ double quot(double a, double b)
 {
-  if constexpr (FD) return div_by(a, b, rcp_near(b));
+  if constexpr (FD) return div_by(a, b, -rcp_near(b));
   else return a / b;
 }
 template <bool FD>
@@ -567,9 +570,9 @@ struct Lane {
   // reference form: geometry and interface diffusivities (dzc is dz on the
   // top layer, whose flux is taken over dz)
   double dz, dzc, Dbio, Ddis;
-  // reference form: reciprocals of its divisors dzc, (1 - phi) dz, phi dz and
-  // phi, and whether the column has a value outside the range in which a
-  // division by them is exact
+  // reference form: negative reciprocals of its divisors dzc, (1 - phi) dz,
+  // phi dz and phi (div_by), and whether the column has a value outside the
+  // range in which a division by them is exact
   double ydzc, yVp, yVd, yphi;
   bool wide;
   // fast form: Dbio/dzc, Ddis/dzc (D/dz on the top layer), 1/(phi dz)
@@ -605,10 +608,10 @@ __device__ __forceinline__ void diffusivities(const sedcol_params &p, double B, 
     L.Dbio = Dbio;
     L.Ddis = Ddis;
     if (ARITH == ARITH_REF) {
-      L.ydzc = 1.0 / L.dzc;
-      L.yVp = 1.0 / ((1.0 - L.phi) * L.dz);
-      L.yVd = 1.0 / (L.phi * L.dz);
-      L.yphi = 1.0 / L.phi;
+      L.ydzc = -1.0 / L.dzc;
+      L.yVp = -1.0 / ((1.0 - L.phi) * L.dz);
+      L.yVd = -1.0 / (L.phi * L.dz);
+      L.yphi = -1.0 / L.phi;
     }
     if (ARITH == ARITH_EXT) {
       // profile 3: B = f_T = 1 (fabm_sediment_driver.F90:622-623)
