@@ -27,9 +27,10 @@ RK4 step (per cell): 4 rhs + stage updates 3 x 11 x 2 + combination
   11 x (2 + 2) + sinks 12  = 692 + 66 + 44 + 12 = 814.
 Linearly implicit ROS2 attempt (method 7, per cell):
   2 rhs                           346
-  reaction Jacobian kin_jac, x 2  254   (127 each: detritus 41, partition 59,
-                                         nitrification/ODU/P 27)
-  transport factor, 11 species    165   (15 per species and layer)
+  reaction Jacobian kin_jac       127   (kept for both stages: detritus 41,
+                                         partition 59, nitrification/ODU/P 27)
+  transport factor                 27   (one for the particulate species, 15 per
+                                         layer, one for the dissolved ones, 12)
   2 W-solves                     1578   (789 each: 2 species sweeps 2 x 132,
                                          2 block solves 2 x 174, J_R k0 67,
                                          transport residual 99, sum 11)
@@ -37,7 +38,7 @@ Linearly implicit ROS2 attempt (method 7, per cell):
   sink gradients                   24
   error norm 11 x 13 + 1          144
   accepted update + sinks          65
-  total                          2620
+  total                          2355
 """
 from __future__ import annotations
 
@@ -60,8 +61,9 @@ KJAC_SOLVE = 174
 KJAC_APPLY = 67
 SPECIES_SWEEP = 12 * NV
 W_SOLVE = 2 * SPECIES_SWEEP + 2 * KJAC_SOLVE + KJAC_APPLY + 9 * NV + NV
-ROS2_ATTEMPT_PER_CELL = (2 * RHS_PER_CELL + 2 * KIN_JAC + 15 * NV + 2 * W_SOLVE + 4 * NV + 24
-                         + (13 * NV + 1) + (5 * NV + 10))  # 2620
+CLASS_FACTORS = 15 + 12
+ROS2_ATTEMPT_PER_CELL = (2 * RHS_PER_CELL + KIN_JAC + CLASS_FACTORS + 2 * W_SOLVE + 4 * NV + 24
+                         + (13 * NV + 1) + (5 * NV + 10))  # 2355
 
 #: HBM bytes a persistent adaptive launch moves per cell and per column,
 #: independent of the number of steps inside it: state in+out (2*11*8), the
