@@ -1548,8 +1548,9 @@ __global__ __launch_bounds__(BLK, SEDCOL_ROS_MIN_WAVES) void k_ros_adaptive(
       store_top(l == 0, Ft, F[0]);
       ros_rows<LPC>(R, C, l, K, act, L.phi, gh, dirmask);
       // The Jacobian stays live for the second stage, and with it the local
-      // solves' pivots: a spin-up of 3000 columns takes 165 ms against 171 with
-      // a second evaluation, though 64 lanes pay 168 bytes of scratch.
+      // solves' pivots: a spin-up of 3000 columns (fast form) takes 165 ms against
+      // 171 with a second evaluation, though 64 lanes then have 172 to 220 bytes
+      // of scratch.
       KJac J;
       kin_jac(p, L.fT, x, J);
       bool ok = ros_wsolve<LPC, true>(R, S, J, C, l, K, kw, act, gh, dirmask, L.phi, f, k1, R.top[0]);
