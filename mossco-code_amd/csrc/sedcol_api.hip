@@ -9,6 +9,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -112,7 +113,7 @@ struct sedcol_handle {
                              // [5], [6] votes of adaptive Euler attempts
   int *h_flag = nullptr;     // pinned host copy of d_flag[0..4]
   bool piped = false;        // counts as a user of the pinned blocks (copy_large)
-  std::vector<double> h_pack;  // small Fortran states, packed
+  std::vector<double> h_pack;  // Fortran states that the host transposes, packed
   double *h_stage = nullptr; // pinned: state, top fluxes and flags of sedcol_step, small domains only
   int *d_work = nullptr;     // ncol: attempts of each column in the last adaptive launch
   int *d_wrec = nullptr;     // ncol: adaptive position between windows (record, time left, attempts)
@@ -499,8 +500,8 @@ int ensure_scratch(sedcol_handle *h)
 
 // The caller's state arrays go to and from the device as they are, without a
 // copy in host memory: packed ones directly, Fortran ones through d_scr and
-// k_layout, small ones excepted.  (With the transposition on the host and pageable copies, setting
-// 238 MB took 59 ms and reading them 76 ms.)
+// k_layout, some excepted (host_transposes).  (With the transposition on the
+// host and pageable copies, setting 238 MB took 59 ms and reading them 76 ms.)
 //
 // Large copies go through pinned blocks that several threads fill or empty: the
 // link takes pinned memory at 55 GB/s, where one thread of the runtime moves
@@ -619,20 +620,43 @@ void transpose_state(const sedcol_handle *h, const double *src, double *dst, boo
     }
 }
 
+// Whether the host transposes this state: a small one of up to host_cells cells,
+// and any for which the device's memory has no room left for *scratch, the array
+// that k_layout needs (allocated here).
+bool host_transposes(sedcol_handle *h, long long host_cells, double **scratch)
+{
+  if (h->layout == SEDCOL_LAYOUT_PACKED) return false;
+  if (h->ncell <= host_cells) return true;
+  if (*scratch || hipMalloc(scratch, sizeof(double) * NV * (size_t)h->ncell) == hipSuccess) return false;
+  (void)hipGetLastError();
+  *scratch = nullptr;
+  return true;
+}
+
+// h_pack for the whole state, made at creation for small ones
+int ensure_pack(sedcol_handle *h)
+{
+  try {
+    h->h_pack.resize(NV * (size_t)h->ncell);
+  } catch (const std::exception &) {
+    return fail(SEDCOL_ENOMEM, "no host memory for the state's transposition");
+  }
+  return SEDCOL_OK;
+}
+
 // caller's state (NV planes) -> packed device array dst (not d_scr if the device
-// transposes); a Fortran state of up to host_cells cells is transposed by the host
-int put_state(sedcol_handle *h, const double *conc, double *dst, long long host_cells)
+// transposes); by_host: host_transposes
+int put_state(sedcol_handle *h, const double *conc, double *dst, bool by_host)
 {
   const size_t bytes = sizeof(double) * NV * (size_t)h->ncell;
   if (h->layout == SEDCOL_LAYOUT_PACKED) return copy_large(h, dst, conc, nullptr, bytes, true);
-  if (h->ncell <= host_cells) {
+  int rc;
+  if (by_host) {
+    if ((rc = ensure_pack(h))) return rc;
     transpose_state(h, conc, h->h_pack.data(), true);
-    HIPOK(hipMemcpyAsync(dst, h->h_pack.data(), bytes, hipMemcpyHostToDevice, h->stream));
-    return SEDCOL_OK;
+    return copy_large(h, dst, h->h_pack.data(), nullptr, bytes, true);
   }
-  if (!h->d_scr) HIPOK(hipMalloc(&h->d_scr, bytes));
-  const int rc = copy_large(h, h->d_scr, conc, nullptr, bytes, true);
-  if (rc) return rc;
+  if ((rc = copy_large(h, h->d_scr, conc, nullptr, bytes, true))) return rc;
   sc::launch_layout(h->stream, h->d_scr, dst, h->ncol, h->kmax, NV, true);
   HIPOK(hipGetLastError());
   return SEDCOL_OK;
@@ -640,15 +664,14 @@ int put_state(sedcol_handle *h, const double *conc, double *dst, long long host_
 
 // packed device array src (not d_scr if the device transposes) -> caller's state;
 // complete after a wait and unpack_state
-int take_state(sedcol_handle *h, double *src, double *conc, long long host_cells)
+int take_state(sedcol_handle *h, double *src, double *conc, bool by_host)
 {
   const size_t bytes = sizeof(double) * NV * (size_t)h->ncell;
-  if (h->layout != SEDCOL_LAYOUT_PACKED && h->ncell <= host_cells) {
-    HIPOK(hipMemcpyAsync(h->h_pack.data(), src, bytes, hipMemcpyDeviceToHost, h->stream));
-    return SEDCOL_OK;
+  if (by_host) {
+    const int rc = ensure_pack(h);
+    return rc ? rc : copy_large(h, src, nullptr, h->h_pack.data(), bytes, false);
   }
   if (h->layout != SEDCOL_LAYOUT_PACKED) {
-    if (!h->d_scr) HIPOK(hipMalloc(&h->d_scr, bytes));
     sc::launch_layout(h->stream, src, h->d_scr, h->ncol, h->kmax, NV, false);
     HIPOK(hipGetLastError());
     src = h->d_scr;
@@ -656,10 +679,9 @@ int take_state(sedcol_handle *h, double *src, double *conc, long long host_cells
   return copy_large(h, src, nullptr, conc, bytes, false);
 }
 
-void unpack_state(sedcol_handle *h, double *conc, long long host_cells)
+void unpack_state(sedcol_handle *h, double *conc, bool by_host)
 {
-  if (h->layout != SEDCOL_LAYOUT_PACKED && h->ncell <= host_cells)
-    transpose_state(h, h->h_pack.data(), conc, false);
+  if (by_host) transpose_state(h, h->h_pack.data(), conc, false);
 }
 
 // upload the current bins as the work lists (after a change of the active set)
@@ -1087,7 +1109,7 @@ int sedcol_set_state(sedcol_handle *h, const double *conc)
 {
   if (!h || !conc) return fail(SEDCOL_EINVAL, "null argument");
   const DeviceScope dscope(h->device);
-  int rc = put_state(h, conc, h->d_conc, kHostCells);
+  int rc = put_state(h, conc, h->d_conc, host_transposes(h, kHostCells, &h->d_scr));
   if (rc) return rc;
   HIPOK(hipStreamSynchronize(h->stream));
   return SEDCOL_OK;
@@ -1132,10 +1154,11 @@ int sedcol_get_state(sedcol_handle *h, double *conc)
 {
   if (!h || !conc) return fail(SEDCOL_EINVAL, "null argument");
   const DeviceScope dscope(h->device);
-  int rc = take_state(h, h->d_conc, conc, kHostCells);
+  const bool by_host = host_transposes(h, kHostCells, &h->d_scr);
+  int rc = take_state(h, h->d_conc, conc, by_host);
   if (rc) return rc;
   HIPOK(hipStreamSynchronize(h->stream));
-  unpack_state(h, conc, kHostCells);
+  unpack_state(h, conc, by_host);
   return SEDCOL_OK;
 }
 
@@ -1149,11 +1172,10 @@ int sedcol_rhs(sedcol_handle *h, const double *conc, double *rhs, double *flux_t
   if ((rc = ensure_scratch(h))) return rc;
   // state in d_scr, rhs in d_scr2.  Where k_layout transposes, d_scr takes the
   // caller's arrays on both ways, so the packed state is a third array
-  const bool third = h->layout == SEDCOL_LAYOUT_FORTRAN && h->ncell > kHostCellsRhs;
-  if (third && !h->d_scr3) HIPOK(hipMalloc(&h->d_scr3, sizeof(double) * NV * (size_t)h->ncell));
-  double *in = third ? h->d_scr3 : h->d_scr;
+  const bool by_host = host_transposes(h, kHostCellsRhs, &h->d_scr3);
+  double *in = h->layout == SEDCOL_LAYOUT_PACKED || by_host ? h->d_scr : h->d_scr3;
   const size_t fl = sizeof(double) * NV * (size_t)h->ncol;
-  if ((rc = put_state(h, conc, in, kHostCellsRhs))) return rc;
+  if ((rc = put_state(h, conc, in, by_host))) return rc;
   HIPOK(hipMemsetAsync(h->d_scr2, 0, sizeof(double) * NV * (size_t)h->ncell, h->stream));
   HIPOK(hipMemsetAsync(h->d_small, 0, fl, h->stream));
   const Dev d = h->dev();
@@ -1161,10 +1183,10 @@ int sedcol_rhs(sedcol_handle *h, const double *conc, double *rhs, double *flux_t
     if (!h->bins[b].empty())
       sc::launch_rhs(kLpc[b], h->stream, d, h->d_list[b], (int)h->bins[b].size(), h->p, 0, in, h->d_scr2, h->d_small);
   HIPOK(hipGetLastError());
-  if ((rc = take_state(h, h->d_scr2, rhs, kHostCellsRhs))) return rc;
+  if ((rc = take_state(h, h->d_scr2, rhs, by_host))) return rc;
   if (flux_top_out) HIPOK(hipMemcpyAsync(flux_top_out, h->d_small, fl, hipMemcpyDeviceToHost, h->stream));
   HIPOK(hipStreamSynchronize(h->stream));
-  unpack_state(h, rhs, kHostCellsRhs);
+  unpack_state(h, rhs, by_host);
   return SEDCOL_OK;
 }
 
