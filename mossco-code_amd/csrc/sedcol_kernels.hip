@@ -436,11 +436,15 @@ __global__ __launch_bounds__(BLOCK, fixed_waves(METHOD, ARITH, FULL)) void k_fix
 // minimum waves per SIMD requested from the register allocator: 2 fits the
 // adaptive step in 256 VGPRs without scratch (1 lets it take 256 + AGPRs,
 // 3 spills about 340 bytes per lane).  With geometric weights the step does not
-// fit (130 to 190 bytes of scratch per lane) and one wave is faster at every
-// size, reference form, 1 h: 1201 columns of 30 to 60 layers 157 -> 104 ms,
-// 9000 columns of 10 to 60 layers 300 -> 235 ms.  It then has room for the
-// boundary values and the solve's coefficients, which were read from LDS in
-// every evaluation (3 h of the 1201 columns 273 -> 264 ms).
+// fit (130 to 190 bytes of scratch per lane) and one wave is faster, reference
+// form, 1 h: 1201 columns of 30 to 60 layers 157 -> 104 ms, 9000 columns of 10 to
+// 60 layers 300 -> 235 ms.  It then has room for the boundary values and the
+// solve's coefficients, which were read from LDS in every evaluation (3 h of the
+// 1201 columns 273 -> 264 ms).  Many columns of long bins only, reference form,
+// 15 min, were faster in two waves before the right-hand side became one stretch
+// of code: 12000 of 34 to 60 layers 128, now 133 ms, 25000 of them 257, now 276.
+// Two waves of the present code spill 172 to 232 bytes: 144 and 288 ms, without
+// the quotients by reciprocals 135 and 265.
 #ifndef SEDCOL_EMP_MIN_WAVES
 #define SEDCOL_EMP_MIN_WAVES 2
 #endif
